@@ -36,6 +36,12 @@ int pspi_tables(const swem_geometry& g, const float* vel, float* vref, int* iref
 void taper_f32(int n, int l, float* t);
 void slowness_f32(const swem_geometry& g, const float* vel, float* po, float* pd);
 
+// 2-D march workgroups.  Subgroup kernels: 8 points per thread, up to 1024 threads (128 VGPRs, four waves per SIMD),
+// or 16 points per thread, up to 512 threads (256 VGPRs): radix-16 passes halve the LDS round
+// trips.  Wave kernels: 256 threads, two waves per SIMD.
+constexpr int kMaxBlock = 1024;
+constexpr int kWaveBlock = 256;
+
 // Mixed-radix transform plan of a length n = 2^a 3^b 5^c <= 4096 (mixed_fft in swem_fft.hpp):
 // the radix of every pass in order (8 while 8 divides the rest, then 4, 2, 5, 3), the product of
 // the radices before it, its twiddle step n / (ns r) and the multiplier that divides by ns
@@ -175,7 +181,7 @@ int march2d_blue_len(int nkx);
 int march2d_kind(int nkx);
 size_t march2d_lds_bytes(int nkx, const March2DShape& sh, int F);
 
-// Arguments of the 3-D split-step kernels (swem_march3d.hip).  A launch covers the items
+// Arguments of the 3-D split-step kernels (swem_march3d.hpp).  A launch covers the items
 // (frequencies f0 .. f0 + nitem of one shot) of a frequency chunk at depth iz.
 // Per-shot values of a 3-D migration read by the kernels from device memory, so that the launch
 // sequence of a shot does not depend on the shot (it is captured once as a graph and replayed).
