@@ -40,92 +40,101 @@ __device__ __forceinline__ float2 mul_si(float2 a)
     return SIGN < 0 ? make_float2(a.y, -a.x) : make_float2(-a.y, a.x);
 }
 
+// exp(SIGN i pi M / 8) for a compile-time M in 0..3 (and i times it for 4..7, by mul_si)
+constexpr float kCos8[4] = {1.f, 0.92387953251128675613f, 0.70710678118654752440f, 0.38268343236508977173f};
+constexpr float kSin8[4] = {0.f, 0.38268343236508977173f, 0.70710678118654752440f, 0.92387953251128675613f};
+
+// a, b <- a + w b, a - w b in six fused multiply-adds: y = a + w b by four, a - w b = 2 a - y by
+// two (a complex product and two sums are ten operations, eight after contraction; the radix-2
+// butterfly of Linzer and Feig, "Implementation of efficient FFT algorithms on fused multiply-add
+// architectures", IEEE Trans. Signal Processing 41 (1993), in its unscaled form).
+__device__ __forceinline__ void bfly(float2& a, float2& b, float2 w)
+{
+    const float yr = fmaf(-w.y, b.y, fmaf(w.x, b.x, a.x));
+    const float yi = fmaf(w.y, b.x, fmaf(w.x, b.y, a.y));
+    b = make_float2(fmaf(2.f, a.x, -yr), fmaf(2.f, a.y, -yi));
+    a = make_float2(yr, yi);
+}
+// The same with the product formed once (eight operations, the two results rounded alike): radix-2
+// passes are a chain of dependent exchanges with little arithmetic between, where two operations
+// less buy nothing and the unequal rounding of 2 a - y shows over the many passes.
+__device__ __forceinline__ void bfly_prod(float2& a, float2& b, float2 w)
+{
+    const float2 t = make_float2(fmaf(w.x, b.x, -(w.y * b.y)), fmaf(w.x, b.y, w.y * b.x));
+    b = csub(a, t);
+    a = cadd(a, t);
+}
+__device__ __forceinline__ void bfly1(float2& a, float2& b)
+{
+    const float2 t = csub(a, b);
+    a = cadd(a, b);
+    b = t;
+}
+
+constexpr int bitrev(int i, int n) { return n <= 1 ? 0 : (i & 1) * (n / 2) + bitrev(i >> 1, n / 2); }
+
+// Twiddles of a radix-R butterfly, R = 2, 4, 8 or 16, whose input r is multiplied by w^r: it runs
+// as log2 R radix-2 stages on inputs in bit-reversed order, and the stage of block size S takes
+// w^(R/S) W_S^m, m < S / 4 (m < 1 for S = 2); the upper quarter is SIGN i times these, a swap.
+// So R / 2 seeds in all: [S = 2: w^(R/2)] [S = 4: w^(R/4)] [S = 8: w^(R/8), w^(R/8) W_8]
+// [S = 16: w, w W_16, w W_8, w W_16^3], each one entry of the twiddle table.
+template <int R>
+constexpr int seed_count()
+{
+    return R / 2;
+}
+constexpr int seed_off(int S) { return S <= 2 ? 0 : S / 4; }
+
+// The radix-R butterfly in place on x[0..R), natural order in and out.  TW: with the seeds s
+// (those of exp(-...), conjugated here for SIGN > 0); otherwise w = 1 and the constants are
+// immediate.  HIN: inputs r >= R / 2 are zero and are not read.
+template <int R, int SIGN, bool TW, bool HIN = false>
+__device__ __forceinline__ void dft_pow2(float2 (&x)[R], const float2* s)
+{
+    float2 y[R];
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+        const int r = bitrev(i, R);
+        if (!HIN || r < R / 2) y[i] = x[r];
+    }
+#pragma unroll
+    for (int S = 2; S <= R; S *= 2) {
+#pragma unroll
+        for (int base = 0; base < R; base += S)
+#pragma unroll
+            for (int m = 0; m < S / 2; ++m) {
+                float2 &a = y[base + m], &b = y[base + m + S / 2];
+                if (HIN && S == 2) {
+                    b = a;
+                    continue;
+                }
+                const int q = S >= 4 ? S / 4 : 1, mm = m % q;
+                if (m >= q) b = mul_si<SIGN>(b);
+                if constexpr (TW) {
+                    const float2 w = s[seed_off(S) + mm];
+                    if constexpr (R == 2) bfly_prod(a, b, SIGN > 0 ? cconj(w) : w);
+                    else bfly(a, b, SIGN > 0 ? cconj(w) : w);
+                } else if (mm == 0) {
+                    bfly1(a, b);
+                } else {
+                    const int k = mm * (16 / S);  // W_S^mm = W_16^k
+                    bfly(a, b, make_float2(kCos8[k], SIGN * kSin8[k]));
+                }
+            }
+    }
+#pragma unroll
+    for (int i = 0; i < R; ++i) x[i] = y[i];
+}
+
 template <int R, int SIGN>
-struct Dft;
-
-template <int SIGN>
-struct Dft<2, SIGN> {
-    static __device__ __forceinline__ void run(float2* v)
-    {
-        float2 a = v[0], b = v[1];
-        v[0] = cadd(a, b);
-        v[1] = csub(a, b);
-    }
-};
-
-template <int SIGN>
-struct Dft<4, SIGN> {
-    static __device__ __forceinline__ void run(float2* v)
-    {
-        float2 t0 = cadd(v[0], v[2]), t1 = csub(v[0], v[2]);
-        float2 t2 = cadd(v[1], v[3]), t3 = mul_si<SIGN>(csub(v[1], v[3]));
-        v[0] = cadd(t0, t2);
-        v[2] = csub(t0, t2);
-        v[1] = cadd(t1, t3);
-        v[3] = csub(t1, t3);
-    }
-};
-
-template <int SIGN>
-struct Dft<8, SIGN> {
-    static __device__ __forceinline__ void run(float2* v)
-    {
-        float2 e[4] = {v[0], v[2], v[4], v[6]};
-        float2 o[4] = {v[1], v[3], v[5], v[7]};
-        Dft<4, SIGN>::run(e);
-        Dft<4, SIGN>::run(o);
-        const float r = 0.70710678118654752440f;
-        // W8^1 o = r (o + SIGN i o), W8^2 o = SIGN i o, W8^3 o = r (SIGN i o - o)
-        float2 o1 = cscale(cadd(o[1], mul_si<SIGN>(o[1])), r);
-        float2 o2 = mul_si<SIGN>(o[2]);
-        float2 o3 = cscale(csub(mul_si<SIGN>(o[3]), o[3]), r);
-        v[0] = cadd(e[0], o[0]);
-        v[4] = csub(e[0], o[0]);
-        v[1] = cadd(e[1], o1);
-        v[5] = csub(e[1], o1);
-        v[2] = cadd(e[2], o2);
-        v[6] = csub(e[2], o2);
-        v[3] = cadd(e[3], o3);
-        v[7] = csub(e[3], o3);
-    }
-};
-
-template <int SIGN>
-struct Dft<16, SIGN> {
-    static __device__ __forceinline__ void run(float2* v)
-    {
-        float2 e[8], o[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            e[i] = v[2 * i];
-            o[i] = v[2 * i + 1];
-        }
-        Dft<8, SIGN>::run(e);
-        Dft<8, SIGN>::run(o);
-        // X_k = E_k + W16^k O_k, X_{k+8} = E_k - W16^k O_k, W16^k = cos(pi k/8) + SIGN i sin(pi k/8)
-        const float c1 = 0.92387953251128675613f, s1 = 0.38268343236508977173f;
-        const float r = 0.70710678118654752440f;
-        float2 t[8];
-        t[0] = o[0];
-        t[1] = cmul(o[1], make_float2(c1, SIGN * s1));
-        t[2] = cscale(cadd(o[2], mul_si<SIGN>(o[2])), r);
-        t[3] = cmul(o[3], make_float2(s1, SIGN * c1));
-        t[4] = mul_si<SIGN>(o[4]);
-        t[5] = cmul(o[5], make_float2(-s1, SIGN * c1));
-        t[6] = cscale(csub(mul_si<SIGN>(o[6]), o[6]), r);
-        t[7] = cmul(o[7], make_float2(-c1, SIGN * s1));
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            v[k] = cadd(e[k], t[k]);
-            v[k + 8] = csub(e[k], t[k]);
-        }
-    }
+struct Dft {  // R = 2, 4, 8, 16
+    static __device__ __forceinline__ void run(float2 (&v)[R]) { dft_pow2<R, SIGN, false>(v, nullptr); }
 };
 
 template <int SIGN>
 struct Dft<3, SIGN> {
     // X1,2 = x0 - (x1 + x2) / 2 +- SIGN i (sqrt(3) / 2) (x1 - x2)
-    static __device__ __forceinline__ void run(float2* v)
+    static __device__ __forceinline__ void run(float2 (&v)[3])
     {
         const float h = 0.86602540378443864676f;
         const float2 a = cadd(v[1], v[2]), b = cscale(mul_si<SIGN>(csub(v[1], v[2])), h);
@@ -140,7 +149,7 @@ template <int SIGN>
 struct Dft<5, SIGN> {
     // with a1 = x1 + x4, a2 = x2 + x3, b1 = x1 - x4, b2 = x2 - x3 and w = exp(SIGN 2 pi i / 5):
     // X1,4 = x0 + c1 a1 + c2 a2 +- SIGN i (s1 b1 + s2 b2), X2,3 = x0 + c2 a1 + c1 a2 +- SIGN i (s2 b1 - s1 b2)
-    static __device__ __forceinline__ void run(float2* v)
+    static __device__ __forceinline__ void run(float2 (&v)[5])
     {
         const float c1 = 0.30901699437494742410f, c2 = -0.80901699437494742410f;
         const float s1 = 0.95105651629515357212f, s2 = 0.58778525229247312917f;
@@ -158,57 +167,6 @@ struct Dft<5, SIGN> {
         v[3] = csub(p2, q2);
     }
 };
-
-// x * exp(SIGN i pi M / 8) for a compile-time M in 0..7 (the twiddles W_R^n of R <= 16).
-template <int M, int SIGN>
-__device__ __forceinline__ float2 cmul_pi8(float2 x)
-{
-    constexpr float C[5] = {1.f, 0.92387953251128675613f, 0.70710678118654752440f, 0.38268343236508977173f, 0.f};
-    if constexpr (M == 0) return x;
-    else if constexpr (M == 4) return mul_si<SIGN>(x);
-    else if constexpr (M == 2) return cscale(cadd(x, mul_si<SIGN>(x)), C[2]);
-    else if constexpr (M == 6) return cscale(csub(mul_si<SIGN>(x), x), C[2]);
-    else {
-        // cos and sin of M pi / 8 (M odd): cos = +-C[M or 8 - M], sin = C[4 - M or M - 4]
-        constexpr float c = M < 4 ? C[M] : -C[8 - M];
-        constexpr float sn = M < 4 ? C[4 - M] : C[M - 4];
-        return cmul(x, make_float2(c, SIGN * sn));
-    }
-}
-
-// R-point DFT whose inputs r >= R/2 are zero: X_2m = DFT_{R/2}(x_n)_m, X_2m+1 = DFT_{R/2}(x_n W_R^n)_m
-// over n < R/2 (W_R = exp(SIGN 2 pi i / R)); v[r] for r >= R/2 is not read.
-template <int R, int SIGN>
-__device__ __forceinline__ void dft_half_in(float2* v)
-{
-    constexpr int H = R / 2;
-    if constexpr (R == 2) {
-        v[1] = v[0];
-    } else {
-        float2 e[H], o[H];
-#pragma unroll
-        for (int n = 0; n < H; ++n) e[n] = v[n];
-        o[0] = v[0];
-        if constexpr (H > 1) o[1] = cmul_pi8<16 / R, SIGN>(v[1]);
-        if constexpr (H > 2) {
-            o[2] = cmul_pi8<32 / R, SIGN>(v[2]);
-            o[3] = cmul_pi8<48 / R, SIGN>(v[3]);
-        }
-        if constexpr (H > 4) {
-            o[4] = cmul_pi8<64 / R, SIGN>(v[4]);
-            o[5] = cmul_pi8<80 / R, SIGN>(v[5]);
-            o[6] = cmul_pi8<96 / R, SIGN>(v[6]);
-            o[7] = cmul_pi8<112 / R, SIGN>(v[7]);
-        }
-        Dft<H, SIGN>::run(e);
-        Dft<H, SIGN>::run(o);
-#pragma unroll
-        for (int m = 0; m < H; ++m) {
-            v[2 * m] = e[m];
-            v[2 * m + 1] = o[m];
-        }
-    }
-}
 
 // Bank-conflict padding: one complex inserted every 2^SH.  The LDS has 64 banks of 4 bytes (32
 // complex per row).  A Stockham pass writes at lane stride R (first pass) or in groups of NS
@@ -250,92 +208,105 @@ constexpr int fft_passes()
     return p;
 }
 
-// Twiddle seeds of fft<N,P>: for each pass after the first (NS > 1, radix R) and each butterfly
-// b of a thread, the powers w^e, w = exp(-2 pi i k / (NS R)), k = (t + b T) mod NS, for the
-// seeded exponents e (1, 2, 3 and the multiples of 4 below R), read from the table at the start
-// of a transform.  The other powers are one product of two seeds, w^(4a + c) = w^(4a) w^c, so
-// a twiddle carries at most one rounding beyond the table's (powers by longer chains of
-// products drift: their systematic error, repeated over every transform of a march, grows the
-// image error tenfold).  Radix 16: 6 loads per butterfly instead of 15, radix 8: 4 instead of 7.
-template <int R>
-constexpr int seed_count()
-{
-    return R <= 4 ? R - 1 : 3 + (R - 1) / 4;
-}
-// the i-th seeded exponent: 1, 2, 3, then 4, 8, 12, ...
-constexpr int seed_exp(int i) { return i < 3 ? i + 1 : 4 * (i - 2); }
+// One pass of fft<N,P>.  Twiddle seeds of a pass after the first (NS > 1, radix R): for each
+// butterfly b of a thread the R / 2 stage twiddles of dft_pow2 with w = exp(-2 pi i k / (NS R)),
+// k = (t + b T) mod NS: w^(R/S) W_S^m is the table entry N / (S NS) (k + m NS), below N / 2.
+template <int N, int P, int NS>
+struct FPass {
+    static constexpr int T = N / P;
+    static constexpr int REM = N / NS;
+    static constexpr int R = REM >= P ? P : REM;
+    static constexpr int B = P / R;
+    static constexpr bool LAST = (NS * R == N);
+    static constexpr int S = seed_count<R>();
+    static constexpr int NTW = NS > 1 ? B * S : 1;  // twiddle seeds per thread (1: unused slot)
+};
 
-template <int N, int P>
-constexpr int fft_seeds_before(int ns_end)
+// The seeds of one radix-R butterfly of pass NS, k = its index mod NS.
+template <int N, int NS, int R>
+__device__ __forceinline__ void pass_seeds(const float2* __restrict__ tw, uint32_t k, float2* s)
 {
-    int n = 1, c = 0;
-    while (n < N && n < ns_end) {
-        const int rem = N / n, r = rem >= P ? P : rem;
-        if (n > 1) c += (P / r) * (r <= 4 ? r - 1 : 3 + (r - 1) / 4);
-        n *= r;
+#pragma unroll
+    for (int S = 2; S <= R; S *= 2)
+#pragma unroll
+        for (int m = 0; m < (S >= 4 ? S / 4 : 1); ++m)
+            s[seed_off(S) + m] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(tw) +
+                                                                  k * (uint32_t)(8 * (N / (S * NS))) + 8 * m * (N / S));
+}
+
+// The seeds of pass NS.  Byte offsets from the wave-uniform table: one 32-bit offset register and an
+// immediate per load instead of a 64-bit address.
+template <int N, int P, int NS>
+__device__ __forceinline__ void fft_seeds(const float2* __restrict__ tw, int t,
+                                          float2 (&w)[FPass<N, P, NS>::NTW])
+{
+    using S = FPass<N, P, NS>;
+    if constexpr (NS > 1) {
+#pragma unroll
+        for (int b = 0; b < S::B; ++b) {
+            // opaque: the loads stay in the transform instead of pinning registers across the
+            // caller's loops
+            uint32_t k = (uint32_t)(t + b * S::T) & (NS - 1);
+            asm volatile("" : "+v"(k));
+            pass_seeds<N, NS, S::R>(tw, k, &w[b * S::S]);
+        }
     }
-    return c;
+}
+
+// Seeds of every pass of fft<N,P>, in pass order.
+template <int N, int P, int NS = 1>
+constexpr int fft_seed_total()
+{
+    using S = FPass<N, P, NS>;
+    const int own = NS > 1 ? S::NTW : 0;
+    if constexpr (S::LAST) return own;
+    else return own + fft_seed_total<N, P, NS * S::R>();
 }
 template <int N, int P>
 struct FftSeeds {
-    static constexpr int count = fft_seeds_before<N, P>(N);
+    static constexpr int count = fft_seed_total<N, P>();
     float2 w[count > 0 ? count : 1];
+    template <int NS = 1>
+    __device__ __forceinline__ void load(const float2* __restrict__ tw, int t)
+    {
+        using S = FPass<N, P, NS>;
+        if constexpr (NS > 1) {
+            constexpr int off = count - fft_seed_total<N, P, NS>();
+            float2 q[S::NTW];
+            fft_seeds<N, P, NS>(tw, t, q);
+#pragma unroll
+            for (int i = 0; i < S::NTW; ++i) w[off + i] = q[i];
+        }
+        if constexpr (!S::LAST) load<NS * S::R>(tw, t);
+    }
 };
 
-// The seeds of pass NS (all passes from NS on when ALL).
-template <int N, int P, int NS, bool ALL>
-__device__ __forceinline__ void fft_seeds_load(FftSeeds<N, P>& s, const float2* __restrict__ tw, int t)
-{
-    constexpr int T = N / P;
-    constexpr int REM = N / NS;
-    constexpr int R = REM >= P ? P : REM;
-    if constexpr (NS > 1) {
-        constexpr int off = fft_seeds_before<N, P>(NS);
-        constexpr int S = seed_count<R>();
-#pragma unroll
-        for (int b = 0; b < P / R; ++b) {
-            // opaque: the loads stay in the transform instead of pinning registers across the
-            // caller's loops
-            int ti = ((t + b * T) & (NS - 1)) * (N / (NS * R));
-            asm volatile("" : "+v"(ti));
-#pragma unroll
-            for (int i = 0; i < S; ++i) s.w[off + b * S + i] = tw[seed_exp(i) * ti];
-        }
-    }
-    if constexpr (ALL && NS * R < N) fft_seeds_load<N, P, NS * R, true>(s, tw, t);
-}
-
-// pw[r] = w^r, r = 1 .. R-1, from the seeds sd[i] = w^seed_exp(i) (conjugated for SIGN > 0)
-template <int R, int SIGN>
-__device__ __forceinline__ void twiddle_powers(const float2* sd, float2 (&pw)[R])
-{
-    constexpr int S = seed_count<R>();
-#pragma unroll
-    for (int i = 0; i < S; ++i) pw[seed_exp(i)] = SIGN > 0 ? cconj(sd[i]) : sd[i];
-#pragma unroll
-    for (int r = 5; r < R; ++r)
-        if (r % 4 != 0) pw[r] = cmul(pw[r & ~3], pw[r & 3]);
-}
+// Where a transform's seeds come from.
+//   kSeedPass   each pass loads its own (every load in flight before the first use: under register
+//               pressure the scheduler would otherwise pair each load with its use and serialise
+//               the latencies)
+//   kSeedAhead  a pass loads the next one's at its start, so that their latency overlaps its
+//               butterflies
+//   kSeedHeld   the caller holds all of them in registers (FftSeeds): they depend on the thread
+//               only, so a march reads them once
+enum { kSeedPass = 0, kSeedAhead = 1, kSeedHeld = 2 };
 
 // One Stockham pass and the passes after it on one wavefield v in the strided mapping.
 // lds: the subgroup's two buffers (2 * LdsLen<N> complex); pp: buffer parity, toggled per
-// round trip; s: the twiddle seeds, loaded at the start of the transform (PRE) or of each pass
-// (every load of a pass in flight before the first use: under register pressure the scheduler
-// would otherwise pair each load with its use and serialise the latencies).
-template <int N, int P, int SIGN, int NS, bool PRE, bool HIN>
+// round trip; w: this pass's twiddle seeds (kSeedHeld: those of this and the later passes).
+template <int N, int P, int SIGN, int NS, int SEED, bool HIN>
 __device__ __forceinline__ void fft_pass(float2 (&v)[P], float2* lds, const float2* __restrict__ tw,
-                                         FftSeeds<N, P>& s, int t, int& pp)
+                                         const float2* w, int t, int& pp)
 {
-    constexpr int T = N / P;
-    constexpr int REM = N / NS;
-    constexpr int R = REM >= P ? P : REM;
-    constexpr int B = P / R;
-    constexpr bool LAST = (NS * R == N);
+    using S = FPass<N, P, NS>;
+    constexpr int T = S::T, R = S::R, B = S::B;
     constexpr int L = LdsLen<N>::value;
     constexpr int SH = PassPad<NS, R>::value;
+    constexpr int NSN = S::LAST ? NS : NS * R;
     float2* buf = lds + pp * L;
-    if constexpr (NS > 1 && !PRE) {
-        fft_seeds_load<N, P, NS, false>(s, tw, t);
+    float2 wn[SEED == kSeedHeld ? 1 : FPass<N, P, NSN>::NTW];
+    if constexpr (!S::LAST && SEED == kSeedAhead) {
+        fft_seeds<N, P, NSN>(tw, t, wn);
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -345,15 +316,9 @@ __device__ __forceinline__ void fft_pass(float2 (&v)[P], float2* lds, const floa
         float2 x[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) x[r] = v[b + r * B];
-        if constexpr (NS > 1) {
-            float2 pw[R];
-            twiddle_powers<R, SIGN>(&s.w[fft_seeds_before<N, P>(NS) + b * seed_count<R>()], pw);
-#pragma unroll
-            for (int r = 1; r < R; ++r) x[r] = cmul(x[r], pw[r]);
-        }
-        if constexpr (HIN && NS == 1 && B == 1) dft_half_in<R, SIGN>(x);
-        else Dft<R, SIGN>::run(x);
-        if constexpr (LAST) {
+        if constexpr (NS > 1) dft_pow2<R, SIGN, true>(x, &w[b * S::S]);
+        else dft_pow2<R, SIGN, false, HIN>(x, nullptr);
+        if constexpr (S::LAST) {
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + r * B] = x[r];
         } else {
@@ -362,27 +327,28 @@ __device__ __forceinline__ void fft_pass(float2 (&v)[P], float2* lds, const floa
             for (int r = 0; r < R; ++r) buf[padsh<SH>(base + r * NS)] = x[r];
         }
     }
-    if constexpr (!LAST) {
+    if constexpr (!S::LAST) {
         __syncthreads();
 #pragma unroll
         for (int q = 0; q < P; ++q) v[q] = buf[padsh<SH>(t + q * T)];
         pp ^= 1;
-        fft_pass<N, P, SIGN, NS * R, PRE, false>(v, lds, tw, s, t, pp);
+        if constexpr (SEED == kSeedPass) {
+            fft_seeds<N, P, NSN>(tw, t, wn);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        fft_pass<N, P, SIGN, NSN, SEED, false>(v, lds, tw, SEED == kSeedHeld ? w + (NS > 1 ? S::NTW : 0) : wn, t, pp);
     }
 }
 
-// The transform of one wavefield v in the strided mapping.  tw[m] = exp(-2 pi i m/N).  PRE:
-// every seed loaded at the start (their latency overlaps the first pass; 2 registers per seed
-// held through it), else per pass.  HIN: the points N/2 .. N-1 (slots q >= P/2) are zero on
-// input and are not read (the first pass runs half-input DFTs).
-template <int N, int P, int SIGN, bool PRE = false, bool HIN = false>
-__device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const float2* __restrict__ tw, int t, int& pp)
+// The transform of one wavefield v in the strided mapping.  tw[m] = exp(-2 pi i m/N).  SEED: see
+// above (held: the seeds).  HIN: the points N/2 .. N-1 (slots q >= P/2) are zero on input and are
+// not read (the first pass runs half-input DFTs).
+template <int N, int P, int SIGN, int SEED = kSeedPass, bool HIN = false>
+__device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const float2* __restrict__ tw, int t, int& pp,
+                                    const float2* held = nullptr)
 {
-    FftSeeds<N, P> s;
-    if constexpr (PRE) fft_seeds_load<N, P, 1, true>(s, tw, t);
-    fft_pass<N, P, SIGN, 1, PRE, HIN>(v, lds, tw, s, t, pp);
+    fft_pass<N, P, SIGN, 1, SEED, HIN>(v, lds, tw, held, t, pp);
 }
-
 
 // Wave-level variant: one 64-lane wave transforms N = 64 P points held as v[q] = x[t + 64 q].
 // All exchanges stay inside the wave, whose LDS instructions execute in program order, so a
@@ -393,7 +359,7 @@ template <int N, int NS>
 struct WPass {
     static constexpr int P = N / 64;
     static constexpr int REM = N / NS;
-    static constexpr int RMAX = P < 8 ? P : 8;
+    static constexpr int RMAX = P < 16 ? P : 16;
     static constexpr int R = REM >= RMAX ? RMAX : REM;
     static constexpr int B = P / R;
     static constexpr bool LAST = (NS * R == N);
@@ -401,28 +367,54 @@ struct WPass {
     static constexpr int NTW = NS > 1 ? B * S : 1;  // twiddle seeds per lane (1: unused slot)
 };
 
-// The twiddle seeds of pass NS of wfft<N> (as in fft): w[b S + i] = tw[seed_exp(i) k N / (NS R)].
+// The twiddle seeds of pass NS of wfft<N> (as in fft).
 template <int N, int NS>
-__device__ __forceinline__ void wfft_twiddles(const float2* __restrict__ tw, int t, float2 (&w)[WPass<N, NS>::NTW])
+__device__ __forceinline__ void wfft_seeds(const float2* __restrict__ tw, int t, float2 (&w)[WPass<N, NS>::NTW])
 {
     using S = WPass<N, NS>;
     if constexpr (NS > 1) {
 #pragma unroll
         for (int b = 0; b < S::B; ++b) {
-            const int k = (t + b * 64) & (NS - 1);
-            int ti = k * (N / (NS * S::R));
-            asm volatile("" : "+v"(ti));  // keep the loads in the transform (see fft)
-#pragma unroll
-            for (int i = 0; i < S::S; ++i) w[b * S::S + i] = tw[seed_exp(i) * ti];
+            uint32_t k = (uint32_t)(t + b * 64) & (NS - 1);
+            asm volatile("" : "+v"(k));  // keep the loads in the transform (see fft)
+            pass_seeds<N, NS, S::R>(tw, k, &w[b * S::S]);
         }
     }
 }
 
-// One pass and the passes after it; w holds this pass's twiddles.  The next pass's twiddles are
-// loaded at the start of this one, so their latency overlaps this pass's butterflies and exchange.
-template <int N, int SIGN, int NS>
+template <int N, int NS = 1>
+constexpr int wfft_seed_total()
+{
+    using S = WPass<N, NS>;
+    const int own = NS > 1 ? S::NTW : 0;
+    if constexpr (S::LAST) return own;
+    else return own + wfft_seed_total<N, NS * S::R>();
+}
+template <int N>
+struct WfftSeeds {
+    static constexpr int count = wfft_seed_total<N>();
+    float2 w[count > 0 ? count : 1];
+    template <int NS = 1>
+    __device__ __forceinline__ void load(const float2* __restrict__ tw, int t)
+    {
+        using S = WPass<N, NS>;
+        if constexpr (NS > 1) {
+            constexpr int off = count - wfft_seed_total<N, NS>();
+            float2 q[S::NTW];
+            wfft_seeds<N, NS>(tw, t, q);
+#pragma unroll
+            for (int i = 0; i < S::NTW; ++i) w[off + i] = q[i];
+        }
+        if constexpr (!S::LAST) load<NS * S::R>(tw, t);
+    }
+};
+
+// One pass and the passes after it; w: this pass's seeds (kSeedHeld: and those of the later ones).
+// Otherwise the next pass's seeds are loaded at the start of this one where that costs at most 8
+// complex registers; larger transforms load their seeds in the pass that uses them.
+template <int N, int SIGN, int NS, int SEED, bool HIN>
 __device__ __forceinline__ void wfft_pass(float2 (&v)[N / 64], float2* buf, const float2* __restrict__ tw, int t,
-                                          const float2 (&w)[WPass<N, NS>::NTW])
+                                          const float2* w)
 {
     using S = WPass<N, NS>;
     constexpr int P = S::P, R = S::R, B = S::B;
@@ -430,11 +422,9 @@ __device__ __forceinline__ void wfft_pass(float2 (&v)[N / 64], float2* buf, cons
     constexpr int SH = PassPad<NS, R>::value;
     static_assert(P % R == 0, "radix must divide the points per lane");
     constexpr int NSN = S::LAST ? NS : NS * R;
-    // prefetch only where it costs at most 7 complex registers; larger transforms load their
-    // seeds in the pass that uses them
-    constexpr bool PRE = WPass<N, NSN>::NTW <= 7;
-    float2 wn[WPass<N, NSN>::NTW];
-    if constexpr (!S::LAST && PRE) wfft_twiddles<N, NSN>(tw, t, wn);
+    constexpr bool PRE = WPass<N, NSN>::NTW <= 8;
+    float2 wn[SEED == kSeedHeld ? 1 : WPass<N, NSN>::NTW];
+    if constexpr (!S::LAST && PRE && SEED != kSeedHeld) wfft_seeds<N, NSN>(tw, t, wn);
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const int j = t + b * T;
@@ -442,13 +432,8 @@ __device__ __forceinline__ void wfft_pass(float2 (&v)[N / 64], float2* buf, cons
         float2 x[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) x[r] = v[b + r * B];
-        if constexpr (NS > 1) {
-            float2 pw[R];
-            twiddle_powers<R, SIGN>(&w[b * S::S], pw);
-#pragma unroll
-            for (int r = 1; r < R; ++r) x[r] = cmul(x[r], pw[r]);
-        }
-        Dft<R, SIGN>::run(x);
+        if constexpr (NS > 1) dft_pow2<R, SIGN, true>(x, &w[b * S::S]);
+        else dft_pow2<R, SIGN, false, HIN>(x, nullptr);
         if constexpr (S::LAST) {
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + r * B] = x[r];
@@ -467,16 +452,68 @@ __device__ __forceinline__ void wfft_pass(float2 (&v)[N / 64], float2* buf, cons
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if constexpr (!PRE) wfft_twiddles<N, NSN>(tw, t, wn);
-        wfft_pass<N, SIGN, NSN>(v, buf, tw, t, wn);
+        if constexpr (!PRE && SEED != kSeedHeld) wfft_seeds<N, NSN>(tw, t, wn);
+        wfft_pass<N, SIGN, NSN, SEED, false>(v, buf, tw, t, SEED == kSeedHeld ? w + (NS > 1 ? S::NTW : 0) : wn);
     }
 }
 
-template <int N, int SIGN>
-__device__ __forceinline__ void wfft(float2 (&v)[N / 64], float2* buf, const float2* __restrict__ tw, int t)
+// SEED: kSeedHeld with the lane's WfftSeeds in `held`, else read in the transform.  HIN: the points
+// N/2 .. N-1 (slots q >= P/2) are zero on input and are not read.
+template <int N, int SIGN, int SEED = kSeedAhead, bool HIN = false>
+__device__ __forceinline__ void wfft(float2 (&v)[N / 64], float2* buf, const float2* __restrict__ tw, int t,
+                                     const float2* held = nullptr)
 {
-    const float2 none[1] = {make_float2(0.f, 0.f)};
-    wfft_pass<N, SIGN, 1>(v, buf, tw, t, none);
+    wfft_pass<N, SIGN, 1, SEED, HIN>(v, buf, tw, t, held);
+}
+
+// Two wavefields transformed in lockstep, one LDS buffer each: every barrier serves both, and one's
+// butterflies overlap the other's exchange.  T = N / P threads; `sync` orders the LDS accesses of
+// those threads (a wave fence for T = 64).  A buffer is read before the next pass writes it, so a
+// pass takes two syncs.  held: the FftSeeds of the thread.
+template <int N, int P, int SIGN, int NS, bool HIN, class Sync>
+__device__ __forceinline__ void fft2_pass(float2 (&u)[P], float2 (&v)[P], float2* bu, float2* bv, const float2* w, int t,
+                                          Sync sync)
+{
+    using S = FPass<N, P, NS>;
+    constexpr int T = S::T, R = S::R, B = S::B;
+    constexpr int SH = PassPad<NS, R>::value;
+    auto butterflies = [&](float2(&f)[P], float2* buf) {
+#pragma unroll
+        for (int b = 0; b < B; ++b) {
+            const int j = t + b * T;
+            const int k = j & (NS - 1);
+            float2 x[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) x[r] = f[b + r * B];
+            if constexpr (NS > 1) dft_pow2<R, SIGN, true>(x, &w[b * S::S]);
+            else dft_pow2<R, SIGN, false, HIN>(x, nullptr);
+            if constexpr (S::LAST) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) f[b + r * B] = x[r];
+            } else {
+                const int base = (j - k) * R + k;
+#pragma unroll
+                for (int r = 0; r < R; ++r) buf[padsh<SH>(base + r * NS)] = x[r];
+            }
+        }
+    };
+    butterflies(u, bu);
+    butterflies(v, bv);
+    if constexpr (!S::LAST) {
+        sync();
+#pragma unroll
+        for (int q = 0; q < P; ++q) u[q] = bu[padsh<SH>(t + q * T)];
+#pragma unroll
+        for (int q = 0; q < P; ++q) v[q] = bv[padsh<SH>(t + q * T)];
+        sync();
+        fft2_pass<N, P, SIGN, NS * R, false>(u, v, bu, bv, w + (NS > 1 ? S::NTW : 0), t, sync);
+    }
+}
+template <int N, int P, int SIGN, bool HIN, class Sync>
+__device__ __forceinline__ void fft2(float2 (&u)[P], float2 (&v)[P], float2* bu, float2* bv, const float2* held, int t,
+                                     Sync sync)
+{
+    fft2_pass<N, P, SIGN, 1, HIN>(u, v, bu, bv, held, t, sync);
 }
 
 // ------------------------------------------------------------------ mixed-radix transforms
@@ -494,6 +531,25 @@ __device__ __forceinline__ void wfft(float2 (&v)[N / 64], float2* buf, const flo
 // seeds as in fft, four loads per radix-8 butterfly, measured slower here, 818 -> 943 ms for a
 // 250 x 250 3-D shot).  LDS indices are unpadded: the loads and the later passes' stores run at unit lane
 // stride, the first pass's stores at stride R.
+
+// The seeds of dft_pow2 from w alone: w^(R/2) .. w by squares, the W_8 multiple by sums.
+template <int R>
+__device__ __forceinline__ void radix_seeds(float2 w, float2 (&s)[R / 2])
+{
+    static_assert(R == 2 || R == 4 || R == 8, "radices of mixed_fft");
+    auto square = [](float2 a) { return make_float2(fmaf(a.x, a.x, -(a.y * a.y)), (a.x + a.x) * a.y); };
+    if constexpr (R == 2) {
+        s[0] = w;
+    } else if constexpr (R == 4) {
+        s[0] = square(w);
+        s[1] = w;
+    } else {
+        s[1] = square(w);
+        s[0] = square(s[1]);
+        s[2] = w;
+        s[3] = make_float2(kCos8[2] * (w.x + w.y), kCos8[2] * (w.y - w.x));
+    }
+}
 
 template <int R, int SIGN, int IT, bool PP, class Sync>
 __device__ __forceinline__ void mixed_pass(const float2* src, float2* dst, const float2* __restrict__ tw, int n,

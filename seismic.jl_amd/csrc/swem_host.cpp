@@ -446,6 +446,7 @@ static int ensure_chunk(swem_plan* p, int c, hipStream_t st)
     t.p2f = p->p2f.p;
     t.pd = p->pd.p;
     t.pdf = p->pdf.p;
+    t.taper = p->taper.p;
     t.ktab = p->ktab.p;
     t.stab = p->stab.p;
     p->resident = -1;
@@ -556,7 +557,6 @@ static March2DArgs base_args(const swem_plan* p, int c, int F)
     a.stab = p->stab.p;
     a.spec_s = p->spec_s.p;
     a.igx = p->igx.p;
-    a.taper = p->taper.p;
     a.sel = p->sel.p;
     a.sel2 = p->sel2.p;
     a.w2 = p->w2.p;

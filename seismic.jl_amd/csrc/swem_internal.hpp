@@ -69,6 +69,7 @@ struct PhaseTableArgs {
     const float* p2f;   // float counterparts (naive FP32)
     const double* pd;   // [nz][nmx] slowness perturbation (SSF)
     const float* pdf;   // float counterpart (naive FP32)
+    const float* taper; // [nmx] (SSF)
     float2* ktab;       // [nfc][nz][nref][nkh]
     float2* stab;       // [nfc][nz][nmx]
 };
@@ -101,7 +102,6 @@ struct March2DArgs {
     const float2* spec_s;   // [nf] source spectrum / sqrt(ntfft)
     const int* igx;         // [nshot]
     const float2* spec_r;   // [nshot][nmx][nf]  receiver spectra w^2 D / sqrt(ntfft)
-    const float* taper;     // [nmx]
     const uint8_t* sel;     // [nz][nkx] iref1 | cut << 7 (PSPI; 0x7f beyond nmx)
     const uint8_t* sel2;    // [nz][nkx] iref2 (PSPI linear)
     const float* w2;        // [nz][nkx] weight of iref2 (PSPI linear)

@@ -82,7 +82,7 @@ March2DShape march2d_shape(int nkx, int variant, int adj)
         break;
     case SWEM_VARIANT_PAIR:
     case SWEM_VARIANT_PACKED:
-        sh.T = nkx >= 1024 ? nkx / 16 : 64, sh.per_freq = 1, sh.max_block = sh.T, sh.bufs = nkx >= 1024 ? 2 : 1;
+        sh.T = nkx >= 1024 ? nkx / 16 : 64, sh.per_freq = 1, sh.max_block = sh.T, sh.bufs = 2;
         break;
     case SWEM_VARIANT_PAIR8:
         sh.T = nkx / 8, sh.per_freq = 1, sh.max_block = sh.T, sh.bufs = 2;

@@ -88,12 +88,15 @@ __device__ __forceinline__ void buf_store2(__amdgpu_buffer_rsrc_t r, uint32_t of
 }
 
 // kz phase of the point k = t + q T of the strided mapping from a table row (L is even in kx,
-// the row holds kk = 0..N/2): kk = k for q < P/2, N - k = (P - q) T - t above.
+// the row holds kk = 0..N/2): kk = k for q < P/2, N - k = (P - q) T - t above.  Byte offsets of 32
+// bits from the wave-uniform row: two offset registers and immediates for all P loads.
 template <int N, int P>
 __device__ __forceinline__ float2 kload(const float2* __restrict__ row, int t, int q)
 {
     constexpr int T = N / P;
-    return row[q < P / 2 ? t + q * T : (P - q) * T - t];
+    const char* r = reinterpret_cast<const char*>(row);
+    const uint32_t lo = 8u * (uint32_t)t, hi = 8u * (uint32_t)(T - t);
+    return *reinterpret_cast<const float2*>(q < P / 2 ? r + lo + q * T * 8 : r + hi + (P - 1 - q) * T * 8);
 }
 
 __device__ __forceinline__ float2 cmul_c(float2 x, float2 L, bool conj) { return conj ? cmulc(x, L) : cmul(x, L); }
@@ -109,36 +112,49 @@ __device__ __forceinline__ void kload_row(float2 (&L)[P], const float2* __restri
     __builtin_amdgcn_sched_barrier(0);
 }
 
-// One x-transform of the wavefield: a wave-level transform (WAVE, P = N/64, no barriers) or a
-// subgroup transform through ping-pong buffers.
-template <int N, int P, int SIGN, bool WAVE, bool PRE = false, bool HIN = false>
-__device__ __forceinline__ void xfft(float2 (&v)[P], float2* lds, const float2* __restrict__ tw, int t, int& pp)
-{
-    if constexpr (WAVE) {
-        static_assert(P * 64 == N, "wave transforms hold N/64 points per lane");
-        wfft<N, SIGN>(v, lds, tw, t);
-    } else
-        fft<N, P, SIGN, PRE, HIN>(v, lds, tw, t, pp);
-}
-
-// Transform policies of the step functions.  XPow2: the transform length is the register array
-// length N (a power of two); PRE: every twiddle seed of a transform loaded at its start, two
-// registers per seed held through the first pass (measured at nkx 2048, 64 shots: 6-11 % faster
-// than per-pass seeds in every 2-D mode, migration and modelling).  XBlue: a transform of runtime length n = nkx (any length) through
+// Transform policies of the step functions, one object per thread.  XPow2: the transform length is
+// the register array length N (a power of two), a wave-level transform (WAVE, P = N/64, no
+// barriers) or a subgroup transform through ping-pong buffers; SEED: where its twiddle seeds come
+// from (swem_fft.hpp).  XBlue: a transform of runtime length n = nkx (any length) through
 // two power-of-two transforms of the array length M >= 2 n - 1 (Bluestein): with
 // w_j = exp(SIGN i pi j^2 / n),  X_k = w_k sum_j (x_j w_j) conj(w_(k-j)),  the sum a cyclic
 // convolution of length M taken as IFFT_M(FFT_M(x w) B) with B = FFT_M(conj w, wrapped) / M
 // built in FP64.  Entries j, k >= n of the array are zero on input and on output.  The PSPI
 // selection tables keep the array length as their row stride (0x7f padding beyond nmx) in both.
-template <int N, int P, bool PRE = true>
+template <int N, int P, bool WAVE_, int SEED>
+struct HeldSeeds {
+    __device__ __forceinline__ HeldSeeds(const float2*, int) {}
+    __device__ __forceinline__ const float2* ptr() const { return nullptr; }
+};
+template <int N, int P>
+struct HeldSeeds<N, P, false, kSeedHeld> {
+    FftSeeds<N, P> s;
+    __device__ __forceinline__ HeldSeeds(const float2* tw, int t) { s.load(tw, t); }
+    __device__ __forceinline__ const float2* ptr() const { return s.w; }
+};
+template <int N, int P>
+struct HeldSeeds<N, P, true, kSeedHeld> {
+    WfftSeeds<N> s;
+    __device__ __forceinline__ HeldSeeds(const float2* tw, int t) { s.load(tw, t); }
+    __device__ __forceinline__ const float2* ptr() const { return s.w; }
+};
+
+template <int N, int P, bool WAVE_ = false, int SEED = kSeedAhead>
 struct XPow2 {
+    HeldSeeds<N, P, WAVE_, SEED> held;
+    __device__ __forceinline__ XPow2(const March2DArgs& a, int t) : held(a.tw, t) {}
     // HIN: slots q >= P/2 are zero on input (see fft)
     template <int SIGN, bool WAVE, bool HIN = false>
-    __device__ __forceinline__ static void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp)
+    __device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp) const
     {
-        xfft<N, P, SIGN, WAVE, PRE, HIN>(v, lds, a.tw, t, pp);
+        static_assert(WAVE == WAVE_, "transform of another shape");
+        if constexpr (WAVE) {
+            static_assert(P * 64 == N, "wave transforms hold N/64 points per lane");
+            wfft<N, SIGN, SEED, HIN>(v, lds, a.tw, t, held.ptr());
+        } else
+            swem::fft<N, P, SIGN, SEED, HIN>(v, lds, a.tw, t, pp, held.ptr());
     }
-    __device__ __forceinline__ static void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs&, int t)
+    __device__ __forceinline__ void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs&, int t) const
     {
         swem::kload_row<N, P>(L, row, t);
     }
@@ -147,8 +163,18 @@ struct XPow2 {
 template <int M, int P>
 struct XBlue {
     static constexpr int T = M / P;
+    uint32_t koff[P];  // byte offsets of the thread's points in a kz row (0 beyond n)
+    __device__ __forceinline__ XBlue(const March2DArgs& a, int t)
+    {
+        const int n = a.nkx;
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+            const int k = t + q * T;
+            koff[q] = 8u * (uint32_t)(k < n ? (k <= n / 2 ? k : n - k) : 0);
+        }
+    }
     template <int SIGN, bool WAVE, bool HIN = false>
-    __device__ __forceinline__ static void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp)
+    __device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp) const
     {
         static_assert(!WAVE, "Bluestein transforms use the subgroup FFT");
         chirp_mul<SIGN>(v, a, t);
@@ -167,7 +193,7 @@ struct XBlue {
     }
     // v_j <- v_j w_j for j < n, 0 beyond (the chirp is reloaded rather than kept in registers)
     template <int SIGN>
-    __device__ __forceinline__ static void chirp_mul(float2 (&v)[P], const March2DArgs& a, int t)
+    __device__ __forceinline__ void chirp_mul(float2 (&v)[P], const March2DArgs& a, int t) const
     {
         const int n = a.nkx;
         float2 w[P];
@@ -181,14 +207,10 @@ struct XBlue {
 #pragma unroll
         for (int q = 0; q < P; ++q) v[q] = cmul(v[q], w[q]);
     }
-    __device__ __forceinline__ static void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs& a, int t)
+    __device__ __forceinline__ void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs&, int) const
     {
-        const int n = a.nkx;
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
-            const int k = t + q * T;
-            L[q] = row[k < n ? (k <= n / 2 ? k : n - k) : 0];
-        }
+        for (int q = 0; q < P; ++q) L[q] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(row) + koff[q]);
         __builtin_amdgcn_sched_barrier(0);
     }
 };
@@ -197,17 +219,31 @@ struct XBlue {
 // transformed in the subgroup's two LDS buffers (mixed_fft); entries j >= n stay zero.
 template <int M, int P>
 struct XMixed {
+    XBlue<M, P> b;  // the kz row offsets
+    __device__ __forceinline__ XMixed(const March2DArgs& a, int t) : b(a, t) {}
     template <int SIGN, bool WAVE, bool HIN = false>
-    __device__ __forceinline__ static void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp)
+    __device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp) const
     {
         static_assert(!WAVE, "mixed-radix transforms use the subgroup buffers");
         mixed_fft<M, P, SIGN, true>(v, lds, lds + LdsLen<M>::value, a.tw, a.mr, t, pp, []() { __syncthreads(); });
     }
-    __device__ __forceinline__ static void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs& a, int t)
+    __device__ __forceinline__ void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs& a, int t) const
     {
-        XBlue<M, P>::kload_row(L, row, a, t);
+        b.kload_row(L, row, a, t);
     }
 };
+
+template <int T>
+__device__ __forceinline__ void subgroup_sync()
+{
+    if constexpr (T == 64) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    } else {
+        __syncthreads();
+    }
+}
 
 struct StepCtx {
     int t, iz, fc;  // thread within the subgroup, depth index, frequency index within the chunk
@@ -225,68 +261,81 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t ss_row(const March2DArgs& a, c
     return buf_rsrc(a.stab + ((size_t)c.fc * a.nz + c.iz) * a.nmx, (uint32_t)a.nmx * 8u);
 }
 
-// ssop adjoint branch (wem.c:313-320, 334-359) on one wavefield.  ACT = false turns the step
-// into FFT / IFFT with unit phases (a numerical identity) so every subgroup of a workgroup runs
-// the same barriers when only one of the two wavefields is stepped at a depth.
-template <int N, int P, bool WAVE, bool ACT, class X = XPow2<N, P>>
-__device__ __forceinline__ void ssf_adj_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a,
-                                             const StepCtx& c, bool conj, const float (&tap)[P])
+// The split-step phases (taper included) of the live slots q < Q; lanes x >= nmx read zero, so the
+// product zeroes them.
+template <int T, int Q>
+__device__ __forceinline__ void ss_load(float2 (&sp)[Q], const March2DArgs& a, const StepCtx& c)
 {
-    constexpr int T = N / P;
-    X::template fft<-1, WAVE>(u, lds, a, c.t, pp);
+    StepCtx u = c;
+    u.iz = __builtin_amdgcn_readfirstlane(c.iz);
+    const auto sr = ss_row(a, u);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) sp[q] = buf_load2(sr, (uint32_t)(c.t + q * T) * 8u);
+    __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first use
+}
+
+template <int P, int Q>
+__device__ __forceinline__ void zero_tail(float2 (&u)[P])
+{
+#pragma unroll
+    for (int q = Q; q < P; ++q) u[q] = make_float2(0.f, 0.f);
+}
+
+// Step functions.  HALF (2 nmx <= N): the slots q >= P / 2 of a wavefield are zero before and after a
+// step, so the first pass of its transform runs half-input butterflies, the last pass of the inverse
+// drops the upper outputs and the pointwise work covers Q = P / 2 slots.
+
+// ssop adjoint branch (wem.c:313-320, 334-359) on one wavefield: FFT, kz phase, IFFT, split-step
+// phase and taper.  ACT = false turns the step into FFT / IFFT with unit phases (a numerical
+// identity) so every subgroup of a workgroup runs the same barriers when only one of the two
+// wavefields is stepped at a depth.
+template <int N, int P, bool WAVE, bool ACT, bool HALF, class X>
+__device__ __forceinline__ void ssf_adj_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a,
+                                             const X& xf, const StepCtx& c, bool conj)
+{
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
+    float2 L[P], sp[Q];
+    if constexpr (ACT) xf.kload_row(L, krow(a, c, 0), a, c.t);
+    xf.template fft<-1, WAVE, HALF>(u, lds, a, c.t, pp);
     if constexpr (ACT) {
-        float2 L[P];
-        X::kload_row(L, krow(a, c, 0), a, c.t);
 #pragma unroll
         for (int q = 0; q < P; ++q) u[q] = cmul_c(u[q], L[q], conj);
+        ss_load<T, Q>(sp, a, c);
     } else {
 #pragma unroll
         for (int q = 0; q < P; ++q) u[q] = cscale(u[q], a.inv_nk);
     }
-    X::template fft<+1, WAVE>(u, lds, a, c.t, pp);
+    xf.template fft<+1, WAVE>(u, lds, a, c.t, pp);
     if constexpr (ACT) {
-        const auto sr = ss_row(a, c);
-        float2 sp[P];
 #pragma unroll
-        for (int q = 0; q < P; ++q) sp[q] = buf_load2(sr, (uint32_t)(c.t + q * T) * 8u);
-        __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first use
-#pragma unroll
-        for (int q = 0; q < P; ++q)  // zero beyond nmx: the split-step row reads zero there
-            u[q] = cscale(cmul_c(u[q], sp[q], conj), tap[q]);
+        for (int q = 0; q < Q; ++q) u[q] = cmul_c(u[q], sp[q], conj);
     } else {
 #pragma unroll
-        for (int q = 0; q < P; ++q)
+        for (int q = 0; q < Q; ++q)
             if (c.t + q * T >= a.nmx) u[q] = make_float2(0.f, 0.f);
     }
+    zero_tail<P, Q>(u);
 }
 
-// ssop forward branch with dz < 0 (wem.c:321-332, 334-348, 362-369): taper, split-step
-// phase, FFT, kz phase, IFFT.
-template <int N, int P, bool WAVE, class X = XPow2<N, P>>
+// ssop forward branch with dz < 0 (wem.c:321-332, 334-348, 362-369): taper and split-step phase,
+// FFT, kz phase, IFFT.
+template <int N, int P, bool WAVE, bool HALF, class X>
 __device__ __forceinline__ void ssf_fwd_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a,
-                                             const StepCtx& c, const float (&tap)[P])
+                                             const X& xf, const StepCtx& c, const float2 (&sp)[HALF ? P / 2 : P])
 {
-    constexpr int T = N / P;
-    const auto sr = ss_row(a, c);
-    {
-        float2 sp[P];
+    constexpr int Q = HALF ? P / 2 : P;
+    float2 L[P];
+    xf.kload_row(L, krow(a, c, 0), a, c.t);
 #pragma unroll
-        for (int q = 0; q < P; ++q) sp[q] = buf_load2(sr, (uint32_t)(c.t + q * T) * 8u);
-        __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first use
+    for (int q = 0; q < Q; ++q) u[q] = cmulc(u[q], sp[q]);
+    xf.template fft<-1, WAVE, HALF>(u, lds, a, c.t, pp);
 #pragma unroll
-        for (int q = 0; q < P; ++q) u[q] = cmulc(cscale(u[q], tap[q]), sp[q]);
-    }
-    X::template fft<-1, WAVE>(u, lds, a, c.t, pp);
-    {
-        float2 L[P];
-        X::kload_row(L, krow(a, c, 0), a, c.t);
+    for (int q = 0; q < P; ++q) u[q] = cmulc(u[q], L[q]);
+    xf.template fft<+1, WAVE>(u, lds, a, c.t, pp);
 #pragma unroll
-        for (int q = 0; q < P; ++q) u[q] = cmulc(u[q], L[q]);
-    }
-    X::template fft<+1, WAVE>(u, lds, a, c.t, pp);
-#pragma unroll
-    for (int q = 0; q < P; ++q)
-        if (c.t + q * T >= a.nmx) u[q] = make_float2(0.f, 0.f);
+    for (int q = 0; q < Q; ++q)
+        if (c.t + q * (N / P) >= a.nmx) u[q] = make_float2(0.f, 0.f);
+    zero_tail<P, Q>(u);
 }
 
 // Weight of reference velocity ir at a point with selection byte s1 (iref1 | cut<<7), iref2
@@ -304,18 +353,25 @@ __device__ __forceinline__ float pspi_linear_weight(int ir, uint8_t s1, uint8_t 
 // pspiop with the reference structure (wem.c:409-460): FFT, for each vref phase + IFFT, then
 // per-x selection.  Compat: u = Re(dref[iref1]) when cut else dref[iref1]; linear: weights.
 // The selection rows are padded to N columns (0x7f beyond nmx: no vref selected).
-template <int N, int P, int MODE, bool WAVE, bool ACT, class X = XPow2<N, P>>
-__device__ __forceinline__ void pspi_select_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a,
+template <int N, int P, int MODE, bool WAVE, bool ACT, bool HALF, class X>
+__device__ __forceinline__ void pspi_select_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a, const X& xf,
                                                  const StepCtx& c, bool conj)
 {
-    constexpr int T = N / P;
-    X::template fft<-1, WAVE>(u, lds, a, c.t, pp);
-    float2 U[P];
-    uint8_t s1[P], s2[P];
-    float w2[P];
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
+    uint32_t todo = a.used[c.iz] & ((1u << a.nref) - 1u);
+    const int first = __builtin_ctz(todo | 0x80000000u);
+    // each vref's row is read while the transform before its use runs
+    float2 L[P];
+    auto next_row = [&]() {
+        if (ACT && todo) xf.kload_row(L, krow(a, c, __builtin_ctz(todo)), a, c.t);
+    };
+    next_row();
+    float2 U[Q];
+    uint8_t s1[Q], s2[Q];
+    float w2[Q];
     const size_t rowx = (size_t)c.iz * N;
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         const int x = c.t + q * T;
         s1[q] = a.sel[rowx + x];
         if constexpr (MODE == kModePspiLinear) {
@@ -324,119 +380,95 @@ __device__ __forceinline__ void pspi_select_step(float2 (&u)[P], float2* lds, in
         }
         U[q] = make_float2(0.f, 0.f);
     }
-    const uint32_t used = a.used[c.iz];
-    const int first = __builtin_ctz(used | 0x80000000u);
-    for (int ir = 0; ir < a.nref; ++ir) {
-        if (!((used >> ir) & 1u)) continue;
+    xf.template fft<-1, WAVE, HALF>(u, lds, a, c.t, pp);
+    while (todo) {
+        const int ir = __builtin_ctz(todo);
+        todo &= todo - 1u;
         float2 B[P];
-        if constexpr (ACT) {
-            X::kload_row(B, krow(a, c, ir), a, c.t);
 #pragma unroll
-            for (int q = 0; q < P; ++q) B[q] = cmul_c(u[q], B[q], conj);
-        } else {
+        for (int q = 0; q < P; ++q) B[q] = ACT ? cmul_c(u[q], L[q], conj) : cscale(u[q], a.inv_nk);
+        next_row();
+        xf.template fft<+1, WAVE>(B, lds, a, c.t, pp);
 #pragma unroll
-            for (int q = 0; q < P; ++q) B[q] = cscale(u[q], a.inv_nk);
-        }
-        X::template fft<+1, WAVE>(B, lds, a, c.t, pp);
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             if constexpr (!ACT) {
                 if (ir == first) U[q] = B[q];
             } else if constexpr (MODE == kModePspiCompat) {
                 if ((s1[q] & 0x7f) == ir) U[q] = (s1[q] >> 7) ? make_float2(B[q].x, 0.f) : B[q];
             } else {
-                U[q] = cadd(U[q], cscale(B[q], pspi_linear_weight(ir, s1[q], s2[q], w2[q])));
+                const float wt = pspi_linear_weight(ir, s1[q], s2[q], w2[q]);
+                U[q] = make_float2(fmaf(B[q].x, wt, U[q].x), fmaf(B[q].y, wt, U[q].y));
             }
         }
     }
 #pragma unroll
-    for (int q = 0; q < P; ++q) u[q] = (c.t + q * T < a.nmx) ? U[q] : make_float2(0.f, 0.f);
+    for (int q = 0; q < Q; ++q) u[q] = (c.t + q * T < a.nmx) ? U[q] : make_float2(0.f, 0.f);
+    zero_tail<P, Q>(u);
 }
 
 // Exact adjoint of the linear select-after step, for the forward receiver (dz < 0):
 // u <- IFFT( sum_ir conj(L_ir) FFT(W_ir u) ).
-template <int N, int P, bool WAVE, class X = XPow2<N, P>>
-__device__ __forceinline__ void pspi_weight_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a,
+template <int N, int P, bool WAVE, bool HALF, class X>
+__device__ __forceinline__ void pspi_weight_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a, const X& xf,
                                                  const StepCtx& c)
 {
-    constexpr int T = N / P;
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
     float2 acc[P];
-    uint8_t s1[P], s2[P];
-    float w2[P];
+    uint8_t s1[Q], s2[Q];
+    float w2[Q];
     const size_t rowx = (size_t)c.iz * N;
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         const int x = c.t + q * T;
         s1[q] = a.sel[rowx + x];
         s2[q] = a.sel2[rowx + x];
         w2[q] = a.w2[rowx + x];
-        acc[q] = make_float2(0.f, 0.f);
     }
-    const uint32_t used = a.used[c.iz];
-    for (int ir = 0; ir < a.nref; ++ir) {
-        if (!((used >> ir) & 1u)) continue;
-        float2 B[P];
 #pragma unroll
-        for (int q = 0; q < P; ++q) B[q] = cscale(u[q], pspi_linear_weight(ir, s1[q], s2[q], w2[q]));
-        X::template fft<-1, WAVE>(B, lds, a, c.t, pp);
-        const float2* row = krow(a, c, ir);
-        float2 L[P];
-        X::kload_row(L, row, a, c.t);
+    for (int q = 0; q < P; ++q) acc[q] = make_float2(0.f, 0.f);
+    for (uint32_t todo = a.used[c.iz] & ((1u << a.nref) - 1u); todo; todo &= todo - 1u) {
+        const int ir = __builtin_ctz(todo);
+        float2 L[P], B[P];
+        xf.kload_row(L, krow(a, c, ir), a, c.t);
 #pragma unroll
-        for (int q = 0; q < P; ++q) acc[q] = cadd(acc[q], cmulc(B[q], L[q]));
+        for (int q = 0; q < Q; ++q) B[q] = cscale(u[q], pspi_linear_weight(ir, s1[q], s2[q], w2[q]));
+        zero_tail<P, Q>(B);
+        xf.template fft<-1, WAVE, HALF>(B, lds, a, c.t, pp);
+#pragma unroll
+        for (int q = 0; q < P; ++q) {
+            acc[q].x = fmaf(B[q].x, L[q].x, fmaf(B[q].y, L[q].y, acc[q].x));
+            acc[q].y = fmaf(B[q].y, L[q].x, fmaf(-B[q].x, L[q].y, acc[q].y));
+        }
     }
-    X::template fft<+1, WAVE>(acc, lds, a, c.t, pp);
+    xf.template fft<+1, WAVE>(acc, lds, a, c.t, pp);
 #pragma unroll
-    for (int q = 0; q < P; ++q) u[q] = (c.t + q * T < a.nmx) ? acc[q] : make_float2(0.f, 0.f);
+    for (int q = 0; q < Q; ++q) u[q] = (c.t + q * T < a.nmx) ? acc[q] : make_float2(0.f, 0.f);
+    zero_tail<P, Q>(u);
 }
 
 // Source / adjoint-receiver step of either method (select-after for PSPI).  act is uniform
 // over the subgroup: the branch is taken once per step, not per element.
-template <int N, int P, int MODE, bool WAVE, class X = XPow2<N, P>>
-__device__ __forceinline__ void adj_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a, const StepCtx& c,
-                                         bool act, bool conj, const float (&tap)[P])
+template <int N, int P, int MODE, bool WAVE, bool HALF, class X>
+__device__ __forceinline__ void adj_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a, const X& xf,
+                                         const StepCtx& c, bool act, bool conj)
 {
     if constexpr (MODE == kModeSSF) {
         if (act)
-            ssf_adj_step<N, P, WAVE, true, X>(u, lds, pp, a, c, conj, tap);
+            ssf_adj_step<N, P, WAVE, true, HALF, X>(u, lds, pp, a, xf, c, conj);
         else
-            ssf_adj_step<N, P, WAVE, false, X>(u, lds, pp, a, c, conj, tap);
+            ssf_adj_step<N, P, WAVE, false, HALF, X>(u, lds, pp, a, xf, c, conj);
     } else {
         if (act)
-            pspi_select_step<N, P, MODE, WAVE, true, X>(u, lds, pp, a, c, conj);
+            pspi_select_step<N, P, MODE, WAVE, true, HALF, X>(u, lds, pp, a, xf, c, conj);
         else
-            pspi_select_step<N, P, MODE, WAVE, false, X>(u, lds, pp, a, c, conj);
-    }
-}
-
-// Forward-receiver step (dz < 0).
-template <int N, int P, int MODE, bool WAVE, class X = XPow2<N, P>>
-__device__ __forceinline__ void fwd_step(float2 (&u)[P], float2* lds, int& pp, const March2DArgs& a, const StepCtx& c,
-                                         const float (&tap)[P])
-{
-    if constexpr (MODE == kModeSSF)
-        ssf_fwd_step<N, P, WAVE, X>(u, lds, pp, a, c, tap);
-    else if constexpr (MODE == kModePspiCompat)
-        pspi_select_step<N, P, MODE, WAVE, true, X>(u, lds, pp, a, c, true);
-    else
-        pspi_weight_step<N, P, WAVE, X>(u, lds, pp, a, c);
-}
-
-template <int N, int P, int MODE>
-__device__ __forceinline__ void load_taper(float (&tap)[P], const March2DArgs& a, int t)
-{
-    constexpr int T = N / P;
-#pragma unroll
-    for (int q = 0; q < P; ++q) {
-        const int x = t + q * T;
-        tap[q] = (MODE == kModeSSF && x < a.nmx) ? a.taper[x] : 1.f;
+            pspi_select_step<N, P, MODE, WAVE, false, HALF, X>(u, lds, pp, a, xf, c, conj);
     }
 }
 
 // Migration march shared by both kernel families.  The workgroup has 2F subgroups of T
 // threads; subgroup s = 2f is the source and 2f + 1 the receiver of frequency f.  BUFS LDS
 // buffers of LdsLen<N> complex per subgroup (1 for wave transforms, 2 for ping-pong).
-template <int N, int P, int MODE, bool WAVE>
+template <int N, int P, int MODE, bool WAVE, class X = XPow2<N, P, WAVE>>
 __device__ __forceinline__ void adj_body(const March2DArgs& a)
 {
     constexpr int T = N / P;
@@ -461,10 +493,9 @@ __device__ __forceinline__ void adj_body(const March2DArgs& a)
     float2* lds = smem + (size_t)s * BUFS * L;
     const float2* xsrc = smem + (size_t)(2 * f) * BUFS * L;
     int pp = 0;
+    const X xf(a, t);
 
     float2 u[P];
-    float tap[P];
-    load_taper<N, P, MODE>(tap, a, t);
     const int igx = a.igx[shot];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
@@ -480,7 +511,7 @@ __device__ __forceinline__ void adj_body(const March2DArgs& a)
         c.iz = iz;
         const float z = a.oz + a.dz * (float)iz;
         const bool ds = z >= a.sz, dr = z >= a.gz;
-        if (ds || dr) adj_step<N, P, MODE, WAVE>(u, lds, pp, a, c, src ? ds : dr, src, tap);
+        if (ds || dr) adj_step<N, P, MODE, WAVE, false, X>(u, lds, pp, a, xf, c, src ? ds : dr, src);
         // imaging condition (wem.c:243-247): the source subgroup hands its wavefield over in LDS
         const int xb = pp * L;
         if (src) {
@@ -525,10 +556,13 @@ __device__ __forceinline__ void adj_body(const March2DArgs& a)
 }
 
 // Modelling march: NSUB subgroups, one frequency each, no interaction between subgroups.
-template <int N, int P, int MODE, bool WAVE, class X = XPow2<N, P>>
+//
+// The receiver's depth reads (stored source, image, split-step phases) are issued one depth ahead:
+// they come from HBM and would otherwise be waited for at the start of every step.
+template <int N, int P, int MODE, bool WAVE, bool HALF, class X = XPow2<N, P, WAVE>>
 __device__ __forceinline__ void fwd_body(const March2DArgs& a)
 {
-    constexpr int T = N / P;
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
     constexpr int L = LdsLen<N>::value;
     constexpr int BUFS = WAVE ? 1 : 2;
     extern __shared__ float2 smem[];
@@ -537,7 +571,7 @@ __device__ __forceinline__ void fwd_body(const March2DArgs& a)
     if (g < 0) return;
     const int NSUB = blockDim.x / T;
     const int tid = threadIdx.x, s = tid / T, t = tid - s * T;
-    const int fc = g * NSUB + s;
+    const int fc = __builtin_amdgcn_readfirstlane(g * NSUB + s);  // uniform: T >= 64
     const bool active = fc < a.nfc;
     const int fl = a.f0 + fc;
     StepCtx c;
@@ -545,10 +579,11 @@ __device__ __forceinline__ void fwd_body(const March2DArgs& a)
     c.fc = __builtin_amdgcn_readfirstlane(active ? fc : 0);
     float2* lds = smem + (size_t)s * BUFS * L;
     int pp = 0;
-    float tap[P];
-    load_taper<N, P, MODE>(tap, a, t);
+    const X xf(a, t);
     const int igx = a.igx[shot];
-    float2* sm = a.smig + ((size_t)shot * a.nfc + (active ? fc : 0)) * (size_t)a.nz * a.nmx;
+    // from the wave-uniform fc: a buffer resource of a base the compiler cannot prove uniform costs a
+    // loop over the lanes at every access
+    float2* sm = a.smig + ((size_t)shot * a.nfc + c.fc) * (size_t)a.nz * a.nmx;
 
     float2 u[P];
 #pragma unroll
@@ -561,52 +596,87 @@ __device__ __forceinline__ void fwd_body(const March2DArgs& a)
         c.iz = iz;
         const float z = a.oz + a.dz * (float)iz;
         const bool ds = z >= a.sz;
-        if (ds) adj_step<N, P, MODE, WAVE, X>(u, lds, pp, a, c, true, true, tap);
+        if (ds) adj_step<N, P, MODE, WAVE, HALF, X>(u, lds, pp, a, xf, c, true, true);
         if (active) {
             const auto sr = buf_rsrc(sm + (size_t)iz * a.nmx, (uint32_t)a.nmx * 8u);
 #pragma unroll
-            for (int q = 0; q < P; ++q)
+            for (int q = 0; q < Q; ++q)
                 buf_store2(sr, (uint32_t)(t + q * T) * 8u, ds ? u[q] : make_float2(0.f, 0.f));
         }
     }
     // receiver march upward with injection (wem.c:266-276)
 #pragma unroll
     for (int q = 0; q < P; ++q) u[q] = make_float2(0.f, 0.f);
-    for (int iz = a.nz - 1; iz >= 0; --iz) {
+    float2 sv[Q], sp[Q];
+    float mv[Q];
+    auto fetch = [&](int iz) {
         c.iz = iz;
-        const float z = a.oz + a.dz * (float)iz;
-        if (!(z >= a.gz)) continue;
         if (active) {
             const auto sr = buf_rsrc(sm + (size_t)iz * a.nmx, (uint32_t)a.nmx * 8u);
             const auto mr = buf_rsrc(a.mT + (size_t)iz * a.nmx, (uint32_t)a.nmx * 4u);
-            float2 sv[P];
-            float mv[P];
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const uint32_t x = (uint32_t)(t + q * T);
                 sv[q] = buf_load2(sr, x * 8u);
                 mv[q] = buf_load1(mr, x * 4u);
             }
-            __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first use
+        } else {
 #pragma unroll
-            for (int q = 0; q < P; ++q) u[q] = cadd(u[q], cscale(sv[q], mv[q]));
+            for (int q = 0; q < Q; ++q) {
+                sv[q] = make_float2(0.f, 0.f);
+                mv[q] = 0.f;
+            }
         }
-        fwd_step<N, P, MODE, WAVE, X>(u, lds, pp, a, c, tap);
+        if constexpr (MODE == kModeSSF) ss_load<T, Q>(sp, a, c);
+        __builtin_amdgcn_sched_barrier(0);  // all loads in flight before the first use
+    };
+    auto stepped = [&](int iz) { return a.oz + a.dz * (float)iz >= a.gz; };
+    int iz = a.nz - 1;
+    while (iz >= 0 && !stepped(iz)) --iz;
+    if (iz >= 0) fetch(iz);
+    while (iz >= 0) {
+        int next = iz - 1;
+        while (next >= 0 && !stepped(next)) --next;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) u[q] = make_float2(fmaf(sv[q].x, mv[q], u[q].x), fmaf(sv[q].y, mv[q], u[q].y));
+        if constexpr (MODE == kModeSSF) {
+            float2 L1[P];
+            c.iz = iz;
+            xf.kload_row(L1, krow(a, c, 0), a, t);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) u[q] = cmulc(u[q], sp[q]);
+            if (next >= 0) fetch(next);
+            xf.template fft<-1, WAVE, HALF>(u, lds, a, t, pp);
+#pragma unroll
+            for (int q = 0; q < P; ++q) u[q] = cmulc(u[q], L1[q]);
+            xf.template fft<+1, WAVE>(u, lds, a, t, pp);
+            zero_tail<P, Q>(u);  // within the live slots the next split-step row cuts at nmx
+        } else {
+            if (next >= 0) fetch(next);
+            c.iz = iz;
+            if constexpr (MODE == kModePspiCompat)
+                pspi_select_step<N, P, MODE, WAVE, true, HALF, X>(u, lds, pp, a, xf, c, true);
+            else
+                pspi_weight_step<N, P, WAVE, HALF, X>(u, lds, pp, a, xf, c);
+        }
+        iz = next;
     }
     if (active) {
         const auto dr = buf_rsrc(a.dgw + (size_t)shot * a.nmx * a.nf, (uint32_t)a.nmx * a.nf * 8u);
 #pragma unroll
-        for (int q = 0; q < P; ++q) buf_store2(dr, ((uint32_t)(t + q * T) * (uint32_t)a.nf + (uint32_t)fl) * 8u, u[q]);
+        for (int q = 0; q < Q; ++q) buf_store2(dr, ((uint32_t)(t + q * T) * (uint32_t)a.nf + (uint32_t)fl) * 8u, u[q]);
     }
 }
 
 // Migration march with one subgroup per frequency that steps the source, then the receiver,
 // through the same LDS buffers (variant PAIR).  One frequency per workgroup; the imaging
 // condition is register-local.
-template <int N, int P, int MODE, bool WAVE, class X = XPow2<N, P>>
+template <int N, int P, int MODE, bool WAVE, bool HALF, class X = XPow2<N, P, WAVE>>
 __device__ __forceinline__ void adj_body_pair(const March2DArgs& a)
 {
-    constexpr int T = N / P;
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
+    // split-step steps on a power-of-two length: both wavefields in lockstep (fft2)
+    constexpr bool LOCK = MODE == kModeSSF && std::is_same<X, XPow2<N, P, WAVE, kSeedHeld>>::value;
     extern __shared__ float2 smem[];
     int g, shot;
     decode_block(a.ngroups, a.nshot, g, shot);
@@ -621,8 +691,7 @@ __device__ __forceinline__ void adj_body_pair(const March2DArgs& a)
     c.fc = __builtin_amdgcn_readfirstlane(active ? fc : 0);
     const float factor = iw == 0 ? 1.f : 2.f;
     int pp = 0;
-    float tap[P];
-    load_taper<N, P, MODE>(tap, a, t);
+    const X xf(a, t);
     const int igx = a.igx[shot];
     float2 us[P], ur[P];
 #pragma unroll
@@ -632,17 +701,66 @@ __device__ __forceinline__ void adj_body_pair(const March2DArgs& a)
         ur[q] = (active && x < a.nmx) ? a.spec_r[((size_t)shot * a.nmx + x) * a.nf + fl] : make_float2(0.f, 0.f);
     }
     float* part = a.partial + ((size_t)shot * a.ngroups + g) * (size_t)a.nz * a.nmx;
-    for (int iz = 0; iz < a.nz; ++iz) {
+    auto image = [&](int iz, bool dr) {  // imaging condition (wem.c:243-247)
+        const auto pr = buf_rsrc(part + (size_t)iz * a.nmx, (uint32_t)a.nmx * 4u);
+#pragma unroll
+        for (int q = 0; q < Q; ++q)
+            buf_store1_nt(pr, (uint32_t)(t + q * T) * 4u, dr ? factor * (ur[q].x * us[q].x + ur[q].y * us[q].y) : 0.f);
+    };
+    // the depths above the deeper of source and receivers, where one of the two steps alone
+    int iz = 0;
+    for (; iz < a.nz; ++iz) {
         c.iz = iz;
         const float z = a.oz + a.dz * (float)iz;
         const bool ds = z >= a.sz, dr = z >= a.gz;
-        if (ds) adj_step<N, P, MODE, WAVE, X>(us, smem, pp, a, c, true, true, tap);
-        if (dr) adj_step<N, P, MODE, WAVE, X>(ur, smem, pp, a, c, true, false, tap);
-        // imaging condition (wem.c:243-247)
-        const auto pr = buf_rsrc(part + (size_t)iz * a.nmx, (uint32_t)a.nmx * 4u);
+        if (LOCK && ds && dr) break;
+        if (ds) adj_step<N, P, MODE, WAVE, HALF, X>(us, smem, pp, a, xf, c, true, true);
+        if (dr) adj_step<N, P, MODE, WAVE, HALF, X>(ur, smem, pp, a, xf, c, true, false);
+        image(iz, dr);
+    }
+    if constexpr (LOCK) {
+        // Both step: one read of each phase row for the two, a depth ahead (the rows stream from
+        // HBM; a 256-point step lasts less than their latency), and the transforms in lockstep.
+        auto sync = [] { subgroup_sync<T>(); };
+        const float2* held = xf.held.ptr();
+        float2 *bu = smem, *bv = smem + LdsLen<N>::value;
+        float2 L[P], sp[Q];
+        if (iz < a.nz) {
+            c.iz = iz;
+            xf.kload_row(L, krow(a, c, 0), a, t);
+            ss_load<T, Q>(sp, a, c);
+        }
+        for (; iz < a.nz; ++iz) {
+            const float z = a.oz + a.dz * (float)iz;
+            if (!(z >= a.sz && z >= a.gz)) {  // a depth axis that turns back (dz < 0)
+                c.iz = iz;
+                if (z >= a.sz) adj_step<N, P, MODE, WAVE, HALF, X>(us, smem, pp, a, xf, c, true, true);
+                if (z >= a.gz) adj_step<N, P, MODE, WAVE, HALF, X>(ur, smem, pp, a, xf, c, true, false);
+                image(iz, z >= a.gz);
+                c.iz = min(iz + 1, a.nz - 1);
+                xf.kload_row(L, krow(a, c, 0), a, t);
+                ss_load<T, Q>(sp, a, c);
+                continue;
+            }
+            c.iz = min(iz + 1, a.nz - 1);
+            fft2<N, P, -1, HALF>(us, ur, bu, bv, held, t, sync);
 #pragma unroll
-        for (int q = 0; q < P; ++q)
-            buf_store1_nt(pr, (uint32_t)(t + q * T) * 4u, dr ? factor * (ur[q].x * us[q].x + ur[q].y * us[q].y) : 0.f);
+            for (int q = 0; q < P; ++q) {
+                us[q] = cmulc(us[q], L[q]);
+                ur[q] = cmul(ur[q], L[q]);
+            }
+            xf.kload_row(L, krow(a, c, 0), a, t);
+            fft2<N, P, +1, false>(us, ur, bu, bv, held, t, sync);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                us[q] = cmulc(us[q], sp[q]);
+                ur[q] = cmul(ur[q], sp[q]);
+            }
+            zero_tail<P, Q>(us);
+            zero_tail<P, Q>(ur);
+            ss_load<T, Q>(sp, a, c);
+            image(iz, true);
+        }
     }
 }
 
@@ -660,12 +778,33 @@ __device__ __forceinline__ void adj_body_pair(const March2DArgs& a)
 // gives their new e: 2 + nref + 1 transforms per depth instead of 2 (1 + nref).  The image is
 // factor Re(r conj s) = factor (Re z Im z - Re e Im e) / a.
 
+// Sum over the 64 lanes of a wave, in every lane: four steps inside the rows of 16 lanes by DPP and
+// two across them by the row swaps (vector-ALU instructions: a butterfly of LDS permutes waits for
+// the LDS six times in turn).
+__device__ __forceinline__ float wave_sum(float v)
+{
+    auto dpp = [](float x, auto ctrl) {
+        return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), decltype(ctrl)::value,
+                                                                     0xf, 0xf, true));
+    };
+    v += dpp(v, std::integral_constant<int, 0xb1>{});   // quad_perm 1 0 3 2
+    v += dpp(v, std::integral_constant<int, 0x4e>{});   // quad_perm 2 3 0 1
+    v += dpp(v, std::integral_constant<int, 0x141>{});  // half-row mirror
+    v += dpp(v, std::integral_constant<int, 0x140>{});  // row mirror
+    auto add = [](unsigned a, unsigned b) { return __builtin_bit_cast(float, a) + __builtin_bit_cast(float, b); };
+    const unsigned a = __builtin_bit_cast(unsigned, v);
+    const auto r = __builtin_amdgcn_permlane16_swap(a, a, false, false);
+    v = add(r[0], r[1]);
+    const unsigned b = __builtin_bit_cast(unsigned, v);
+    const auto h = __builtin_amdgcn_permlane32_swap(b, b, false, false);
+    return add(h[0], h[1]);
+}
+
 // Sum over the T threads of a subgroup in a fixed order (red: T/64 floats of LDS scratch).
 template <int T>
 __device__ __forceinline__ float subgroup_sum(float v, float* red)
 {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    v = wave_sum(v);
     if constexpr (T == 64) {
         return v;
     } else {
@@ -679,30 +818,24 @@ __device__ __forceinline__ float subgroup_sum(float v, float* red)
     }
 }
 
-
-template <int T>
-__device__ __forceinline__ void subgroup_sync()
-{
-    if constexpr (T == 64) {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    } else {
-        __syncthreads();
-    }
-}
-
 // HALF: nmx <= N / 2, so the points q >= P / 2 (x >= N / 2) are zero in the state and never selected:
 // those constants let the first forward pass and the last inverse pass drop their work.
 // X: the transform policy (XPow2: nkx = N; XMixed: a mixed-radix nkx <= N, whose twiddle table
 // holds nkx entries and whose spectra are zero at k >= nkx).
-template <int N, int P, bool WAVE, bool HALF, class X = XPow2<N, P, true>>
+//
+// What bounds it (nkx 2048, two waves per workgroup, two waves per SIMD): vector-ALU issue and the
+// latencies that two waves cannot hide, so nothing that can be known early is waited for: the seeds
+// of the transforms stay in registers for the whole march, a kz row is read while the transform
+// before it runs, the selection bytes and the direct sums' twiddles at the start of the depth, and
+// the wave sums take no LDS.
+template <int N, int P, bool WAVE, bool HALF, class X = XPow2<N, P, WAVE, kSeedHeld>>
 __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
 {
     constexpr int T = N / P;
+    constexpr int Q = HALF ? P / 2 : P;  // live slots
     constexpr int K = kUncutSparse;
     constexpr int NW = T / 64;  // waves of the subgroup
-    constexpr bool POW2 = std::is_same<X, XPow2<N, P, true>>::value;
+    constexpr bool POW2 = std::is_same<X, XPow2<N, P, WAVE, kSeedHeld>>::value;
     // Bluestein lengths: the table tw is of the array length, not of nkx, so no direct sums (the
     // uncut points' e and output always come from transforms)
     constexpr bool BLUE = std::is_same<X, XBlue<N, P>>::value;
@@ -723,10 +856,11 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
     c.fc = __builtin_amdgcn_readfirstlane(active ? fc : 0);
     const float factor = iw == 0 ? 1.f : 2.f;
     int pp = 0;
+    const X xf(a, t);
     const int igx = a.igx[shot];
     const float2 ss = active ? a.spec_s[fl] : make_float2(0.f, 0.f);
-    // scratch after the transform buffers: reduction slots, e at the previous depth's uncut
-    // points, per-wave partial sums of the new e at this depth's uncut points
+    // scratch after the transform buffers: reduction slots, e at the previous depth's second and
+    // later uncut points, per-wave partial sums of the direct sums
     float2* scr = smem + (WAVE ? 1 : 2) * LdsLen<N>::value;
     float* red = reinterpret_cast<float*>(scr);
     float2* scr_e = scr + 4;
@@ -763,42 +897,55 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
         e[q] = make_float2(us.y, -alpha * e[q].y);
         if (HALF && q >= P / 2) z[q] = e[q] = make_float2(0.f, 0.f);
     }
-    // e before the step: dense (the initial imaginary parts), sparse (nonzero only at the
-    // listed uncut points of the previous depth: prev_cnt <= K) or zero
+    // e before the step: dense in e (the initial imaginary parts; more than K uncut points), or
+    // nonzero only at the prev_cnt <= K uncut points of the previous depth: its value at the first
+    // of them (ev, known to every thread) with the twiddles of that point (w0 = w^(t x), st =
+    // w^(T x), w = exp(-2 pi i / nkx)), the others in scr_e
     int prev_cnt = -1;  // -1: dense
     const int* prev_row = a.cref;
+    float2 ev = make_float2(0.f, 0.f), w0 = ev, st = ev;
     for (int iz = 0; iz < a.nz; ++iz) {
         c.iz = iz;
         const int* crow = a.cref + (size_t)iz * kCrefStride;
         const int cr = crow[0], cnt = crow[1];
+        const bool sparse = !BLUE && cnt > 0 && cnt <= K;
+        // Few uncut points, and no cut point selecting their vref cr: their output under cr, like
+        // their new e, comes from direct sums instead of an inverse transform of cr (HALF kernels:
+        // the others have no registers left for the second set of sums).
+        const bool direct_cr = HALF && sparse && crow[2] != 0;
+        uint32_t todo = a.used[iz] & ((1u << a.nref) - 1u);
+        if (direct_cr) todo &= ~(1u << cr);
+        // the rows of the depth in turn: those of todo, then cr's for the uncut points; each is
+        // read while the transform before its use runs
+        float2 Lr[P];
+        auto next_row = [&](uint32_t left) {
+            if (left || cnt > 0) xf.kload_row(Lr, krow(a, c, left ? __builtin_ctz(left) : cr), a, t);
+        };
+        next_row(todo);
+        uint32_t s1[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) s1[q] = a.sel[(size_t)iz * N + t + q * T];
         // HALF: slots q >= P/2 of z and e are zero (x >= N/2 >= nmx is never selected)
-        X::template fft<-1, WAVE, HALF>(z, smem, a, t, pp);
+        xf.template fft<-1, WAVE, HALF>(z, smem, a, t, pp);
         if (prev_cnt < 0 || prev_cnt > (BLUE ? 0 : K)) {
-            X::template fft<-1, WAVE, HALF>(e, smem, a, t, pp);
+            xf.template fft<-1, WAVE, HALF>(e, smem, a, t, pp);
         } else if (prev_cnt > 0) {
-            // E(k) = sum_j e(x_j) w^(k x_j), w = exp(-2 pi i / N): the owners publish e(x_j)
+            // E(k) = sum_j e(x_j) w^(k x_j), by recurrence over the thread's points k = t + q T
+            float2 p = cmul(ev, w0);
 #pragma unroll
-            for (int j = 0; j < K; ++j) {
-                if (j >= prev_cnt) break;
-                const int xj = prev_row[3 + j];
-#pragma unroll
-                for (int q = 0; q < P; ++q)
-                    if (t + q * T == xj) scr_e[j] = e[q];
+            for (int q = 0; q < P; ++q) {
+                e[q] = p;
+                p = cmul(p, st);
             }
-            subgroup_sync<T>();
-#pragma unroll
-            for (int q = 0; q < P; ++q) e[q] = make_float2(0.f, 0.f);
-#pragma unroll
-            for (int j = 0; j < K; ++j) {
-                if (j >= prev_cnt) break;
+#pragma unroll 1
+            for (int j = 1; j < prev_cnt; ++j) {
                 const int xj = prev_row[3 + j];
-                const float2 ev = scr_e[j];
-                float2 w = twid(t * xj);
-                const float2 st = twid(T * xj);
+                const float2 sj = twid(T * xj);
+                p = cmul(scr_e[j], twid(t * xj));
 #pragma unroll
                 for (int q = 0; q < P; ++q) {
-                    e[q] = cadd(e[q], cmul(ev, w));
-                    w = cmul(w, st);
+                    e[q] = cadd(e[q], p);
+                    p = cmul(p, sj);
                 }
             }
             if constexpr (!POW2) {  // the spectrum of a length nkx < N ends at nkx
@@ -806,148 +953,143 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
                 for (int q = 0; q < P; ++q)
                     if (t + q * T >= a.nkx) e[q] = make_float2(0.f, 0.f);
             }
-        }  // prev_cnt == 0: e == 0, E == 0
-        // selection bytes packed four to a register: (sel(q) = s1w[q / 4] >> 8 (q % 4)) & 0xff
-        uint32_t s1w[(P + 3) / 4];
-        float2 out[P];
+        } else {
 #pragma unroll
-        for (int q = 0; q < (P + 3) / 4; ++q) s1w[q] = 0u;
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            s1w[q >> 2] |= (uint32_t)a.sel[(size_t)iz * N + t + q * T] << (8 * (q & 3));
-            out[q] = make_float2(0.f, 0.f);
+            for (int q = 0; q < P; ++q) e[q] = make_float2(0.f, 0.f);
         }
-        auto s1 = [&](int q) { return (s1w[q >> 2] >> (8 * (q & 3))) & 0xffu; };
-        const uint32_t used = a.used[iz];
-        // Few uncut points, and no cut point selecting their vref cr: their output under cr, like
-        // their new e, comes from direct sums instead of an inverse transform of cr (HALF kernels:
-        // the others have no registers left for the second set of sums).
-        const bool direct_cr = !BLUE && HALF && cnt > 0 && cnt <= K && crow[2] != 0;
-        for (int ir = 0; ir < a.nref; ++ir) {
-            if (!((used >> ir) & 1u) || (direct_cr && ir == cr)) continue;
-            const float2* row = krow(a, c, ir);
+        if (sparse) {  // for this depth's sums and the next depth's E
+            w0 = twid(t * crow[3]);
+            st = twid(T * crow[3]);
+        }
+        float2 out[Q];
+#pragma unroll
+        for (int q = 0; q < Q; ++q) out[q] = make_float2(0.f, 0.f);
+        while (todo) {
+            const uint32_t ir = (uint32_t)__builtin_ctz(todo);
+            todo &= todo - 1u;
             float2 w[P];
-            X::kload_row(w, row, a, c.t);
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const float2 L = w[q];
+                const float2 L = Lr[q];
                 w[q] = make_float2(z[q].x * L.x + e[q].x * L.y, z[q].y * L.x + e[q].y * L.y);
             }
-            X::template fft<+1, WAVE>(w, smem, a, t, pp);
+            next_row(todo);
+            xf.template fft<+1, WAVE>(w, smem, a, t, pp);
 #pragma unroll
-            for (int q = 0; q < (HALF ? P / 2 : P); ++q)
-                if ((int)(s1(q) & 0x7fu) == ir) out[q] = w[q];
+            for (int q = 0; q < Q; ++q)
+                if ((s1[q] & 0x7fu) == ir) out[q] = w[q];
         }
-        if (cnt > 0) {
+        float2 en[Q];  // the new e
+#pragma unroll
+        for (int q = 0; q < Q; ++q) en[q] = make_float2(0.f, 0.f);
+        if (cnt > 0 && !sparse) {
             // imaginary parts at the uncut points of this depth (all select vref cr):
             // e_new = IFFT(Re L E - Im L Z), the conjugate of IFFT(V) by L(-k) = L(k)
-            const float2* row = krow(a, c, cr);
-            float2 lv[P];
-            X::kload_row(lv, row, a, c.t);
-            if (BLUE || cnt > K) {
 #pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    const float2 L = lv[q];
-                    e[q] = make_float2(L.x * e[q].x - L.y * z[q].x, L.x * e[q].y - L.y * z[q].y);
+            for (int q = 0; q < P; ++q) {
+                const float2 L = Lr[q];
+                e[q] = make_float2(L.x * e[q].x - L.y * z[q].x, L.x * e[q].y - L.y * z[q].y);
+            }
+            xf.template fft<+1, WAVE>(e, smem, a, t, pp);
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                const int x = t + q * T;
+                if (x < a.nmx && !(s1[q] >> 7)) en[q] = e[q];
+            }
+        } else if (sparse) {
+            // e_new(x_j) = sum_k U(k) conj(w^(k x_j)) with U = Re L E - Im L Z at the few uncut points
+            // and, when direct_cr, out(x_j) = sum_k W(k) conj(w^(k x_j)) with W = Re L Z + Im L E:
+            // per thread by Horner's rule over its points k = t + q T, then over the subgroup in
+            // a fixed order.  U into e and W into z, in place (the spectra end here).
+#pragma unroll
+            for (int q = 0; q < P; ++q) {
+                const float2 L = Lr[q];
+                const float2 u = make_float2(L.x * e[q].x - L.y * z[q].x, L.x * e[q].y - L.y * z[q].y);
+                if (HALF) z[q] = make_float2(z[q].x * L.x + e[q].x * L.y, z[q].y * L.x + e[q].y * L.y);
+                e[q] = u;
+            }
+            auto sums = [&](float2 w, float2 s, int j, float2& su, float2& sw) {
+                su = e[P - 1];
+                sw = HALF ? z[P - 1] : su;
+#pragma unroll
+                for (int q = P - 2; q >= 0; --q) {
+                    su = make_float2(fmaf(su.x, s.x, fmaf(su.y, s.y, e[q].x)), fmaf(su.y, s.x, fmaf(-su.x, s.y, e[q].y)));
+                    if (HALF)
+                        sw = make_float2(fmaf(sw.x, s.x, fmaf(sw.y, s.y, z[q].x)), fmaf(sw.y, s.x, fmaf(-sw.x, s.y, z[q].y)));
                 }
-                X::template fft<+1, WAVE>(e, smem, a, t, pp);
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    const int x = t + q * T;
-                    if ((HALF && q >= P / 2) || !(x < a.nmx && !(s1(q) >> 7))) e[q] = make_float2(0.f, 0.f);
+                su = cmulc(su, w);
+                su = make_float2(wave_sum(su.x), wave_sum(su.y));
+                if (HALF) {
+                    sw = cmulc(sw, w);
+                    sw = make_float2(wave_sum(sw.x), wave_sum(sw.y));
                 }
-            } else {
-                // e_new(x_j) = sum_k U(k) conj(w^(k x_j)) at the few uncut points and, when direct_cr,
-                // out(x_j) = sum_k W(k) conj(w^(k x_j)) with W = Re L Z + Im L E: partial sums per
-                // thread, then over the subgroup in a fixed order
-                // U into e and W into lv, in place (the spectra z are not needed after them)
-#pragma unroll
-                for (int q = 0; q < P; ++q) {
-                    const float2 L = lv[q];
-                    const float2 u = make_float2(L.x * e[q].x - L.y * z[q].x, L.x * e[q].y - L.y * z[q].y);
-                    lv[q] = make_float2(z[q].x * L.x + e[q].x * L.y, z[q].y * L.x + e[q].y * L.y);
-                    e[q] = u;
-                }
-                float2 acc[K], accw[K];
-#pragma unroll
-                for (int j = 0; j < K; ++j) {
-                    acc[j] = accw[j] = make_float2(0.f, 0.f);
-                    if (j >= cnt) continue;
-                    const int xj = crow[3 + j];
-                    float2 w = twid(t * xj);
-                    const float2 st = twid(T * xj);
-#pragma unroll
-                    for (int q = 0; q < P; ++q) {
-                        acc[j] = cadd(acc[j], cmulc(e[q], w));
-                        if (direct_cr) accw[j] = cadd(accw[j], cmulc(lv[q], w));
-                        w = cmul(w, st);
+                if constexpr (NW > 1)
+                    if ((t & 63) == 0) {
+                        scr_v[(t >> 6) * K + j] = su;
+                        scr_v[(NW + (t >> 6)) * K + j] = sw;
                     }
+            };
+            float2 wn, wc;
+            sums(w0, st, 0, wn, wc);
+            // the second and later points: rare (equal maxima of the depth's velocity)
+#pragma unroll 1
+            for (int j = 1; j < cnt; ++j) {
+                const int xj = crow[3 + j];
+                float2 su, sw;
+                sums(twid(t * xj), twid(T * xj), j, su, sw);
+                if (NW == 1 && t == 0) scr_v[j] = su, scr_v[K + j] = sw;
+            }
+            subgroup_sync<T>();
+            auto total = [&](int j, float2& su, float2& sw) {
+                su = scr_v[j];
+                sw = scr_v[NW * K + j];
 #pragma unroll
-                    for (int o = 32; o > 0; o >>= 1) {
-                        acc[j].x += __shfl_xor(acc[j].x, o, 64);
-                        acc[j].y += __shfl_xor(acc[j].y, o, 64);
-                        if (direct_cr) {
-                            accw[j].x += __shfl_xor(accw[j].x, o, 64);
-                            accw[j].y += __shfl_xor(accw[j].y, o, 64);
-                        }
+                for (int wv = 1; wv < NW; ++wv) {
+                    su = cadd(su, scr_v[wv * K + j]);
+                    sw = cadd(sw, scr_v[(NW + wv) * K + j]);
+                }
+            };
+            auto place = [&](int xj, float2 su, float2 sw) {
+                const int tj = xj & (T - 1), qj = xj / T;  // the owner's thread and slot
+#pragma unroll
+                for (int q = 0; q < Q; ++q)
+                    if (q == qj && t == tj) {
+                        en[q] = su;
+                        if (direct_cr) out[q] = sw;
                     }
-                    if constexpr (NW > 1)
-                        if ((t & 63) == 0) {
-                            scr_v[(t >> 6) * K + j] = acc[j];
-                            scr_v[(NW + (t >> 6)) * K + j] = accw[j];
-                        }
-                }
-                if constexpr (NW > 1) {
-                    subgroup_sync<T>();
-#pragma unroll
-                    for (int j = 0; j < K; ++j) {
-                        if (j >= cnt) break;
-                        acc[j] = scr_v[j];
-                        accw[j] = scr_v[NW * K + j];
-#pragma unroll
-                        for (int wv = 1; wv < NW; ++wv) {
-                            acc[j] = cadd(acc[j], scr_v[wv * K + j]);
-                            accw[j] = cadd(accw[j], scr_v[(NW + wv) * K + j]);
-                        }
-                    }
-                }
-#pragma unroll
-                for (int q = 0; q < P; ++q) e[q] = make_float2(0.f, 0.f);
-#pragma unroll
-                for (int j = 0; j < K; ++j) {
-                    if (j >= cnt) break;
-                    const int xj = crow[3 + j];
-#pragma unroll
-                    for (int q = 0; q < (HALF ? P / 2 : P); ++q)
-                        if (t + q * T == xj) {
-                            e[q] = acc[j];
-                            if (direct_cr) out[q] = accw[j];
-                        }
-                }
+            };
+            if constexpr (NW > 1) total(0, wn, wc);
+            ev = wn;
+            place(crow[3], wn, wc);
+#pragma unroll 1
+            for (int j = 1; j < cnt; ++j) {
+                float2 su, sw;
+                total(j, su, sw);
+                place(crow[3 + j], su, sw);
+                if (t == 0) scr_e[j] = su;
             }
         }
         prev_cnt = cnt;
         prev_row = crow;
-        // imaging condition (wem.c:243-247): factor Re(ur conj(us)).  Without uncut points e is
-        // zeroed, so the arithmetic above needs no branch.
+        // imaging condition (wem.c:243-247): factor Re(ur conj(us))
         const auto pr = buf_rsrc(part + (size_t)iz * a.nmx, (uint32_t)a.nmx * 4u);
-        float n2s = 0.f, n2r = 0.f;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            z[q] = out[q];
-            if (cnt == 0 || (HALF && q >= P / 2)) e[q] = make_float2(0.f, 0.f);
-            if (HALF && q >= P / 2) {
-                z[q] = make_float2(0.f, 0.f);
-                continue;  // x >= nmx: nothing to image
+            if (q >= Q) {  // x >= nmx: nothing to image
+                z[q] = e[q] = make_float2(0.f, 0.f);
+                continue;
             }
+            z[q] = out[q];
+            e[q] = en[q];
             buf_store1_nt(pr, (uint32_t)(t + q * T) * 4u, factor * (z[q].x * z[q].y - e[q].x * e[q].y) * inv_alpha);
         }
         // keep the two packed wavefields of comparable size (the rounding of each transform is
         // relative to their sum): every 8 depths, rescale the receiver part when the ratio of
         // their energies leaves [1/4, 4]
         if ((iz & 7) != 7) continue;
+        float n2s = 0.f, n2r = 0.f;
 #pragma unroll
-        for (int q = 0; q < (HALF ? P / 2 : P); ++q) {
+        for (int q = 0; q < Q; ++q) {
             n2s += z[q].x * z[q].x + e[q].x * e[q].x;
             n2r += z[q].y * z[q].y + e[q].y * e[q].y;
         }
@@ -960,6 +1102,9 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
                 z[q].y *= beta;
                 e[q].y *= beta;
             }
+            ev.y *= beta;
+            if (t == 0)
+                for (int j = 1; j < cnt && j < K; ++j) scr_e[j].y *= beta;
             alpha *= beta;
             inv_alpha = 1.f / alpha;
         }
@@ -996,8 +1141,8 @@ __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void
 template <int N, int MODE, int P>
 __global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_adj(March2DArgs a) { adj_body<N, P, MODE, false>(a); }
 
-template <int N, int MODE, int P>
-__global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_fwd(March2DArgs a) { fwd_body<N, P, MODE, false>(a); }
+template <int N, int MODE, int P, bool HALF>
+__global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_fwd(March2DArgs a) { fwd_body<N, P, MODE, false, HALF>(a); }
 
 template <int N, int MODE>
 __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_w(March2DArgs a)
@@ -1005,24 +1150,24 @@ __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2)))
     adj_body<N, N / 64, MODE, true>(a);
 }
 
-template <int N, int MODE>
+template <int N, int MODE, bool HALF>
 __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_w(March2DArgs a)
 {
-    fwd_body<N, N / 64, MODE, true>(a);
+    fwd_body<N, N / 64, MODE, true, HALF>(a);
 }
 
 // PAIR: 16 points per thread from nkx = 1024 (nkx/16 threads, radix-16 passes), one wave with
 // nkx/64 points per lane below it.
-template <int N, int MODE, int P>
+template <int N, int MODE, int P, bool HALF>
 __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_pair(March2DArgs a)
 {
-    adj_body_pair<N, P, MODE, false>(a);
+    adj_body_pair<N, P, MODE, false, HALF, XPow2<N, P, false, MODE == kModeSSF ? kSeedHeld : kSeedAhead>>(a);
 }
 
-template <int N, int MODE>
+template <int N, int MODE, bool HALF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_pair_w(March2DArgs a)
 {
-    adj_body_pair<N, N / 64, MODE, true>(a);
+    adj_body_pair<N, N / 64, MODE, true, HALF, XPow2<N, N / 64, true, MODE == kModeSSF ? kSeedHeld : kSeedAhead>>(a);
 }
 
 // Transform lengths that are not powers of two: Bluestein through the array length M (one
@@ -1032,25 +1177,25 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ma
 template <int M, int MODE, int P>
 __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_blue(March2DArgs a)
 {
-    adj_body_pair<M, P, MODE, false, XBlue<M, P>>(a);
+    adj_body_pair<M, P, MODE, false, true, XBlue<M, P>>(a);
 }
 
 template <int M, int MODE, int P>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_blue(March2DArgs a)
 {
-    fwd_body<M, P, MODE, false, XBlue<M, P>>(a);
+    fwd_body<M, P, MODE, false, true, XBlue<M, P>>(a);
 }
 
-template <int M, int MODE, int P>
+template <int M, int MODE, int P, bool HALF>
 __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_mixed(March2DArgs a)
 {
-    adj_body_pair<M, P, MODE, false, XMixed<M, P>>(a);
+    adj_body_pair<M, P, MODE, false, HALF, XMixed<M, P>>(a);
 }
 
-template <int M, int MODE, int P>
+template <int M, int MODE, int P, bool HALF>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_mixed(March2DArgs a)
 {
-    fwd_body<M, P, MODE, false, XMixed<M, P>>(a);
+    fwd_body<M, P, MODE, false, HALF, XMixed<M, P>>(a);
 }
 
 // ------------------------------------------------------------------ launches of one array length
@@ -1079,29 +1224,30 @@ static int launch_one(const March2DArgs& a, const March2DShape& sh, int F, int a
             return half ? launch_kernel(march2d_adj_packed<N, 16, true>, a, block, lds_p, st)
                         : launch_kernel(march2d_adj_packed<N, 16, false>, a, block, lds_p, st);
     }
+    const bool half = 2 * a.nmx <= N;
+    auto go = [&](auto with_half, auto without) { return launch_kernel(half ? with_half : without, a, block, lds, st); };
     if (sh.variant == SWEM_VARIANT_PAIR || sh.variant == SWEM_VARIANT_PACKED) {
         if constexpr (N < 1024)
-            return launch_kernel(march2d_adj_pair_w<N, MODE>, a, block, lds, st);
+            return go(march2d_adj_pair_w<N, MODE, true>, march2d_adj_pair_w<N, MODE, false>);
         else
-            return launch_kernel(march2d_adj_pair<N, MODE, 16>, a, block, lds, st);
+            return go(march2d_adj_pair<N, MODE, 16, true>, march2d_adj_pair<N, MODE, 16, false>);
     }
     if (sh.variant == SWEM_VARIANT_PAIR8) {
-        if constexpr (N >= 512)
-            return launch_kernel(march2d_adj_pair<N, MODE, 8>, a, block, lds, st);
+        if constexpr (N >= 512) return go(march2d_adj_pair<N, MODE, 8, true>, march2d_adj_pair<N, MODE, 8, false>);
     }
     if constexpr (N <= 2048) {
         if (sh.variant == SWEM_VARIANT_WAVE)
             return adj ? launch_kernel(march2d_adj_w<N, MODE>, a, block, lds, st)
-                       : launch_kernel(march2d_fwd_w<N, MODE>, a, block, lds, st);
+                       : go(march2d_fwd_w<N, MODE, true>, march2d_fwd_w<N, MODE, false>);
     }
     if constexpr (N >= 1024) {
         if (sh.variant == SWEM_VARIANT_SUBGROUP16)
             return adj ? launch_kernel(march2d_adj<N, MODE, 16>, a, block, lds, st)
-                       : launch_kernel(march2d_fwd<N, MODE, 16>, a, block, lds, st);
+                       : go(march2d_fwd<N, MODE, 16, true>, march2d_fwd<N, MODE, 16, false>);
     }
     constexpr int P = Pts<N>::value;
     return adj ? launch_kernel(march2d_adj<N, MODE, P>, a, block, lds, st)
-               : launch_kernel(march2d_fwd<N, MODE, P>, a, block, lds, st);
+               : go(march2d_fwd<N, MODE, P, true>, march2d_fwd<N, MODE, P, false>);
 }
 
 template <int M, int MODE>
@@ -1120,9 +1266,13 @@ static int launch_blue_mode(const March2DArgs& a, const March2DShape& sh, int F,
             return launch_kernel(march2d_adj_packed_blue<M, P, true>, a, block, lds_p, st);
         }
     }
-    if (sh.mixed)
-        return adj ? launch_kernel(march2d_adj_mixed<M, MODE, P>, a, block, lds, st)
-                   : launch_kernel(march2d_fwd_mixed<M, MODE, P>, a, block, lds, st);
+    if (sh.mixed) {
+        if (2 * a.nmx <= M)
+            return adj ? launch_kernel(march2d_adj_mixed<M, MODE, P, true>, a, block, lds, st)
+                       : launch_kernel(march2d_fwd_mixed<M, MODE, P, true>, a, block, lds, st);
+        return adj ? launch_kernel(march2d_adj_mixed<M, MODE, P, false>, a, block, lds, st)
+                   : launch_kernel(march2d_fwd_mixed<M, MODE, P, false>, a, block, lds, st);
+    }
     return adj ? launch_kernel(march2d_adj_blue<M, MODE, P>, a, block, lds, st)
                : launch_kernel(march2d_fwd_blue<M, MODE, P>, a, block, lds, st);
 }
@@ -1169,10 +1319,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
     c.fc = __builtin_amdgcn_readfirstlane(active ? fc : 0);
     float2* lds = smem + (size_t)s * 2 * L;
     int pp = 0;
-    float tap[P];
-    load_taper<N, P, kModeSSF>(tap, a, t);
+    const X xf(a, t);
     const int igx = a.igx[shot];
-    float2* vol = a.smig + (size_t)(active ? fc : 0) * a.nz * a.nmx;
+    float2* vol = a.smig + (size_t)c.fc * a.nz * a.nmx;
     float2 u[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
@@ -1183,7 +1332,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void a
         c.iz = iz;
         const float z = a.oz + a.dz * (float)iz;
         const bool ds = z >= a.sz;
-        if (ds) ssf_fwd_step<N, P, false, X>(u, lds, pp, a, c, tap);
+        if (ds) {
+            float2 sp[P];
+            ss_load<T, P>(sp, a, c);
+            ssf_fwd_step<N, P, false, false, X>(u, lds, pp, a, xf, c, sp);
+        }
         if (active) {
             const auto sr = buf_rsrc(vol + (size_t)iz * a.nmx, (uint32_t)a.nmx * 8u);
 #pragma unroll
@@ -1209,6 +1362,7 @@ __global__ __launch_bounds__(N / P) void angle_cols(March2DArgs az, AngleArgs b)
     const size_t base = (size_t)(l / b.inner) * b.outer + (size_t)(l % b.inner) * b.inner_stride;
     const int t = threadIdx.x;
     int pp = 0;
+    const X xf(az, t);
     const float2* col = b.vol + base;
     float2 v[P];
 #pragma unroll
@@ -1217,13 +1371,13 @@ __global__ __launch_bounds__(N / P) void angle_cols(March2DArgs az, AngleArgs b)
         v[q] = iz < b.nz ? col[(size_t)iz * b.elem] : make_float2(0.f, 0.f);
     }
     __builtin_amdgcn_sched_barrier(0);
-    X::template fft<-1, false>(v, smem, az, t, pp);
+    xf.template fft<-1, false>(v, smem, az, t, pp);
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         const int k = t + q * T;
         v[q] = times_i(v[q], k < b.nz ? kbin(k, b.nz, b.dkz) : 0.f);
     }
-    X::template fft<+1, false>(v, smem, az, t, pp);
+    xf.template fft<+1, false>(v, smem, az, t, pp);
     float* out = b.dzmag + base;
     const float inv = 1.f / (float)b.nz;
 #pragma unroll
@@ -1245,6 +1399,7 @@ __global__ __launch_bounds__(N / P) void angle_rows(March2DArgs ax, AngleArgs b)
     const size_t base = (size_t)(l / b.inner) * b.outer + (size_t)(l % b.inner) * b.inner_stride;
     const int t = threadIdx.x;
     int pp = 0;
+    const X xf(ax, t);
     const int n = ax.nkx;
     const float deg = (float)(180.0 / 3.141592653589793);
     const float inv = 1.f / (float)n;
@@ -1272,23 +1427,23 @@ __global__ __launch_bounds__(N / P) void angle_rows(March2DArgs ax, AngleArgs b)
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int q = 0; q < P; ++q) mu[q] = sqrtf(A[q].x * A[q].x + A[q].y * A[q].y);
-        X::template fft<-1, false>(A, smem, ax, t, pp);
+        xf.template fft<-1, false>(A, smem, ax, t, pp);
         float mx[P], ml[P];
         float2 B[P];
 #pragma unroll
         for (int q = 0; q < P; ++q) B[q] = times_i(A[q], kx[q]);
-        X::template fft<+1, false>(B, smem, ax, t, pp);
+        xf.template fft<+1, false>(B, smem, ax, t, pp);
 #pragma unroll
         for (int q = 0; q < P; ++q) mx[q] = sqrtf(B[q].x * B[q].x + B[q].y * B[q].y) * inv;
         // negative wavenumbers only (k > n/2), then positive only (k <= n/2)
 #pragma unroll
         for (int q = 0; q < P; ++q) B[q] = times_i(A[q], (t + q * T) <= n / 2 ? 0.f : kx[q]);
-        X::template fft<+1, false>(B, smem, ax, t, pp);
+        xf.template fft<+1, false>(B, smem, ax, t, pp);
 #pragma unroll
         for (int q = 0; q < P; ++q) ml[q] = sqrtf(B[q].x * B[q].x + B[q].y * B[q].y);
 #pragma unroll
         for (int q = 0; q < P; ++q) B[q] = times_i(A[q], (t + q * T) <= n / 2 ? kx[q] : 0.f);
-        X::template fft<+1, false>(B, smem, ax, t, pp);
+        xf.template fft<+1, false>(B, smem, ax, t, pp);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
             const float mr = sqrtf(B[q].x * B[q].x + B[q].y * B[q].y);
@@ -1348,7 +1503,7 @@ int launch_angles_len(int which, int kind, const March2DArgs& ax, const March2DA
 // (i1, i2) -> (o1, o2) through the wavenumber domain; o1, o2 are zero at x >= nmx.
 template <int N, int P, class X>
 __device__ __forceinline__ void esep(const float2 (&i1)[P], const float2 (&i2)[P], float2 (&o1)[P], float2 (&o2)[P],
-                                     float2* lds, int& pp, const March2DArgs& a, const EwemArgs& e, int t, float w,
+                                     float2* lds, int& pp, const March2DArgs& a, const X& xf, const EwemArgs& e, int t, float w,
                                      float vp, float vs, bool sep, bool adj)
 {
     constexpr int T = N / P;
@@ -1358,8 +1513,8 @@ __device__ __forceinline__ void esep(const float2 (&i1)[P], const float2 (&i2)[P
         o1[q] = i1[q];
         o2[q] = i2[q];
     }
-    X::template fft<-1, false>(o1, lds, a, t, pp);
-    X::template fft<-1, false>(o2, lds, a, t, pp);
+    xf.template fft<-1, false>(o1, lds, a, t, pp);
+    xf.template fft<-1, false>(o2, lds, a, t, pp);
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         const int k = t + q * T;
@@ -1370,8 +1525,8 @@ __device__ __forceinline__ void esep(const float2 (&i1)[P], const float2 (&i2)[P
         o1[q] = k < n ? cscale(r1, a.inv_nk) : make_float2(0.f, 0.f);
         o2[q] = k < n ? cscale(r2, a.inv_nk) : make_float2(0.f, 0.f);
     }
-    X::template fft<+1, false>(o1, lds, a, t, pp);
-    X::template fft<+1, false>(o2, lds, a, t, pp);
+    xf.template fft<+1, false>(o1, lds, a, t, pp);
+    xf.template fft<+1, false>(o2, lds, a, t, pp);
 #pragma unroll
     for (int q = 0; q < P; ++q)
         if (t + q * T >= a.nmx) o1[q] = o2[q] = make_float2(0.f, 0.f);
@@ -1396,8 +1551,7 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
     c.t = t;
     c.fc = __builtin_amdgcn_readfirstlane(active ? fc : 0);
     int pp = 0;
-    float tap[P];
-    load_taper<N, P, kModeSSF>(tap, ap, t);
+    const X xf(ap, t);
     const int igx = ap.igx[shot];
     const float factor = iw == 0 ? 1.f : 2.f;
     const size_t sp = (size_t)shot * ap.nmx * e.nf;  // this shot's spectra
@@ -1416,14 +1570,14 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
             c.iz = iz;
             const float z = ap.oz + ap.dz * (float)iz;
             const bool ds = z >= ap.sz, dr = z >= ap.gz;
-            if (ds) ssf_adj_step<N, P, false, true, X>(us, smem, pp, ap, c, true, tap);
+            if (ds) ssf_adj_step<N, P, false, true, false, X>(us, smem, pp, ap, xf, c, true);
             float2 up[P], u2[P];
             if (dr) {
                 const float vp = e.vp0[iz], vs = e.vs0[iz];
-                esep<N, P, X>(rx, rz, up, u2, smem, pp, ap, e, t, w, vp, vs, true, true);
-                ssf_adj_step<N, P, false, true, X>(up, smem, pp, ap, c, false, tap);
-                ssf_adj_step<N, P, false, true, X>(u2, smem, pp, as, c, false, tap);
-                esep<N, P, X>(up, u2, rx, rz, smem, pp, ap, e, t, w, vp, vs, false, true);
+                esep<N, P, X>(rx, rz, up, u2, smem, pp, ap, xf, e, t, w, vp, vs, true, true);
+                ssf_adj_step<N, P, false, true, false, X>(up, smem, pp, ap, xf, c, false);
+                ssf_adj_step<N, P, false, true, false, X>(u2, smem, pp, as, xf, c, false);
+                esep<N, P, X>(up, u2, rx, rz, smem, pp, ap, xf, e, t, w, vp, vs, false, true);
             }
             if (active) {
                 const auto rp = buf_rsrc(e.ppart + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 4u);
@@ -1442,7 +1596,7 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
             c.iz = iz;
             const float z = ap.oz + ap.dz * (float)iz;
             const bool ds = z >= ap.sz;
-            if (ds) ssf_adj_step<N, P, false, true, X>(us, smem, pp, ap, c, true, tap);
+            if (ds) ssf_adj_step<N, P, false, true, false, X>(us, smem, pp, ap, xf, c, true);
             if (active) {
                 const auto sr = buf_rsrc(e.smig + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 8u);
 #pragma unroll
@@ -1456,7 +1610,7 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
             if (!(z >= ap.gz)) continue;
             const float vp = e.vp0[iz], vs = e.vs0[iz];
             float2 up[P], u2[P];
-            esep<N, P, X>(rx, rz, up, u2, smem, pp, ap, e, t, w, vp, vs, true, false);
+            esep<N, P, X>(rx, rz, up, u2, smem, pp, ap, xf, e, t, w, vp, vs, true, false);
             if (active) {
                 const auto sr = buf_rsrc(e.smig + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 8u);
                 const auto mp = buf_rsrc(e.mppT + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 4u);
@@ -1477,9 +1631,12 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
                     u2[q] = cadd(u2[q], cscale(sv[q], msv[q]));
                 }
             }
-            ssf_fwd_step<N, P, false, X>(up, smem, pp, ap, c, tap);
-            ssf_fwd_step<N, P, false, X>(u2, smem, pp, as, c, tap);
-            esep<N, P, X>(up, u2, rx, rz, smem, pp, ap, e, t, w, vp, vs, false, false);
+            float2 sp[P];
+            ss_load<T, P>(sp, ap, c);
+            ssf_fwd_step<N, P, false, false, X>(up, smem, pp, ap, xf, c, sp);
+            ss_load<T, P>(sp, as, c);
+            ssf_fwd_step<N, P, false, false, X>(u2, smem, pp, as, xf, c, sp);
+            esep<N, P, X>(up, u2, rx, rz, smem, pp, ap, xf, e, t, w, vp, vs, false, false);
         }
         if (active) {
 #pragma unroll

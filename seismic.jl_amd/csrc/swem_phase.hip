@@ -6,7 +6,8 @@
 //           s = w^2 p2[iz][ir] - kx^2, kx = kk dkx, kk = 0..nkx/2 (L is even in kx)
 //           (ssop wem.c:341-344 with p2 = po^2; pspiop wem.c:434-437 with p2 = 1/vref^2;
 //           the two 1/sqrt(nk) of wem.c:344,354 folded in)
-// SS table  S[f][iz][x] = exp(i w pd[x][iz] dz)            (ssop wem.c:326,353)
+// SS table  S[f][iz][x] = taper[x] exp(i w pd[x][iz] dz)   (ssop wem.c:326,353; boundary_condition
+//           wem.c:546-564: both orders of ssop multiply by the two together)
 // Tables hold the +dz orientation; a -dz step uses their complex conjugate.
 // KZ64: every quantity in double (s, sqrt, sincos, exp), rounded to float at the end.
 // FP32: the reference's float expressions (s = (w*w)*p2 - kx*kx in float, sqrtf, sincosf).
@@ -81,12 +82,12 @@ __global__ __launch_bounds__(256) void build_ss_table(PhaseTableArgs a)
             if (a.prec == SWEM_PREC_KZ64) {
                 double sn, cs;
                 sincos((double)iw * a.dw * a.pd[(size_t)iz * a.nmx + x] * a.dz, &sn, &cs);
-                S = make_float2((float)cs, (float)sn);
+                S = make_float2((float)(cs * a.taper[x]), (float)(sn * a.taper[x]));
             } else {
 #pragma clang fp contract(off)
                 float sn, cs;
                 sincosf((float)iw * a.dwf * a.pdf[(size_t)iz * a.nmx + x] * (float)a.dz, &sn, &cs);
-                S = make_float2(cs, sn);
+                S = make_float2(cs * a.taper[x], sn * a.taper[x]);
             }
             row[x] = S;
         }
