@@ -350,14 +350,14 @@ __device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const float2* _
     fft_pass<N, P, SIGN, 1, SEED, HIN>(v, lds, tw, held, t, pp);
 }
 
-// Wave-level variant: one 64-lane wave transforms N = 64 P points held as v[q] = x[t + 64 q].
-// All exchanges stay inside the wave, whose LDS instructions execute in program order, so a
-// read issued after a write observes it and one buffer (LdsLen<N> complex, private to the wave)
+// Wave-level variant: G lanes of a wave (G a power of two, 64 / G lines side by side) transform
+// N = G P points held as v[q] = x[t + G q].  All exchanges stay inside the wave, whose LDS instructions execute in program order, so a
+// read issued after a write observes it and one buffer (LdsLen<N> complex, private to the line)
 // suffices with no s_barrier; wave_barrier only stops the compiler from reordering the LDS
 // accesses across the exchange.
-template <int N, int NS>
+template <int N, int NS, int G = 64>
 struct WPass {
-    static constexpr int P = N / 64;
+    static constexpr int P = N / G;
     static constexpr int REM = N / NS;
     static constexpr int RMAX = P < 16 ? P : 16;
     static constexpr int R = REM >= RMAX ? RMAX : REM;
@@ -368,14 +368,14 @@ struct WPass {
 };
 
 // The twiddle seeds of pass NS of wfft<N> (as in fft).
-template <int N, int NS>
-__device__ __forceinline__ void wfft_seeds(const float2* __restrict__ tw, int t, float2 (&w)[WPass<N, NS>::NTW])
+template <int N, int NS, int G = 64>
+__device__ __forceinline__ void wfft_seeds(const float2* __restrict__ tw, int t, float2 (&w)[WPass<N, NS, G>::NTW])
 {
-    using S = WPass<N, NS>;
+    using S = WPass<N, NS, G>;
     if constexpr (NS > 1) {
 #pragma unroll
         for (int b = 0; b < S::B; ++b) {
-            uint32_t k = (uint32_t)(t + b * 64) & (NS - 1);
+            uint32_t k = (uint32_t)(t + b * G) & (NS - 1);
             asm volatile("" : "+v"(k));  // keep the loads in the transform (see fft)
             pass_seeds<N, NS, S::R>(tw, k, &w[b * S::S]);
         }
@@ -412,19 +412,19 @@ struct WfftSeeds {
 // One pass and the passes after it; w: this pass's seeds (kSeedHeld: and those of the later ones).
 // Otherwise the next pass's seeds are loaded at the start of this one where that costs at most 8
 // complex registers; larger transforms load their seeds in the pass that uses them.
-template <int N, int SIGN, int NS, int SEED, bool HIN>
-__device__ __forceinline__ void wfft_pass(float2 (&v)[N / 64], float2* buf, const float2* __restrict__ tw, int t,
+template <int N, int SIGN, int NS, int SEED, bool HIN, int G>
+__device__ __forceinline__ void wfft_pass(float2 (&v)[N / G], float2* buf, const float2* __restrict__ tw, int t,
                                           const float2* w)
 {
-    using S = WPass<N, NS>;
+    using S = WPass<N, NS, G>;
     constexpr int P = S::P, R = S::R, B = S::B;
-    constexpr int T = 64;
+    constexpr int T = G;
     constexpr int SH = PassPad<NS, R>::value;
     static_assert(P % R == 0, "radix must divide the points per lane");
     constexpr int NSN = S::LAST ? NS : NS * R;
-    constexpr bool PRE = WPass<N, NSN>::NTW <= 8;
-    float2 wn[SEED == kSeedHeld ? 1 : WPass<N, NSN>::NTW];
-    if constexpr (!S::LAST && PRE && SEED != kSeedHeld) wfft_seeds<N, NSN>(tw, t, wn);
+    constexpr bool PRE = WPass<N, NSN, G>::NTW <= 8;
+    float2 wn[SEED == kSeedHeld ? 1 : WPass<N, NSN, G>::NTW];
+    if constexpr (!S::LAST && PRE && SEED != kSeedHeld) wfft_seeds<N, NSN, G>(tw, t, wn);
 #pragma unroll
     for (int b = 0; b < B; ++b) {
         const int j = t + b * T;
@@ -452,18 +452,18 @@ __device__ __forceinline__ void wfft_pass(float2 (&v)[N / 64], float2* buf, cons
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if constexpr (!PRE && SEED != kSeedHeld) wfft_seeds<N, NSN>(tw, t, wn);
-        wfft_pass<N, SIGN, NSN, SEED, false>(v, buf, tw, t, SEED == kSeedHeld ? w + (NS > 1 ? S::NTW : 0) : wn);
+        if constexpr (!PRE && SEED != kSeedHeld) wfft_seeds<N, NSN, G>(tw, t, wn);
+        wfft_pass<N, SIGN, NSN, SEED, false, G>(v, buf, tw, t, SEED == kSeedHeld ? w + (NS > 1 ? S::NTW : 0) : wn);
     }
 }
 
 // SEED: kSeedHeld with the lane's WfftSeeds in `held`, else read in the transform.  HIN: the points
 // N/2 .. N-1 (slots q >= P/2) are zero on input and are not read.
-template <int N, int SIGN, int SEED = kSeedAhead, bool HIN = false>
-__device__ __forceinline__ void wfft(float2 (&v)[N / 64], float2* buf, const float2* __restrict__ tw, int t,
+template <int N, int SIGN, int SEED = kSeedAhead, bool HIN = false, int G = 64>
+__device__ __forceinline__ void wfft(float2 (&v)[N / G], float2* buf, const float2* __restrict__ tw, int t,
                                      const float2* held = nullptr)
 {
-    wfft_pass<N, SIGN, 1, SEED, HIN>(v, buf, tw, t, held);
+    wfft_pass<N, SIGN, 1, SEED, HIN, G>(v, buf, tw, t, held);
 }
 
 // Two wavefields transformed in lockstep, one LDS buffer each: every barrier serves both, and one's

@@ -28,6 +28,20 @@
 
 namespace swem {
 
+// Lanes and points per lane of a line of N array points.  A whole wave from 512 points on.  Below,
+// 64 / G lines share a wave: a 256-point line of 4 points per lane takes four radix-4 passes (three
+// exchanges through LDS), one of 16 per lane two radix-16 passes (one exchange); a mixed-radix pass
+// has n / R butterflies, which leave most of 64 lanes idle on a short line (8 points per lane there:
+// 16 spill).
+constexpr int line_lanes(int n, int kind) { return n >= 512 ? 64 : (kind == kLenPow2 ? n / 16 : n / 8); }
+template <int N, int KIND>
+struct Line {
+    static constexpr int G = line_lanes(N, KIND);
+    static constexpr int P = N / G;
+};
+template <int N, int KIND>
+using LinePoints = float2[Line<N, KIND>::P];
+
 namespace {
 
 constexpr double kTwoPi = 6.283185307179586;
@@ -99,9 +113,10 @@ __device__ __forceinline__ float2 kz_phase(const March3DArgs& a, double w, doubl
 }
 
 // split-step phase exp(i w pd dz) (+dz orientation, wem.c:326,353)
+template <int PREC = -1>  // -1: read from the arguments
 __device__ __forceinline__ float2 ss_phase(const March3DArgs& a, double w, size_t ixy)
 {
-    if (a.prec == SWEM_PREC_KZ64) return cis_rev(reduce_rev(w * a.pd[(size_t)a.iz * a.nm + ixy] * a.dzd));
+    if (PREC < 0 ? a.prec == SWEM_PREC_KZ64 : PREC == SWEM_PREC_KZ64) return cis_rev(reduce_rev(w * a.pd[(size_t)a.iz * a.nm + ixy] * a.dzd));
     {
 #pragma clang fp contract(off)
         float sn, cs;
@@ -129,20 +144,20 @@ __device__ __forceinline__ bool yin(const March3DArgs& a, int i)
     return BY == kLenPow2 || i < a.nky;
 }
 
-// Transform of one line of n points held by a wave as N array points (lane t, slot q: point
-// t + 64 q).  KIND kLenPow2: n = N, the wave FFT.  kLenMixed: n = 2^a 3^b 5^c <= N, the
+// Transform of one line of n points held by G lanes as N array points (lane t, slot q: point
+// t + G q).  KIND kLenPow2: n = N, the wave FFT.  kLenMixed: n = 2^a 3^b 5^c <= N, the
 // mixed-radix transform in the wave's LDS buffer (tw: [n] of n).  kLenBluestein: Bluestein's
 // chirp-z identity on the power-of-two array length N >= 2n - 1, X_k = c_k IFFT_N(FFT_N(c x) B)_k
 // with the chirp c_j = exp(SIGN i pi j^2 / n) and B the spectrum of the wrapped conjugate chirp
 // over N, built in FP64 on the host (c = 0 for j >= n, so points beyond n enter and leave as zero).
 template <int N, int SIGN, int KIND>
-__device__ __forceinline__ void line_fft(float2 (&v)[N / 64], float2* buf, const float2* __restrict__ tw,
+__device__ __forceinline__ void line_fft(LinePoints<N, KIND>& v, float2* buf, const float2* __restrict__ tw,
                                          const float2* __restrict__ chirp, const float2* __restrict__ bch,
                                          const MixedRadix& mr, int n, int t)
 {
-    constexpr int P = N / 64;
+    constexpr int G = Line<N, KIND>::G, P = Line<N, KIND>::P;
     if constexpr (KIND == kLenPow2) {
-        wfft<N, SIGN>(v, buf, tw, t);
+        wfft<N, SIGN, kSeedAhead, false, G>(v, buf, tw, t);
     } else if constexpr (KIND == kLenMixed) {
         int pp = 0;
         mixed_fft<N, P, SIGN, false>(v, buf, buf, tw, mr, t, pp, []() { wave_sync_lds(); });
@@ -151,7 +166,7 @@ __device__ __forceinline__ void line_fft(float2 (&v)[N / 64], float2* buf, const
             float2 c[P];
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int j = t + 64 * q;
+                const int j = t + G * q;
                 const float2 cj = j < n ? chirp[j] : make_float2(0.f, 0.f);  // exp(-i pi j^2 / n)
                 c[q] = SIGN < 0 ? cj : make_float2(cj.x, -cj.y);
             }
@@ -159,27 +174,27 @@ __device__ __forceinline__ void line_fft(float2 (&v)[N / 64], float2* buf, const
             for (int q = 0; q < P; ++q) v[q] = cmul(v[q], c[q]);
         };
         chirp_mul();
-        wfft<N, -1>(v, buf, tw, t);
+        wfft<N, -1, kSeedAhead, false, G>(v, buf, tw, t);
         const float2* B = bch + (SIGN < 0 ? 0 : N);
         float2 bq[P];
 #pragma unroll
-        for (int q = 0; q < P; ++q) bq[q] = B[t + 64 * q];
+        for (int q = 0; q < P; ++q) bq[q] = B[t + G * q];
 #pragma unroll
         for (int q = 0; q < P; ++q) v[q] = cmul(v[q], bq[q]);
         wave_sync_lds();
-        wfft<N, +1>(v, buf, tw, t);
+        wfft<N, +1, kSeedAhead, false, G>(v, buf, tw, t);
         chirp_mul();
     }
 }
 
 template <int N, int SIGN, int BX>
-__device__ __forceinline__ void xfft(float2 (&v)[N / 64], float2* buf, const March3DArgs& a, int t)
+__device__ __forceinline__ void xfft(LinePoints<N, BX>& v, float2* buf, const March3DArgs& a, int t)
 {
     line_fft<N, SIGN, BX>(v, buf, a.twx, a.chx, a.bchx, a.mrx, a.nkx, t);
 }
 
 template <int N, int SIGN, int BY>
-__device__ __forceinline__ void yfft(float2 (&v)[N / 64], float2* buf, const March3DArgs& a, int t)
+__device__ __forceinline__ void yfft(LinePoints<N, BY>& v, float2* buf, const March3DArgs& a, int t)
 {
     line_fft<N, SIGN, BY>(v, buf, a.twy, a.chy, a.bchy, a.mry, a.nky, t);
 }
@@ -192,11 +207,11 @@ __device__ __forceinline__ void yfft(float2 (&v)[N / 64], float2* buf, const Mar
 template <int NY, int BY>
 __global__ __launch_bounds__(256) void march3d_init(March3DArgs a)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     constexpr int L = LdsLen<NY>::value;
-    __shared__ float2 lds[4 * L];
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
-    const size_t row = (size_t)blockIdx.x * 4 + w;
+    __shared__ float2 lds[256 / G * L];
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
+    const size_t row = (size_t)blockIdx.x * (256 / G) + w;
     const size_t nrow = (size_t)a.nitem * 2 * a.nmx;
     if (row >= nrow) return;  // whole waves only: the transform below has no workgroup barrier
     const int x = (int)(row % a.nmx);
@@ -206,7 +221,7 @@ __global__ __launch_bounds__(256) void march3d_init(March3DArgs a)
     float2 v[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int y = t + 64 * q;
+        const int y = t + G * q;
         float2 u = make_float2(0.f, 0.f);
         if (y < a.nmy) {
             const size_t ixy = (size_t)x * a.nmy + y;
@@ -220,7 +235,7 @@ __global__ __launch_bounds__(256) void march3d_init(March3DArgs a)
     yfft<NY, -1, BY>(v, lds + w * L, a, t);
     float2* dst = state(a, item, wf) + (size_t)x * a.nky;
 #pragma unroll
-    for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = v[q];
+    for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = v[q];
 }
 
 // kz phase of the KZ64 path with the column's part hoisted: c0 = w^2 po^2 - ky^2 (FP64, once per
@@ -231,21 +246,53 @@ __device__ __forceinline__ float2 kz_phase64(const March3DArgs& a, double c0, in
     return kz_phase_s64(a, fma(-(double)(kxi * kxi), a.dkx2, c0));
 }
 
-// kz phases of a lane's points ikx = t + 64 q of one ky column on a power-of-two nkx = N (KZ64):
+// kz phases of a lane's points ikx = t + G q of one ky column on a power-of-two nkx = N (KZ64):
 // q <= P/2 directly, the others from their mirror nkx - ikx (the same |kx|, so the same phase bit
-// for bit), which lane 64 - t holds at slot P - 1 - q (lane 0: its own slot P - q).
+// for bit), which lane G - t of the line holds at slot P - 1 - q (lane 0: its own slot P - q).
 template <int N>
-__device__ __forceinline__ void kz_phases64_col(const March3DArgs& a, double c0, int t, float2 (&ph)[N / 64])
+__device__ __forceinline__ void kz_phases64_col(const March3DArgs& a, double c0, int t, LinePoints<N, kLenPow2>& ph)
 {
-    constexpr int P = N / 64;
+    constexpr int G = Line<N, kLenPow2>::G, P = Line<N, kLenPow2>::P;
 #pragma unroll
-    for (int q = 0; q <= P / 2 && q < P; ++q) ph[q] = kz_phase64(a, c0, t + 64 * q);
-    const int src = (64 - t) & 63;
+    for (int q = 0; q <= P / 2 && q < P; ++q) ph[q] = kz_phase64(a, c0, t + G * q);
+    const int src = ((int)threadIdx.x & 63 & ~(G - 1)) | ((G - t) & (G - 1));
 #pragma unroll
     for (int q = P / 2 + 1; q < P; ++q) {
         const float2 m = ph[P - 1 - q];
         const float x = __shfl(m.x, src, 64), y = __shfl(m.y, src, 64);
         ph[q] = t == 0 ? ph[P - q] : make_float2(x, y);
+    }
+}
+
+// Staging of an x-pass workgroup's tile of C columns through LDS: thread (x0, c) = (threadIdx / C,
+// threadIdx mod C) moves the rows x0 + G j of column c, so global accesses are row segments of C
+// complex.  A line of fewer than 64 lanes stages its two wavefields in turn through one buffer per
+// column (ONE): with both in LDS at once it would hold half the waves per compute unit.
+template <int P, int G>
+__device__ __forceinline__ void tile_load(float2 (&st)[P], const float2* src, const March3DArgs& a, int x0, bool in)
+{
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int x = x0 + G * j;
+        st[j] = x < a.nmx && in ? src[(size_t)x * a.nky] : make_float2(0.f, 0.f);
+    }
+}
+template <int P, int G>
+__device__ __forceinline__ void tile_put(const float2 (&st)[P], float2* dst, const March3DArgs& a, int x0)
+{
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int x = x0 + G * j;
+        if (x < a.nmx) dst[lds_pad(x)] = st[j];
+    }
+}
+template <int P, int G>
+__device__ __forceinline__ void tile_store(float2* dst, const float2* src, const March3DArgs& a, int x0, bool in)
+{
+#pragma unroll
+    for (int j = 0; j < P; ++j) {
+        const int x = x0 + G * j;
+        if (x < a.nmx && in) dst[(size_t)x * a.nky] = src[lds_pad(x)];
     }
 }
 
@@ -255,10 +302,10 @@ __device__ __forceinline__ void kz_phases64_col(const March3DArgs& a, double c0,
 // of C complex.  conj_src / conj_rec: use conj(L) (-dz).  Workgroups are renumbered so that each
 // XCD (consecutive workgroup ids go round robin over the 8 XCDs) takes a contiguous run of tiles:
 // neighbouring tiles share 128-byte lines, which then meet in one L2.
-template <int NX, int NWF, int C, int BX>
-__global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 1024 ? 2 : 4))) void march3d_cols(March3DArgs a)
+template <int NX, int NWF, int C, int BX, int PREC>
+__global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 1024 ? 2 : (NWF == 2 && line_lanes(NX, BX) * 16 == NX ? 3 : 4)))) void march3d_cols(March3DArgs a)
 {
-    constexpr int P = NX / 64;
+    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;
     constexpr int L = LdsLen<NX>::value;
     extern __shared__ float2 smem[];
     const int tiles = (a.nky + C - 1) / C;  // the last tile is partial when C does not divide nky
@@ -268,41 +315,44 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
     if (b < full) b = (b & 7) * (full >> 3) + (b >> 3);
     const int item = b / tiles;
     const int ky0 = (b - item * tiles) * C;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int wf1 = (a.wmask & 1) ? 0 : 1;  // the wavefield of an NWF = 1 launch
     auto wf_of = [&](int k) { return NWF == 2 ? k : wf1; };
-    // stage: buffer (c * NWF + k) holds column ky0 + c of the k-th stepped wavefield.  The loads of
-    // one wavefield are all issued before its LDS writes (rows x0 + 64 j, j < P cover x < nmx).
+    // buffer (c * NB + k) holds column ky0 + c of the k-th stepped wavefield (ONE: of each in turn);
+    // the loads of both wavefields are all issued before the first LDS write
+    constexpr bool ONE = NWF == 2 && G < 64;
+    constexpr int NB = ONE ? 1 : NWF;
     const int c = threadIdx.x % C, x0 = threadIdx.x / C;
     const bool kin = ky0 + c < a.nky;
-#pragma unroll
-    for (int k = 0; k < NWF; ++k) {
-        const float2* src = state(a, item, wf_of(k)) + ky0 + c;
-        float2* dst = smem + (c * NWF + k) * L;
-        float2 st[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int x = x0 + 64 * j;
-            st[j] = x < a.nmx && kin ? src[(size_t)x * a.nky] : make_float2(0.f, 0.f);
-        }
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int x = x0 + 64 * j;
-            if (x < a.nmx) dst[lds_pad(x)] = st[j];
-        }
-    }
-    __syncthreads();
     float2 v[NWF][P];
-#pragma unroll
-    for (int k = 0; k < NWF; ++k) {
-        float2* buf = smem + (w * NWF + k) * L;
+    auto column = [&](int k) {  // a column from its buffer into registers, forward x-FFT
+        float2* buf = smem + (w * NB + (ONE ? 0 : k)) * L;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int x = t + 64 * q;
+            const int x = t + G * q;
             v[k][q] = x < a.nmx ? buf[lds_pad(x)] : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
         xfft<NX, -1, BX>(v[k], buf, a, t);
+    };
+    {
+        float2 st[NWF][P];
+#pragma unroll
+        for (int k = 0; k < NWF; ++k) tile_load<P, G>(st[k], state(a, item, wf_of(k)) + ky0 + c, a, x0, kin);
+#pragma unroll
+        for (int k = 0; k < NWF; ++k) {
+            if (ONE && k > 0) __syncthreads();  // the buffers are still in use by the first's transforms
+            tile_put<P, G>(st[k], smem + (c * NB + (ONE ? 0 : k)) * L, a, x0);
+            if (ONE) {
+                __syncthreads();
+                column(k);
+            }
+        }
+    }
+    if constexpr (!ONE) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NWF; ++k) column(k);
     }
     const int iw = a.ifmin + a.f0 + item;
     const double wd = (double)iw * a.dw;
@@ -315,42 +365,43 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
 #pragma unroll
     for (int k = 0; k < NWF; ++k) cj[k] = wf_of(k) == 0 ? a.conj_src : a.conj_rec;
     float2 phm[P];
-    const bool mirror = BX == kLenPow2 && a.prec == SWEM_PREC_KZ64;
+    const bool mirror = BX == kLenPow2 && PREC == SWEM_PREC_KZ64;
     if constexpr (BX == kLenPow2)
         if (mirror) kz_phases64_col<NX>(a, c0, t, phm);
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         const float2 ph = mirror ? phm[q]
-                          : a.prec == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + 64 * q)
-                                                     : kz_phase(a, wd, p2, a.p2f[a.iz], t + 64 * q, iky);
+                          : PREC == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + G * q)
+                                                     : kz_phase(a, wd, p2, a.p2f[a.iz], t + G * q, iky);
 #pragma unroll
         for (int k = 0; k < NWF; ++k) v[k][q] = cmul(v[k][q], make_float2(ph.x, cj[k] ? -ph.y : ph.y));
     }
+    // recomputed rather than kept live through the transforms (register pressure)
+    int c1 = c, x1 = x0;
+    asm volatile("" : "+v"(c1), "+v"(x1));
+    const bool kout = ky0 + c1 < a.nky;
 #pragma unroll
     for (int k = 0; k < NWF; ++k) {
-        float2* buf = smem + (w * NWF + k) * L;
+        float2* buf = smem + (w * NB + (ONE ? 0 : k)) * L;
+        if (ONE && k > 0) __syncthreads();  // the first wavefield's tile has been read
         wave_sync_lds();
         xfft<NX, +1, BX>(v[k], buf, a, t);
         wave_sync_lds();
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int x = t + 64 * q;
+            const int x = t + G * q;
             if (x < a.nmx) buf[lds_pad(x)] = v[k][q];
         }
-    }
-    __syncthreads();
-    // recomputed rather than kept live through the transforms (register pressure)
-    int c1 = c, x1 = x0;
-    asm volatile("" : "+v"(c1), "+v"(x1));
-#pragma unroll
-    for (int k = 0; k < NWF; ++k) {
-        float2* dst = state(a, item, wf_of(k)) + ky0 + c1;
-        const float2* src = smem + (c1 * NWF + k) * L;
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int x = x1 + 64 * j;
-            if (x < a.nmx && ky0 + c1 < a.nky) dst[(size_t)x * a.nky] = src[lds_pad(x)];
+        if (ONE) {
+            __syncthreads();
+            tile_store<P, G>(state(a, item, wf_of(k)) + ky0 + c1, smem + c1 * L, a, x1, kout);
         }
+    }
+    if constexpr (!ONE) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NWF; ++k)
+            tile_store<P, G>(state(a, item, wf_of(k)) + ky0 + c1, smem + (c1 * NB + k) * L, a, x1, kout);
     }
 }
 
@@ -368,11 +419,11 @@ __device__ __forceinline__ float2* rslice(const March3DArgs& a, int item, int wf
 
 // x-pass: as march3d_cols up to the forward x-FFT, then per vref in use: kz phase of
 // vref[ir][iz] (conj for a -dz step), inverse x-FFT, slice tile written through LDS.
-template <int NX, int NWF, int C, int BX>
-__global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 512 ? 2 : 4))) void march3d_cols_pspi(
+template <int NX, int NWF, int C, int BX, int PREC>
+__global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 512 || line_lanes(NX, BX) * 16 == NX ? 2 : 4))) void march3d_cols_pspi(
     March3DArgs a)
 {
-    constexpr int P = NX / 64;
+    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;
     constexpr int L = LdsLen<NX>::value;
     extern __shared__ float2 smem[];
     const int tiles = (a.nky + C - 1) / C;  // the last tile is partial when C does not divide nky
@@ -382,39 +433,44 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
     if (b < full) b = (b & 7) * (full >> 3) + (b >> 3);
     const int item = b / tiles;
     const int ky0 = (b - item * tiles) * C;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int wf1 = (a.wmask & 1) ? 0 : 1;
     auto wf_of = [&](int k) { return NWF == 2 ? k : wf1; };
+    // buffer (c * NB + k) holds column ky0 + c of the k-th stepped wavefield (ONE: of each in turn);
+    // the loads of both wavefields are all issued before the first LDS write
+    constexpr bool ONE = NWF == 2 && G < 64;
+    constexpr int NB = ONE ? 1 : NWF;
     const int c = threadIdx.x % C, x0 = threadIdx.x / C;
     const bool kin = ky0 + c < a.nky;
-#pragma unroll
-    for (int k = 0; k < NWF; ++k) {
-        const float2* src = state(a, item, wf_of(k)) + ky0 + c;
-        float2* dst = smem + (c * NWF + k) * L;
-        float2 st[P];
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int x = x0 + 64 * j;
-            st[j] = x < a.nmx && kin ? src[(size_t)x * a.nky] : make_float2(0.f, 0.f);
-        }
-#pragma unroll
-        for (int j = 0; j < P; ++j) {
-            const int x = x0 + 64 * j;
-            if (x < a.nmx) dst[lds_pad(x)] = st[j];
-        }
-    }
-    __syncthreads();
     float2 v[NWF][P];
-#pragma unroll
-    for (int k = 0; k < NWF; ++k) {
-        float2* buf = smem + (w * NWF + k) * L;
+    auto column = [&](int k) {  // a column from its buffer into registers, forward x-FFT
+        float2* buf = smem + (w * NB + (ONE ? 0 : k)) * L;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int x = t + 64 * q;
+            const int x = t + G * q;
             v[k][q] = x < a.nmx ? buf[lds_pad(x)] : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
         xfft<NX, -1, BX>(v[k], buf, a, t);
+    };
+    {
+        float2 st[NWF][P];
+#pragma unroll
+        for (int k = 0; k < NWF; ++k) tile_load<P, G>(st[k], state(a, item, wf_of(k)) + ky0 + c, a, x0, kin);
+#pragma unroll
+        for (int k = 0; k < NWF; ++k) {
+            if (ONE && k > 0) __syncthreads();  // the buffers are still in use by the first's transforms
+            tile_put<P, G>(st[k], smem + (c * NB + (ONE ? 0 : k)) * L, a, x0);
+            if (ONE) {
+                __syncthreads();
+                column(k);
+            }
+        }
+    }
+    if constexpr (!ONE) {
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < NWF; ++k) column(k);
     }
     const int iw = a.ifmin + a.f0 + item;
     const double wd = (double)iw * a.dw;
@@ -427,6 +483,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
     const uint32_t used = a.used[a.iz];
     int c1 = c, x1 = x0;
     asm volatile("" : "+v"(c1), "+v"(x1));
+    const bool kout = ky0 + c1 < a.nky;
     for (int ir = 0; ir < a.nref; ++ir) {
         if (!((used >> ir) & 1u)) continue;
         const double p2 = a.p2[(size_t)a.iz * a.nref + ir];
@@ -435,7 +492,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
         // the two wavefields of a migration share each phase (the one-wavefield shapes keep
         // computing it per point: the mirrored set would spill there)
         float2 phm[P];
-        const bool mirror = NWF == 2 && BX == kLenPow2 && a.prec == SWEM_PREC_KZ64;
+        const bool mirror = NWF == 2 && BX == kLenPow2 && PREC == SWEM_PREC_KZ64;
         if constexpr (NWF == 2 && BX == kLenPow2)
             if (mirror) kz_phases64_col<NX>(a, c0, t, phm);
 #pragma unroll
@@ -444,32 +501,32 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
 #pragma unroll
             for (int q = 0; q < P; ++q) {
                 const float2 ph = mirror ? phm[q]
-                                  : a.prec == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + 64 * q)
-                                                             : kz_phase(a, wd, p2, p2f, t + 64 * q, iky);
+                                  : PREC == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + G * q)
+                                                             : kz_phase(a, wd, p2, p2f, t + G * q, iky);
                 bq[q] = cmul(v[k][q], make_float2(ph.x, cj[k] ? -ph.y : ph.y));
             }
-            float2* buf = smem + (w * NWF + k) * L;
+            float2* buf = smem + (w * NB + (ONE ? 0 : k)) * L;
             wave_sync_lds();
             xfft<NX, +1, BX>(bq, buf, a, t);
             wave_sync_lds();
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int x = t + 64 * q;
+                const int x = t + G * q;
                 if (x < a.nmx) buf[lds_pad(x)] = bq[q];
             }
-        }
-        __syncthreads();
-#pragma unroll
-        for (int k = 0; k < NWF; ++k) {
-            float2* dst = rslice(a, item, wf_of(k), ir) + ky0 + c1;
-            const float2* src = smem + (c1 * NWF + k) * L;
-#pragma unroll
-            for (int j = 0; j < P; ++j) {
-                const int x = x1 + 64 * j;
-                if (x < a.nmx && ky0 + c1 < a.nky) dst[(size_t)x * a.nky] = src[lds_pad(x)];
+            if (ONE) {
+                __syncthreads();
+                tile_store<P, G>(rslice(a, item, wf_of(k), ir) + ky0 + c1, smem + c1 * L, a, x1, kout);
+                __syncthreads();  // the tile is rewritten by the next wavefield or vref
             }
         }
-        __syncthreads();  // the tile is rewritten by the next vref
+        if constexpr (!ONE) {
+            __syncthreads();
+#pragma unroll
+            for (int k = 0; k < NWF; ++k)
+                tile_store<P, G>(rslice(a, item, wf_of(k), ir) + ky0 + c1, smem + (c1 * NB + k) * L, a, x1, kout);
+            __syncthreads();  // the tile is rewritten by the next vref
+        }
     }
 }
 
@@ -477,11 +534,11 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
 // vref in use at the depth, the slice R[ir] (the weighted wavefield, y transformed) is x
 // transformed and multiplied by its kz phase (conj for the -dz step), the products are summed,
 // and one inverse x-FFT gives the stepped receiver (y transformed) in the state.
-template <int NX, int C, int BX>
-__global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 512 ? 2 : 4))) void march3d_cols_gather(
+template <int NX, int C, int BX, int PREC>
+__global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 512 ? 2 : 4))) void march3d_cols_gather(
     March3DArgs a)
 {
-    constexpr int P = NX / 64;
+    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;
     constexpr int L = LdsLen<NX>::value;
     extern __shared__ float2 smem[];
     const int tiles = (a.nky + C - 1) / C;
@@ -491,7 +548,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
     if (b < full) b = (b & 7) * (full >> 3) + (b >> 3);
     const int item = b / tiles;
     const int ky0 = (b - item * tiles) * C;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int c = threadIdx.x % C, x0 = threadIdx.x / C;
     const bool kin = ky0 + c < a.nky;
     const int iw = a.ifmin + a.f0 + item;
@@ -513,12 +570,12 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
             float2 st[P];
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                const int x = x0 + 64 * j;
+                const int x = x0 + G * j;
                 st[j] = x < a.nmx && kin ? src[(size_t)x * a.nky] : make_float2(0.f, 0.f);
             }
 #pragma unroll
             for (int j = 0; j < P; ++j) {
-                const int x = x0 + 64 * j;
+                const int x = x0 + G * j;
                 if (x < a.nmx) dst[lds_pad(x)] = st[j];
             }
         }
@@ -526,7 +583,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
         float2 v[P];
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int x = t + 64 * q;
+            const int x = t + G * q;
             v[q] = x < a.nmx ? buf[lds_pad(x)] : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
@@ -536,8 +593,8 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
         const double c0 = wd * wd * p2 - ky * ky;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const float2 ph = a.prec == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + 64 * q)
-                                                       : kz_phase(a, wd, p2, p2f, t + 64 * q, iky);
+            const float2 ph = PREC == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + G * q)
+                                                       : kz_phase(a, wd, p2, p2f, t + G * q, iky);
             acc[q] = cadd(acc[q], cmul(v[q], make_float2(ph.x, a.conj_rec ? -ph.y : ph.y)));
         }
         __syncthreads();  // the tile is restaged for the next vref
@@ -546,7 +603,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
     wave_sync_lds();
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int x = t + 64 * q;
+        const int x = t + G * q;
         if (x < a.nmx) buf[lds_pad(x)] = acc[q];
     }
     __syncthreads();
@@ -556,7 +613,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
     const float2* src = smem + c1 * L;
 #pragma unroll
     for (int j = 0; j < P; ++j) {
-        const int x = x1 + 64 * j;
+        const int x = x1 + G * j;
         if (x < a.nmx && ky0 + c1 < a.nky) dst[(size_t)x * a.nky] = src[lds_pad(x)];
     }
 }
@@ -564,16 +621,16 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 51
 // u = the pspiop selection of row x of wavefield wf from the slices of depth iz_sel: inverse
 // y-FFT of each slice in use, per point the slice of its iref1, real part where cut.
 template <int NY, int BY>
-__device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, int wf, int x, float2 (&u)[NY / 64],
+__device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, int wf, int x, LinePoints<NY, BY>& u,
                                                 float2* buf, int t)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     const uint32_t used = a.used[a.iz_sel];
     const uint8_t* sr = a.sel + (size_t)a.iz_sel * a.nm + (size_t)x * a.nmy;
     uint8_t s1[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int y = t + 64 * q;
+        const int y = t + G * q;
         s1[q] = y < a.nmy ? sr[y] : (uint8_t)0x7f;
         u[q] = make_float2(0.f, 0.f);
     }
@@ -586,7 +643,7 @@ __device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, 
         const float* wr = a.w2 + (size_t)a.iz_sel * a.nm + (size_t)x * a.nmy;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
+            const int y = t + G * q;
             s2[q] = y < a.nmy ? sr2[y] : (uint8_t)0x7f;
             wt2[q] = y < a.nmy ? wr[y] : 0.f;
         }
@@ -596,7 +653,7 @@ __device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, 
         const float2* row = rslice(a, item, wf, ir) + (size_t)x * a.nky;
         float2 bq[P];
 #pragma unroll
-        for (int q = 0; q < P; ++q) bq[q] = yin<BY>(a, t + 64 * q) ? row[t + 64 * q] : make_float2(0.f, 0.f);
+        for (int q = 0; q < P; ++q) bq[q] = yin<BY>(a, t + G * q) ? row[t + G * q] : make_float2(0.f, 0.f);
         yfft<NY, +1, BY>(bq, buf, a, t);
         wave_sync_lds();
         if (a.linear) {
@@ -637,12 +694,12 @@ __device__ __forceinline__ float pspi3_weight(uint8_t s1, uint8_t s2, float w2, 
 template <int NY, int BY>
 __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, int phase)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const int ngroups = (a.nitem + F - 1) / F;
     const int g = blockIdx.x % ngroups, x = blockIdx.x / ngroups;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int item = g * F + w;
     const bool active = item < a.nitem;
     float2* buf = smem + w * L;
@@ -660,14 +717,14 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         } else {
             const float2* src = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
-            for (int q = 0; q < P; ++q) u[q] = yin<BY>(a, t + 64 * q) ? src[t + 64 * q] : make_float2(0.f, 0.f);
+            for (int q = 0; q < P; ++q) u[q] = yin<BY>(a, t + G * q) ? src[t + G * q] : make_float2(0.f, 0.f);
             yfft<NY, +1, BY>(u, buf, a, t);
             wave_sync_lds();
         }
         if (phase == 5) {
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int y = t + 64 * q;
+                const int y = t + G * q;
                 if (y < a.nmy) a.dgw[((size_t)x * a.nmy + y) * a.nf + fl] = u[q];
             }
             return;
@@ -679,7 +736,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         float wt2[P];
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
+            const int y = t + G * q;
             if (y < a.nmy) {
                 u[q] = cadd(u[q], cscale(sm[y], mt[y]));
                 s1[q] = a.sel[o + y];
@@ -701,7 +758,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
             yfft<NY, -1, BY>(v, buf, a, t);
             float2* dst = rslice(a, item, 1, ir) + (size_t)x * a.nky;
 #pragma unroll
-            for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = v[q];
+            for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = v[q];
         }
         return;
     }
@@ -714,7 +771,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
             float2* sm = a.smig + ((size_t)item * a.nz + a.iz) * a.nm + (size_t)x * a.nmy;
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int y = t + 64 * q;
+                const int y = t + G * q;
                 if (y < a.nmy) sm[y] = a.ds ? u[q] : make_float2(0.f, 0.f);
             }
             if (!(a.ds && a.next_s)) return;
@@ -728,7 +785,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
             if (phase == 3) {
 #pragma unroll
                 for (int q = 0; q < P; ++q) {
-                    const int y = t + 64 * q;
+                    const int y = t + G * q;
                     if (y < a.nmy) a.dgw[((size_t)x * a.nmy + y) * a.nf + fl] = u[q];
                 }
                 return;
@@ -737,7 +794,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
             const float* mt = a.mT + (size_t)a.iz * a.nm + (size_t)x * a.nmy;
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int y = t + 64 * q;
+                const int y = t + G * q;
                 if (y < a.nmy) u[q] = cadd(u[q], cscale(sm[y], mt[y]));
             }
         }
@@ -745,7 +802,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         yfft<NY, -1, BY>(u, buf, a, t);
         float2* dst = state(a, item, phase == 1 ? 0 : 1) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = u[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = u[q];
         return;
     }
     // phase 0: migration
@@ -759,7 +816,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         // an unstepped source: its state is FFT_y(u), so the inverse transform returns nky u
         const float2* src = state(a, item, 0) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) vs[q] = yin<BY>(a, t + 64 * q) ? src[t + 64 * q] : make_float2(0.f, 0.f);
+        for (int q = 0; q < P; ++q) vs[q] = yin<BY>(a, t + G * q) ? src[t + G * q] : make_float2(0.f, 0.f);
         yfft<NY, +1, BY>(vs, buf, a, t);
         wave_sync_lds();
         const float rn = 1.f / (float)a.nky;  // exact when nky is a power of two
@@ -771,13 +828,13 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
     const float factor = iw == 0 ? 1.f : 2.f;
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        if (t + 64 * q >= a.nmy) vs[q] = vr[q] = make_float2(0.f, 0.f);
+        if (t + G * q >= a.nmy) vs[q] = vr[q] = make_float2(0.f, 0.f);
         cc[q] = (active && a.dr) ? factor * (vr[q].x * vs[q].x + vr[q].y * vs[q].y) : 0.f;
     }
     wave_sync_lds();
     float* red = reinterpret_cast<float*>(buf);
 #pragma unroll
-    for (int q = 0; q < P; ++q) red[t + 64 * q] = cc[q];
+    for (int q = 0; q < P; ++q) red[t + G * q] = cc[q];
     __syncthreads();
     float* part = a.partial + (size_t)g * a.nm + (size_t)x * a.nmy;
     for (int y = threadIdx.x; y < a.nmy; y += blockDim.x) {
@@ -790,14 +847,14 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         yfft<NY, -1, BY>(vs, buf, a, t);
         float2* dst = state(a, item, 0) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = vs[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vs[q];
         wave_sync_lds();
     }
     if (active && a.dr && a.next_r) {
         yfft<NY, -1, BY>(vr, buf, a, t);
         float2* dst = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = vr[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vr[q];
     }
 }
 
@@ -805,15 +862,15 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
 // of frequency item g F + f.  ds / dr: the source / receiver was stepped at this depth; next_s /
 // next_r: it is stepped at the next depth (its forward y-FFT is needed); the imaging runs when dr.
 // The split-step phase is computed once and applied conjugated to the source.
-template <int NY, int BY>
+template <int NY, int BY, int PREC>
 __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs a, int F)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const int ngroups = (a.nitem + F - 1) / F;
     const int g = blockIdx.x % ngroups, x = blockIdx.x / ngroups;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int item = g * F + w;
     const bool active = item < a.nitem;
     const int iw = a.ifmin + a.f0 + (active ? item : 0);
@@ -827,12 +884,12 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
     if (need_s) {
         const float2* src = state(a, item, 0) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) vs[q] = yin<BY>(a, t + 64 * q) ? src[t + 64 * q] : make_float2(0.f, 0.f);
+        for (int q = 0; q < P; ++q) vs[q] = yin<BY>(a, t + G * q) ? src[t + G * q] : make_float2(0.f, 0.f);
     }
     if (need_r) {
         const float2* src = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) vr[q] = yin<BY>(a, t + 64 * q) ? src[t + 64 * q] : make_float2(0.f, 0.f);
+        for (int q = 0; q < P; ++q) vr[q] = yin<BY>(a, t + G * q) ? src[t + G * q] : make_float2(0.f, 0.f);
     }
     if (need_s) {
         yfft<NY, +1, BY>(vs, buf, a, t);
@@ -849,10 +906,10 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
     const float tx = a.taper_x[x];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int y = t + 64 * q;
+        const int y = t + G * q;
         if (y < a.nmy) {
             if (a.ds || a.dr) {
-                const float2 sp = ss_phase(a, wd, (size_t)x * a.nmy + y);
+                const float2 sp = ss_phase<PREC>(a, wd, (size_t)x * a.nmy + y);
                 const float tp = tx * a.taper_y[y];
                 if (a.ds) vs[q] = cscale(cmulc(vs[q], sp), tp);
                 if (a.dr) vr[q] = cscale(cmul(vr[q], sp), tp);
@@ -866,7 +923,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
     wave_sync_lds();
     float* red = reinterpret_cast<float*>(buf);
 #pragma unroll
-    for (int q = 0; q < P; ++q) red[t + 64 * q] = cc[q];
+    for (int q = 0; q < P; ++q) red[t + G * q] = cc[q];
     __syncthreads();
     float* part = a.partial + (size_t)g * a.nm + (size_t)x * a.nmy;
     for (int y = threadIdx.x; y < a.nmy; y += blockDim.x) {
@@ -880,14 +937,14 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
         yfft<NY, -1, BY>(vs, buf, a, t);
         float2* dst = state(a, item, 0) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = vs[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vs[q];
         wave_sync_lds();
     }
     if (active && a.dr && a.next_r) {
         yfft<NY, -1, BY>(vr, buf, a, t);
         float2* dst = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = vr[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vr[q];
     }
 }
 
@@ -901,15 +958,15 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
 //           receiver's step; at the first call the state is the source trace, later IFFTy of
 //           the previous step's result is stored in smig at depth iz_sel; with ds the next step
 //           starts (taper, conj(SS), FFTy).
-template <int NY, int BY>
+template <int NY, int BY, int PREC>
 __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs a, int F, int phase)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const int ngroups = (a.nitem + F - 1) / F;
     const int g = blockIdx.x % ngroups, x = blockIdx.x / ngroups;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int item = g * F + w;
     if (item >= a.nitem) return;  // no workgroup barriers in this kernel
     const int fl = a.f0 + item;
@@ -923,31 +980,31 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
         if (a.first) {
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int y = t + 64 * q;
+                const int y = t + G * q;
                 v[q] = (y < a.nmy && x * a.nmy + y == a.igx) ? a.spec_s[fl] : make_float2(0.f, 0.f);
             }
         } else {
 #pragma unroll
-            for (int q = 0; q < P; ++q) v[q] = yin<BY>(a, t + 64 * q) ? row[t + 64 * q] : make_float2(0.f, 0.f);
+            for (int q = 0; q < P; ++q) v[q] = yin<BY>(a, t + G * q) ? row[t + G * q] : make_float2(0.f, 0.f);
             yfft<NY, +1, BY>(v, buf, a, t);
             float2* sm = a.smig + ((size_t)item * a.nz + a.iz_sel) * a.nm + (size_t)x * a.nmy;
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int y = t + 64 * q;
+                const int y = t + G * q;
                 if (y < a.nmy) sm[y] = v[q];
             }
         }
         if (!a.ds) return;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
-            v[q] = y < a.nmy ? cmulc(cscale(v[q], tx * a.taper_y[y]), ss_phase(a, wd, (size_t)x * a.nmy + y))
+            const int y = t + G * q;
+            v[q] = y < a.nmy ? cmulc(cscale(v[q], tx * a.taper_y[y]), ss_phase<PREC>(a, wd, (size_t)x * a.nmy + y))
                              : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
         yfft<NY, -1, BY>(v, buf, a, t);
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) row[t + 64 * q] = v[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) row[t + G * q] = v[q];
         return;
     }
     if (phase == 1 && a.first) {
@@ -955,7 +1012,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
         for (int q = 0; q < P; ++q) v[q] = make_float2(0.f, 0.f);
     } else {
 #pragma unroll
-        for (int q = 0; q < P; ++q) v[q] = yin<BY>(a, t + 64 * q) ? row[t + 64 * q] : make_float2(0.f, 0.f);
+        for (int q = 0; q < P; ++q) v[q] = yin<BY>(a, t + G * q) ? row[t + G * q] : make_float2(0.f, 0.f);
         yfft<NY, +1, BY>(v, buf, a, t);
     }
     const float tx = a.taper_x[x];
@@ -963,23 +1020,23 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
     const float* mt = a.mT + (size_t)a.iz * a.nm + (size_t)x * a.nmy;
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int y = t + 64 * q;
+        const int y = t + G * q;
         if (y >= a.nmy) {
             v[q] = make_float2(0.f, 0.f);
             continue;
         }
         if (phase == 0) {
-            if (a.ds) v[q] = cscale(cmulc(v[q], ss_phase(a, wd, (size_t)x * a.nmy + y)), tx * a.taper_y[y]);
+            if (a.ds) v[q] = cscale(cmulc(v[q], ss_phase<PREC>(a, wd, (size_t)x * a.nmy + y)), tx * a.taper_y[y]);
             sm[y] = a.ds ? v[q] : make_float2(0.f, 0.f);
         } else if (phase == 1) {
             const float2 u = cadd(v[q], cscale(sm[y], mt[y]));
-            v[q] = cmulc(cscale(u, tx * a.taper_y[y]), ss_phase(a, wd, (size_t)x * a.nmy + y));
+            v[q] = cmulc(cscale(u, tx * a.taper_y[y]), ss_phase<PREC>(a, wd, (size_t)x * a.nmy + y));
         }
     }
     if (phase == 2) {
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
+            const int y = t + G * q;
             if (y < a.nmy) a.dgw[((size_t)x * a.nmy + y) * a.nf + fl] = v[q];
         }
         return;
@@ -988,7 +1045,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
     wave_sync_lds();
     yfft<NY, -1, BY>(v, buf, a, t);
 #pragma unroll
-    for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) row[t + 64 * q] = v[q];
+    for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) row[t + G * q] = v[q];
 }
 
 // ------------------------------------------------------------------------ elastic WEM (3-D)
@@ -1009,11 +1066,11 @@ __device__ __forceinline__ float2* eslot(const March3DArgs& a, const Ewem3DArgs&
 template <int NY, int BY>
 __global__ __launch_bounds__(256) void ewem3d_init(March3DArgs a, Ewem3DArgs e)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     constexpr int L = LdsLen<NY>::value;
-    __shared__ float2 lds[4 * L];
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
-    const size_t row = (size_t)blockIdx.x * 4 + w;
+    __shared__ float2 lds[256 / G * L];
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
+    const size_t row = (size_t)blockIdx.x * (256 / G) + w;
     if (row >= (size_t)a.nitem * 3 * a.nmx) return;  // whole waves only
     const int x = (int)(row % a.nmx);
     const int s = (int)((row / a.nmx) % 3);
@@ -1022,7 +1079,7 @@ __global__ __launch_bounds__(256) void ewem3d_init(March3DArgs a, Ewem3DArgs e)
     float2 v[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int y = t + 64 * q;
+        const int y = t + G * q;
         float2 u = make_float2(0.f, 0.f);
         if (y < a.nmy) {
             const size_t ixy = (size_t)x * a.nmy + y;
@@ -1034,7 +1091,7 @@ __global__ __launch_bounds__(256) void ewem3d_init(March3DArgs a, Ewem3DArgs e)
     yfft<NY, -1, BY>(v, lds + w * L, a, t);
     float2* dst = eslot(a, e, item, s) + (size_t)x * a.nky;
 #pragma unroll
-    for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = v[q];
+    for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = v[q];
 }
 
 // x-pass.  NWF = 1 (e.mode 3): the source (slot 0), kz phase of vp (conj_src).  NWF = 2: the
@@ -1043,10 +1100,10 @@ __global__ __launch_bounds__(256) void ewem3d_init(March3DArgs a, Ewem3DArgs e)
 // truncation to x < nmx between them; else e.mode 2, the kz phases of vp and vs (conj_rec).
 // Columns staged through LDS in tiles of C.
 template <int NX, int NWF, int C, int BX, bool MAPS>
-__global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 1024 ? 2 : (MAPS && NX >= 512 ? 3 : 4)))) void ewem3d_cols(
+__global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 1024 ? 2 : (MAPS && NX >= 512 ? 3 : 4)))) void ewem3d_cols(
     March3DArgs ap, March3DArgs as, Ewem3DArgs e)
 {
-    constexpr int P = NX / 64;
+    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;
     constexpr int L = LdsLen<NX>::value;
     extern __shared__ float2 smem[];
     const March3DArgs& a = ap;
@@ -1057,7 +1114,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
     if (b < full) b = (b & 7) * (full >> 3) + (b >> 3);
     const int item = b / tiles;
     const int ky0 = (b - item * tiles) * C;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     auto slot_of = [&](int k) { return NWF == 1 ? 0 : 1 + k; };
     const int c = threadIdx.x % C, x0 = threadIdx.x / C;
     const bool kin = ky0 + c < a.nky;
@@ -1068,12 +1125,12 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
         float2 st[P];
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            const int x = x0 + 64 * j;
+            const int x = x0 + G * j;
             st[j] = x < a.nmx && kin ? src[(size_t)x * a.nky] : make_float2(0.f, 0.f);
         }
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            const int x = x0 + 64 * j;
+            const int x = x0 + G * j;
             if (x < a.nmx) dst[lds_pad(x)] = st[j];
         }
     }
@@ -1085,7 +1142,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
         float2* buf = smem + (w * NWF + k) * L;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int x = t + 64 * q;
+            const int x = t + G * q;
             u[q] = x < a.nmx ? buf[lds_pad(x)] : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
@@ -1099,7 +1156,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
         wave_sync_lds();
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int x = t + 64 * q;
+            const int x = t + G * q;
             if (x < a.nmx) buf[lds_pad(x)] = u[q];
         }
     };
@@ -1115,7 +1172,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
             const float vp = e.vp0[iz], vs = e.vs0[iz];
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const int k = t + 64 * q;
+                const int k = t + G * q;
                 const float kx = (float)k < (float)n / 2.f ? e.dkxf * (float)k : -(e.dkxf * (float)n - e.dkxf * (float)k);
                 float2 r1, r2;
                 esep_k(kx, wf, vp, vs, sep, e.sep_adj != 0, v[0][q], v[1][q], r1, r2);
@@ -1133,7 +1190,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
                 xfft<NX, +1, BX>(v[k], buf, a, t);
 #pragma unroll
                 for (int q = 0; q < P; ++q)
-                    if (t + 64 * q >= a.nmx) v[k][q] = make_float2(0.f, 0.f);
+                    if (t + G * q >= a.nmx) v[k][q] = make_float2(0.f, 0.f);
                 wave_sync_lds();
                 xfft<NX, -1, BX>(v[k], buf, a, t);
             }
@@ -1163,8 +1220,8 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
 #pragma unroll
             for (int q = 0; q < P; ++q) {
                 const float2 ph = mirror ? phm[q]
-                                  : a.prec == SWEM_PREC_KZ64 ? kz_phase64(pl, c0, t + 64 * q)
-                                                             : kz_phase(pl, wd, p2, pl.p2f[a.iz], t + 64 * q, iky);
+                                  : a.prec == SWEM_PREC_KZ64 ? kz_phase64(pl, c0, t + G * q)
+                                                             : kz_phase(pl, wd, p2, pl.p2f[a.iz], t + G * q, iky);
                 v[q] = cmul(v[q], make_float2(ph.x, cj ? -ph.y : ph.y));
             }
             put(k, v);
@@ -1179,7 +1236,7 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
         const float2* src = smem + (c1 * NWF + k) * L;
 #pragma unroll
         for (int j = 0; j < P; ++j) {
-            const int x = x1 + 64 * j;
+            const int x = x1 + G * j;
             if (x < a.nmx && ky0 + c1 < a.nky) dst[(size_t)x * a.nky] = src[lds_pad(x)];
         }
     }
@@ -1199,13 +1256,13 @@ __global__ __launch_bounds__(64 * C) __attribute__((amdgpu_waves_per_eu(NX >= 10
 template <int NY, int BY>
 __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs as, Ewem3DArgs e, int F, int phase)
 {
-    constexpr int P = NY / 64;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const March3DArgs& a = ap;
     const int ngroups = (a.nitem + F - 1) / F;
     const int g = blockIdx.x % ngroups, x = blockIdx.x / ngroups;
-    const int w = threadIdx.x >> 6, t = threadIdx.x & 63;
+    const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const int item = g * F + w;
     const bool active = item < a.nitem;
     const int fl = a.f0 + (active ? item : 0);
@@ -1215,14 +1272,14 @@ __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs a
     auto load_row = [&](int s, float2 (&v)[P]) {
         const float2* src = eslot(a, e, item, s) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) v[q] = yin<BY>(a, t + 64 * q) ? src[t + 64 * q] : make_float2(0.f, 0.f);
+        for (int q = 0; q < P; ++q) v[q] = yin<BY>(a, t + G * q) ? src[t + G * q] : make_float2(0.f, 0.f);
     };
     auto store_row = [&](int s, float2 (&v)[P]) {
         wave_sync_lds();
         yfft<NY, -1, BY>(v, buf, a, t);
         float2* dst = eslot(a, e, item, s) + (size_t)x * a.nky;
 #pragma unroll
-        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + 64 * q)) dst[t + 64 * q] = v[q];
+        for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = v[q];
     };
     if (phase == 0) {
         const bool do_s = active && e.ds, do_r = active && e.dr;
@@ -1247,7 +1304,7 @@ __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs a
         const float factor = a.ifmin + fl == 0 ? 1.f : 2.f;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
+            const int y = t + G * q;
             cp[q] = cs[q] = 0.f;
             if (y >= a.nmy) {
                 vs[q] = v1[q] = v2[q] = make_float2(0.f, 0.f);
@@ -1271,7 +1328,7 @@ __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs a
             wave_sync_lds();
             float* red = reinterpret_cast<float*>(buf);
 #pragma unroll
-            for (int q = 0; q < P; ++q) red[t + 64 * q] = im == 0 ? cp[q] : cs[q];
+            for (int q = 0; q < P; ++q) red[t + G * q] = im == 0 ? cp[q] : cs[q];
             __syncthreads();
             float* part = (im == 0 ? e.ppart : e.spart) + (size_t)g * a.nm + (size_t)x * a.nmy;
             for (int y = threadIdx.x; y < a.nmy; y += blockDim.x) {
@@ -1298,7 +1355,7 @@ __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs a
         float2* sm = e.smig + ((size_t)item * a.nz + a.iz) * a.nm + (size_t)x * a.nmy;
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
+            const int y = t + G * q;
             if (y >= a.nmy) {
                 vs[q] = make_float2(0.f, 0.f);
                 continue;
@@ -1318,7 +1375,7 @@ __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs a
     if (phase == 4) {
 #pragma unroll
         for (int q = 0; q < P; ++q) {
-            const int y = t + 64 * q;
+            const int y = t + G * q;
             if (y < a.nmy) {
                 const size_t o = ((size_t)x * a.nmy + y) * a.nf + fl;
                 e.dgx[o] = v1[q];
@@ -1331,7 +1388,7 @@ __global__ __launch_bounds__(512) void ewem3d_rows(March3DArgs ap, March3DArgs a
     const size_t mo = (size_t)a.iz * a.nm + (size_t)x * a.nmy;
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        const int y = t + 64 * q;
+        const int y = t + G * q;
         if (y >= a.nmy) {
             v1[q] = v2[q] = make_float2(0.f, 0.f);
             continue;
@@ -1353,10 +1410,10 @@ template <int N, int BL>
 int launch_ewem3d_n(int which, const March3DArgs& ap, const March3DArgs& as, const Ewem3DArgs& e, int F,
                            int phase, hipStream_t st)
 {
-    constexpr int L = LdsLen<N>::value;
+    constexpr int L = LdsLen<N>::value, G = Line<N, BL>::G;
     if (which == 0) {
         const size_t rows = (size_t)ap.nitem * 3 * ap.nmx;
-        hipLaunchKernelGGL((ewem3d_init<N, BL>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, ap, e);
+        hipLaunchKernelGGL((ewem3d_init<N, BL>), dim3((unsigned)((rows + 256 / G - 1) / (256 / G))), dim3(256), 0, st, ap, e);
         SWEM_HIP(hipGetLastError());
         return SWEM_OK;
     }
@@ -1367,7 +1424,7 @@ int launch_ewem3d_n(int which, const March3DArgs& ap, const March3DArgs& as, con
         constexpr int C2 = N >= 1024 ? 4 : 8, C1 = 2 * C2, CM = N >= 512 ? 4 : 8;
         const int C = src ? C1 : (maps ? CM : C2), nwf = src ? 1 : 2;
         const size_t lds = (size_t)C * nwf * L * sizeof(float2);
-        const dim3 grid(ap.nitem * ((ap.nky + C - 1) / C)), block(64 * C);
+        const dim3 grid(ap.nitem * ((ap.nky + C - 1) / C)), block(G * C);
         auto k = src ? ewem3d_cols<N, 1, C1, BL, false>
                      : (maps ? ewem3d_cols<N, 2, CM, BL, true> : ewem3d_cols<N, 2, C2, BL, false>);
         if (lds > 48 * 1024) SWEM_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -1379,14 +1436,19 @@ int launch_ewem3d_n(int which, const March3DArgs& ap, const March3DArgs& as, con
     const size_t lds = (size_t)F * L * sizeof(float2);
     if (lds > 48 * 1024)
         SWEM_HIP(hipFuncSetAttribute((const void*)ewem3d_rows<N, BL>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-    hipLaunchKernelGGL((ewem3d_rows<N, BL>), dim3(ngroups * ap.nmx), dim3(64 * F), lds, st, ap, as, e, F, phase);
+    hipLaunchKernelGGL((ewem3d_rows<N, BL>), dim3(ngroups * ap.nmx), dim3(G * F), lds, st, ap, as, e, F, phase);
     SWEM_HIP(hipGetLastError());
     return SWEM_OK;
 }
 
-// Columns (waves) per x-pass workgroup: 16 buffers of staging per workgroup (8 columns of two
-// wavefields or 16 of one) below nkx = 1024, half that at 1024.
-static int march3d_cols_tile(int nwf, int nkx) { return (nkx >= 1024 ? 8 : 16) / nwf; }
+// Columns per x-pass workgroup.  Whole-wave lines: 16 buffers of staging per workgroup (8 columns of
+// two wavefields or 16 of one) below nkx = 1024, half that at 1024.  Shorter ones (one buffer per
+// column): 256 threads, 38 KB.
+constexpr int tile_cols(int n, int kind, int nwf)
+{
+    return line_lanes(n, kind) < 64 ? 256 / line_lanes(n, kind) : (n >= 1024 ? 8 : 16) / nwf;
+}
+constexpr int tile_bufs(int n, int kind, int nwf) { return line_lanes(n, kind) < 64 ? 1 : nwf; }
 
 template <typename K, typename... X>
 static int launch3(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t st, const March3DArgs& a, X... extra)
@@ -1398,55 +1460,64 @@ static int launch3(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t st, 
     return SWEM_OK;
 }
 
-template <int N, int BL>
-int launch3_n(int which, const March3DArgs& a, int F, int phase, hipStream_t st)
+template <int N, int BL, int PREC>
+static int launch3_prec(int which, const March3DArgs& a, int F, int phase, hipStream_t st)
 {
-    constexpr int L = LdsLen<N>::value;
+    constexpr int L = LdsLen<N>::value, G = Line<N, BL>::G;
     if (which == 0) {  // init
         const size_t rows = (size_t)a.nitem * 2 * a.nmx;
-        hipLaunchKernelGGL((march3d_init<N, BL>), dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, st, a);
+        hipLaunchKernelGGL((march3d_init<N, BL>), dim3((unsigned)((rows + 256 / G - 1) / (256 / G))), dim3(256), 0, st, a);
         SWEM_HIP(hipGetLastError());
         return SWEM_OK;
     }
     if (which == 1) {  // cols
         const int nwf = (a.wmask & 1) + ((a.wmask >> 1) & 1);
-        const int C = march3d_cols_tile(nwf, N);
-        const size_t lds = (size_t)C * nwf * L * sizeof(float2);
-        const dim3 grid(a.nitem * ((a.nky + C - 1) / C)), block(64 * C);
-        constexpr int C2 = N >= 1024 ? 4 : 8, C1 = 2 * C2;
-        return nwf == 2 ? launch3(march3d_cols<N, 2, C2, BL>, grid, block, lds, st, a)
-                        : launch3(march3d_cols<N, 1, C1, BL>, grid, block, lds, st, a);
+        constexpr int C2 = tile_cols(N, BL, 2), C1 = tile_cols(N, BL, 1);
+        const int C = nwf == 2 ? C2 : C1;
+        const size_t lds = (size_t)C * tile_bufs(N, BL, nwf) * L * sizeof(float2);
+        const dim3 grid(a.nitem * ((a.nky + C - 1) / C)), block(G * C);
+        return nwf == 2 ? launch3(march3d_cols<N, 2, C2, BL, PREC>, grid, block, lds, st, a)
+                        : launch3(march3d_cols<N, 1, C1, BL, PREC>, grid, block, lds, st, a);
     }
     if (which == 4) {  // PSPI x-pass
         const int nwf = (a.wmask & 1) + ((a.wmask >> 1) & 1);
-        const int C = march3d_cols_tile(nwf, N);
-        const size_t lds = (size_t)C * nwf * L * sizeof(float2);
-        const dim3 grid(a.nitem * ((a.nky + C - 1) / C)), block(64 * C);
-        constexpr int C2 = N >= 1024 ? 4 : 8, C1 = 2 * C2;
-        return nwf == 2 ? launch3(march3d_cols_pspi<N, 2, C2, BL>, grid, block, lds, st, a)
-                        : launch3(march3d_cols_pspi<N, 1, C1, BL>, grid, block, lds, st, a);
+        constexpr int C2 = tile_cols(N, BL, 2), C1 = tile_cols(N, BL, 1);
+        const int C = nwf == 2 ? C2 : C1;
+        const size_t lds = (size_t)C * tile_bufs(N, BL, nwf) * L * sizeof(float2);
+        const dim3 grid(a.nitem * ((a.nky + C - 1) / C)), block(G * C);
+        return nwf == 2 ? launch3(march3d_cols_pspi<N, 2, C2, BL, PREC>, grid, block, lds, st, a)
+                        : launch3(march3d_cols_pspi<N, 1, C1, BL, PREC>, grid, block, lds, st, a);
     }
     if (which == 6) {  // linear-mode modelling receiver x-pass (gather over vrefs)
-        constexpr int CG = N >= 1024 ? 8 : 16;
+        constexpr int CG = tile_cols(N, BL, 1);
         const size_t lds = (size_t)CG * L * sizeof(float2);
-        const dim3 grid(a.nitem * ((a.nky + CG - 1) / CG)), block(64 * CG);
-        return launch3(march3d_cols_gather<N, CG, BL>, grid, block, lds, st, a);
+        const dim3 grid(a.nitem * ((a.nky + CG - 1) / CG)), block(G * CG);
+        return launch3(march3d_cols_gather<N, CG, BL, PREC>, grid, block, lds, st, a);
     }
     const int ngroups = (a.nitem + F - 1) / F;
     if (which == 5) {
         const size_t lds = (size_t)F * L * sizeof(float2);
-        return launch3(march3d_rows_pspi<N, BL>, dim3(ngroups * a.nmx), dim3(64 * F), lds, st, a, F, phase);
+        return launch3(march3d_rows_pspi<N, BL>, dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F, phase);
     }
     if (which == 2) {
         const size_t lds = (size_t)F * L * sizeof(float2);
-        return launch3(march3d_rows_adj<N, BL>, dim3(ngroups * a.nmx), dim3(64 * F), lds, st, a, F);
+        return launch3(march3d_rows_adj<N, BL, PREC>, dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F);
     }
     const size_t lds = (size_t)F * L * sizeof(float2);
-    SWEM_HIP(hipFuncSetAttribute((const void*)march3d_rows_fwd<N, BL>, hipFuncAttributeMaxDynamicSharedMemorySize,
+    SWEM_HIP(hipFuncSetAttribute((const void*)march3d_rows_fwd<N, BL, PREC>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                  (int)lds));
-    hipLaunchKernelGGL((march3d_rows_fwd<N, BL>), dim3(ngroups * a.nmx), dim3(64 * F), lds, st, a, F, phase);
+    hipLaunchKernelGGL((march3d_rows_fwd<N, BL, PREC>), dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F, phase);
     SWEM_HIP(hipGetLastError());
     return SWEM_OK;
+}
+
+// The naive-FP32 phases (library sine and cosine per point) are kernels of their own: beside the KZ64
+// path in one kernel they triple its code.
+template <int N, int BL>
+int launch3_n(int which, const March3DArgs& a, int F, int phase, hipStream_t st)
+{
+    return a.prec == SWEM_PREC_KZ64 ? launch3_prec<N, BL, SWEM_PREC_KZ64>(which, a, F, phase, st)
+                                    : launch3_prec<N, BL, SWEM_PREC_FP32>(which, a, F, phase, st);
 }
 
 }  // namespace swem
