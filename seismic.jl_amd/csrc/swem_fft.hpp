@@ -168,6 +168,66 @@ struct Dft<5, SIGN> {
     }
 };
 
+// cos and sin of 2 pi m / R, m = 1 .. (R - 1) / 2
+template <int R>
+struct OddTable;
+template <>
+struct OddTable<7> {
+    static constexpr float c[3] = {0.62348980185873359439f, -0.22252093395631433737f, -0.90096886790241903498f};
+    static constexpr float s[3] = {0.78183148246802980363f, 0.97492791218182361934f, 0.43388373911755823142f};
+};
+template <>
+struct OddTable<11> {
+    static constexpr float c[5] = {0.84125353283118120551f, 0.41541501300188643508f, -0.1423148382732850048f, -0.65486073394528498959f, -0.95949297361449736865f};
+    static constexpr float s[5] = {0.54064081745559755543f, 0.90963199535451833011f, 0.98982144188093279524f, 0.7557495743542582689f, 0.28173255684142967104f};
+};
+template <>
+struct OddTable<13> {
+    static constexpr float c[6] = {0.88545602565320991051f, 0.56806474673115592289f, 0.12053668025532300601f, -0.35460488704253545489f, -0.74851074817110119231f, -0.9709418174260520118f};
+    static constexpr float s[6] = {0.46472317204376850652f, 0.82298386589365635224f, 0.99270887409805397272f, 0.93501624268541483342f, 0.66312265824079519305f, 0.23931566428755768339f};
+};
+
+// Prime radices 7, 11, 13: with a_j = x_j + x_(R-j), b_j = x_j - x_(R-j), j = 1 .. H = (R - 1) / 2,
+// X_k and X_(R-k) = x_0 + sum_j cos(2 pi j k / R) a_j +- SIGN i sum_j sin(2 pi j k / R) b_j.
+template <int R, int SIGN>
+struct DftOdd {
+    static __device__ __forceinline__ void run(float2 (&v)[R])
+    {
+        constexpr int H = (R - 1) / 2;
+        float2 a[H], b[H];
+        const float2 x0 = v[0];
+        float2 sum = x0;
+#pragma unroll
+        for (int j = 0; j < H; ++j) {
+            a[j] = cadd(v[j + 1], v[R - 1 - j]);
+            b[j] = csub(v[j + 1], v[R - 1 - j]);
+            sum = cadd(sum, a[j]);
+        }
+        v[0] = sum;
+#pragma unroll
+        for (int k = 1; k <= H; ++k) {
+            float2 p = x0, q = make_float2(0.f, 0.f);
+#pragma unroll
+            for (int j = 0; j < H; ++j) {
+                const int m = ((j + 1) * k) % R;  // angle 2 pi m / R: m <= H, or the mirrored R - m
+                const float c = OddTable<R>::c[(m <= H ? m : R - m) - 1];
+                const float s = m <= H ? OddTable<R>::s[m - 1] : -OddTable<R>::s[R - m - 1];
+                p = make_float2(fmaf(c, a[j].x, p.x), fmaf(c, a[j].y, p.y));
+                q = make_float2(fmaf(s, b[j].x, q.x), fmaf(s, b[j].y, q.y));
+            }
+            q = mul_si<SIGN>(q);
+            v[k] = cadd(p, q);
+            v[R - k] = csub(p, q);
+        }
+    }
+};
+template <int SIGN>
+struct Dft<7, SIGN> : DftOdd<7, SIGN> {};
+template <int SIGN>
+struct Dft<11, SIGN> : DftOdd<11, SIGN> {};
+template <int SIGN>
+struct Dft<13, SIGN> : DftOdd<13, SIGN> {};
+
 // Bank-conflict padding: one complex inserted every 2^SH.  The LDS has 64 banks of 4 bytes (32
 // complex per row).  A Stockham pass writes at lane stride R (first pass) or in groups of NS
 // lanes, then reads back at unit lane stride; SH is chosen per pass so both the writes and the
@@ -517,7 +577,7 @@ __device__ __forceinline__ void fft2(float2 (&u)[P], float2 (&v)[P], float2* bu,
 }
 
 // ------------------------------------------------------------------ mixed-radix transforms
-// A length n = 2^a 3^b 5^c held in an array of M >= n points (M a power of two; T = M / P
+// A length n = 2^a 3^b 5^c 7^d 11^e 13^f held in an array of M >= n points (M a power of two; T = M / P
 // threads, point j = t + q T in v[q]; entries j >= n are zero on input and on output).  The
 // transform runs in LDS: the points are stored in natural order; every pass of radix R (in the
 // plan's order) reads butterfly b < n / R at b + r n / R, multiplies input r by
@@ -595,7 +655,8 @@ __device__ __forceinline__ void mixed_pass(const float2* src, float2* dst, const
     sync();
 }
 
-template <int M, int P, int SIGN, bool PP, class Plan, class Sync>
+// PRIME: the plan may hold the radices 7, 11 and 13.
+template <int M, int P, int SIGN, bool PP, bool PRIME, class Plan, class Sync>
 __device__ __forceinline__ void mixed_fft(float2 (&v)[P], float2* buf0, float2* buf1, const float2* __restrict__ tw,
                                           const Plan& mr, int t, int& pp, Sync sync)
 {
@@ -612,7 +673,17 @@ __device__ __forceinline__ void mixed_fft(float2 (&v)[P], float2* buf0, float2* 
         float2* nxt = PP ? (cur == buf0 ? buf1 : buf0) : cur;
         const int ns = mr.ns[p], tws = mr.tws[p];
         const uint32_t mg = mr.magic[p];
-        switch (mr.r[p]) {
+        const int r = mr.r[p];
+        if constexpr (PRIME) {
+            if (r == 7 || r > 8) {
+                if (r == 7) mixed_pass<7, SIGN, (P + 6) / 7, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
+                else if (r == 11) mixed_pass<11, SIGN, (P + 10) / 11, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
+                else mixed_pass<13, SIGN, (P + 12) / 13, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
+                cur = nxt;
+                continue;
+            }
+        }
+        switch (r) {
         case 8: mixed_pass<8, SIGN, (P + 7) / 8, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
         case 4: mixed_pass<4, SIGN, (P + 3) / 4, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
         case 2: mixed_pass<2, SIGN, (P + 1) / 2, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;

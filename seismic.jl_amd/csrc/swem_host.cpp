@@ -246,7 +246,7 @@ static void bluestein_tables(int n, int m, std::vector<float2>& chirp, std::vect
 static int length_tables(int n, int m, int kind, DevBuf<float2>& tw, DevBuf<float2>& chirp, DevBuf<float2>& bchirp,
                          MixedRadix& mr)
 {
-    const int len = kind == kLenMixed ? n : m;
+    const int len = is_mixed(kind) ? n : m;
     std::vector<float2> t(len);
     for (int j = 0; j < len; j++) {
         const double a = -2.0 * kPi * (double)j / (double)len;
@@ -254,7 +254,7 @@ static int length_tables(int n, int m, int kind, DevBuf<float2>& tw, DevBuf<floa
     }
     SWEM_TRY(tw.upload(t.data(), t.size()));
     mr = MixedRadix{};
-    if (kind == kLenMixed && !mixed_radix_plan(n, &mr))
+    if (is_mixed(kind) && !mixed_radix_plan(n, &mr))
         return set_error(SWEM_EDEVICE, "no mixed-radix plan for n=%d", n);
     if (kind == kLenBluestein) {
         std::vector<float2> c, bc;

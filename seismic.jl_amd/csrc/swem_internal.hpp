@@ -42,8 +42,9 @@ void slowness_f32(const swem_geometry& g, const float* vel, float* po, float* pd
 constexpr int kMaxBlock = 1024;
 constexpr int kWaveBlock = 256;
 
-// Mixed-radix transform plan of a length n = 2^a 3^b 5^c <= 4096 (mixed_fft in swem_fft.hpp):
-// the radix of every pass in order (8 while 8 divides the rest, then 4, 2, 5, 3), the product of
+// Mixed-radix transform plan of a length n = 2^a 3^b 5^c <= 4096, or with factors 7, 11 and 13 too up
+// to 2048 (mixed_fft in swem_fft.hpp): the radix of every pass in order (the largest primes first,
+// then 8 while 8 divides the rest, 4, 2), the product of
 // the radices before it, its twiddle step n / (ns r) and the multiplier that divides by ns
 // (b / ns = umulhi(b, magic) for b ns < 2^32; 0 where ns = 1).
 constexpr int kMixedMaxPass = 12;
@@ -54,11 +55,16 @@ struct MixedRadix {
     uint32_t magic[kMixedMaxPass];
     uint8_t r[kMixedMaxPass];
 };
-// The plan of n (mr may be null); false when n is not 2^a 3^b 5^c or exceeds 4096.
+// The plan of n (mr may be null); false when n is no such length.
 bool mixed_radix_plan(int n, MixedRadix* mr);
 // How a transform of length n runs: a power-of-two kernel on n itself, Bluestein's identity on a
-// longer power-of-two array, or the mixed-radix transform on the next power of two.
-enum { kLenPow2 = 0, kLenBluestein = 1, kLenMixed = 2 };
+// longer power-of-two array, or the mixed-radix transform on the next power of two (kLenMixedPrime:
+// with a radix 7, 11 or 13; kernels of their own, since those butterflies hold up to 38 complex values
+// and cost the 2, 3, 5 lengths 20 to 48 registers, a third of their waves, when compiled beside them).
+enum { kLenPow2 = 0, kLenBluestein = 1, kLenMixed = 2, kLenMixedPrime = 3 };
+constexpr bool is_mixed(int kind) { return kind == kLenMixed || kind == kLenMixedPrime; }
+// kLenMixed or kLenMixedPrime of a length with a plan, else kLenBluestein.
+int mixed_kind(int n);
 
 // Arguments of the FP64 phase-table builders (swem_phase.hip).
 struct PhaseTableArgs {
@@ -169,7 +175,7 @@ struct March2DShape {
     int max_block;  // largest workgroup
     int bufs;       // LDS buffers per subgroup
     int blue;       // array length of a length that is not a power of two 128..4096 (0: nkx is one)
-    int mixed;      // that length runs the mixed-radix transform (else Bluestein's)
+    int mixed;      // that length runs the mixed-radix transform (2: with a radix 7, 11 or 13), 0: Bluestein's
 };
 March2DShape march2d_shape(int nkx, int variant, int adj);
 bool march2d_supported(int nkx);
@@ -177,7 +183,7 @@ bool march2d_supported(int nkx);
 // of two (at least 128) for mixed-radix lengths up to 4096, Bluestein's 2 nkx - 1 rounded up for
 // the others up to 2048 (0: a power-of-two kernel takes nkx, or nkx is out of range).
 int march2d_blue_len(int nkx);
-// kLenPow2, kLenBluestein or kLenMixed for a supported 2-D length.
+// kLenPow2, kLenBluestein, kLenMixed or kLenMixedPrime for a supported 2-D length.
 int march2d_kind(int nkx);
 size_t march2d_lds_bytes(int nkx, const March2DShape& sh, int F);
 
@@ -210,7 +216,7 @@ struct March3DArgs {
     const float2* twx;          // [march3d_len(nkx)] twiddles of the x array length; [nkx] of nkx
                                 // for a mixed-radix length
     const float2* twy;          // [march3d_len(nky)] (mixed radix: [nky])
-    MixedRadix mrx, mry;        // mixed-radix plans of nkx, nky (kLenMixed axes)
+    MixedRadix mrx, mry;        // mixed-radix plans of nkx, nky (mixed-radix axes)
     // Bluestein tables of an axis whose array length differs from its nk: [nk] chirp
     // exp(-i pi j^2 / nk), [2][array length] kernel spectra (transform sign -1, +1)
     const float2 *chx, *bchx, *chy, *bchy;

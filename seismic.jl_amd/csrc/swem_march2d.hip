@@ -34,14 +34,14 @@ int launch_ewem_len(int kind, const March2DArgs& ap, const March2DArgs& as, cons
 int march2d_kind(int nkx)
 {
     if (nkx >= 128 && !(nkx & (nkx - 1))) return kLenPow2;
-    return mixed_radix_plan(nkx, nullptr) ? kLenMixed : kLenBluestein;
+    return mixed_kind(nkx);
 }
 
 int march2d_blue_len(int nkx)
 {
     if (nkx < 1 || (nkx >= 128 && !(nkx & (nkx - 1)))) return 0;
     int m = 128;
-    if (march2d_kind(nkx) == kLenMixed) {
+    if (is_mixed(march2d_kind(nkx))) {
         while (m < nkx) m <<= 1;
         return m <= 4096 ? m : 0;
     }
@@ -55,7 +55,7 @@ March2DShape march2d_shape(int nkx, int variant, int adj)
     March2DShape sh{};
     if (const int m = march2d_blue_len(nkx)) {
         sh.blue = m;
-        sh.mixed = march2d_kind(nkx) == kLenMixed;
+        sh.mixed = march2d_kind(nkx) == kLenMixed ? 1 : march2d_kind(nkx) == kLenMixedPrime ? 2 : 0;
         sh.variant = adj ? SWEM_VARIANT_PAIR : SWEM_VARIANT_SUBGROUP;
         if (adj && variant == SWEM_VARIANT_PACKED) sh.variant = SWEM_VARIANT_PACKED;
         sh.T = m >= 1024 ? m / 8 : 64;
@@ -148,7 +148,7 @@ int angles_supported(int n) { return n >= 2 && (march2d_blue_len(n) || (n >= 128
 // The tables a launch needs for its transform length are present.
 static bool len_tables(const March2DArgs& a, int kind)
 {
-    return kind == kLenPow2 || (kind == kLenMixed ? a.mr.n == a.nkx : a.chirp && a.bchirp);
+    return kind == kLenPow2 || (is_mixed(kind) ? a.mr.n == a.nkx : a.chirp && a.bchirp);
 }
 
 int launch_angles(int which, const March2DArgs& ax, const March2DArgs& az, const AngleArgs& b, int F, hipStream_t st)

@@ -215,9 +215,9 @@ struct XBlue {
     }
 };
 
-// XMixed: a mixed-radix length n = nkx (2^a 3^b 5^c) in the power-of-two array of M >= n points,
+// XMixed: a mixed-radix length n = nkx (PRIME: with factors 7, 11, 13) in the power-of-two array of M >= n points,
 // transformed in the subgroup's two LDS buffers (mixed_fft); entries j >= n stay zero.
-template <int M, int P>
+template <int M, int P, bool PRIME = false>
 struct XMixed {
     XBlue<M, P> b;  // the kz row offsets
     __device__ __forceinline__ XMixed(const March2DArgs& a, int t) : b(a, t) {}
@@ -225,7 +225,7 @@ struct XMixed {
     __device__ __forceinline__ void fft(float2 (&v)[P], float2* lds, const March2DArgs& a, int t, int& pp) const
     {
         static_assert(!WAVE, "mixed-radix transforms use the subgroup buffers");
-        mixed_fft<M, P, SIGN, true>(v, lds, lds + LdsLen<M>::value, a.tw, a.mr, t, pp, []() { __syncthreads(); });
+        mixed_fft<M, P, SIGN, true, PRIME>(v, lds, lds + LdsLen<M>::value, a.tw, a.mr, t, pp, []() { __syncthreads(); });
     }
     __device__ __forceinline__ void kload_row(float2 (&L)[P], const float2* __restrict__ row, const March2DArgs& a, int t) const
     {
@@ -1125,10 +1125,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void ma
 
 // Packed compat migration of a mixed-radix or Bluestein nkx on the array length M (the subgroup
 // shape of the other non-power-of-two kernels: M / 8 threads from M = 1024, one wave below).
-template <int M, int P, bool HALF>
+template <int M, int P, bool HALF, bool PRIME>
 __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_packed_mixed(March2DArgs a)
 {
-    adj_body_packed<M, P, false, HALF, XMixed<M, P>>(a);
+    adj_body_packed<M, P, false, HALF, XMixed<M, P, PRIME>>(a);
 }
 template <int M, int P, bool HALF>
 __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_packed_blue(March2DArgs a)
@@ -1186,16 +1186,16 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void m
     fwd_body<M, P, MODE, false, true, XBlue<M, P>>(a);
 }
 
-template <int M, int MODE, int P, bool HALF>
+template <int M, int MODE, int P, bool HALF, bool PRIME>
 __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_mixed(March2DArgs a)
 {
-    adj_body_pair<M, P, MODE, false, HALF, XMixed<M, P>>(a);
+    adj_body_pair<M, P, MODE, false, HALF, XMixed<M, P, PRIME>>(a);
 }
 
-template <int M, int MODE, int P, bool HALF>
+template <int M, int MODE, int P, bool HALF, bool PRIME>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_mixed(March2DArgs a)
 {
-    fwd_body<M, P, MODE, false, HALF, XMixed<M, P>>(a);
+    fwd_body<M, P, MODE, false, HALF, XMixed<M, P, PRIME>>(a);
 }
 
 // ------------------------------------------------------------------ launches of one array length
@@ -1256,23 +1256,30 @@ static int launch_blue_mode(const March2DArgs& a, const March2DShape& sh, int F,
     constexpr int P = M >= 1024 ? 8 : M / 64;
     const size_t lds = march2d_lds_bytes(a.nkx, sh, F);
     dim3 block(sh.T * sh.per_freq * F);
-    if constexpr (MODE == kModePspiCompat) {
-        if (adj && sh.variant == SWEM_VARIANT_PACKED) {
-            const size_t lds_p = lds + kPackedScratch * sizeof(float2);
-            if (sh.mixed)
-                return 2 * a.nmx <= M ? launch_kernel(march2d_adj_packed_mixed<M, P, true>, a, block, lds_p, st)
-                                      : launch_kernel(march2d_adj_packed_mixed<M, P, false>, a, block, lds_p, st);
-            // Bluestein: M >= 2 nkx - 1 >= 2 nmx - 1, and M even, so the upper half is always zero
-            return launch_kernel(march2d_adj_packed_blue<M, P, true>, a, block, lds_p, st);
+    const bool half = 2 * a.nmx <= M;
+    // one launch of the mixed-radix kernels with or without the radices 7, 11, 13 (lengths up to 2048)
+    auto mixed = [&](auto prime) {
+        constexpr bool PR = decltype(prime)::value;
+        if constexpr (MODE == kModePspiCompat) {
+            if (adj && sh.variant == SWEM_VARIANT_PACKED) {
+                const size_t lds_p = lds + kPackedScratch * sizeof(float2);
+                return launch_kernel(half ? march2d_adj_packed_mixed<M, P, true, PR> : march2d_adj_packed_mixed<M, P, false, PR>, a,
+                                     block, lds_p, st);
+            }
         }
-    }
-    if (sh.mixed) {
-        if (2 * a.nmx <= M)
-            return adj ? launch_kernel(march2d_adj_mixed<M, MODE, P, true>, a, block, lds, st)
-                       : launch_kernel(march2d_fwd_mixed<M, MODE, P, true>, a, block, lds, st);
-        return adj ? launch_kernel(march2d_adj_mixed<M, MODE, P, false>, a, block, lds, st)
-                   : launch_kernel(march2d_fwd_mixed<M, MODE, P, false>, a, block, lds, st);
-    }
+        if (adj)
+            return launch_kernel(half ? march2d_adj_mixed<M, MODE, P, true, PR> : march2d_adj_mixed<M, MODE, P, false, PR>, a, block,
+                                 lds, st);
+        return launch_kernel(half ? march2d_fwd_mixed<M, MODE, P, true, PR> : march2d_fwd_mixed<M, MODE, P, false, PR>, a, block, lds,
+                             st);
+    };
+    if (sh.mixed == 1) return mixed(std::false_type{});
+    if constexpr (M <= 2048)
+        if (sh.mixed == 2) return mixed(std::true_type{});
+    if constexpr (MODE == kModePspiCompat)
+        if (adj && sh.variant == SWEM_VARIANT_PACKED)
+            // Bluestein: M >= 2 nkx - 1 >= 2 nmx - 1, and M even, so the upper half is always zero
+            return launch_kernel(march2d_adj_packed_blue<M, P, true>, a, block, lds + kPackedScratch * sizeof(float2), st);
     return adj ? launch_kernel(march2d_adj_blue<M, MODE, P>, a, block, lds, st)
                : launch_kernel(march2d_fwd_blue<M, MODE, P>, a, block, lds, st);
 }
@@ -1487,6 +1494,8 @@ int launch_angles_len(int which, int kind, const March2DArgs& ax, const March2DA
 {
     constexpr int P = N >= 1024 ? 8 : N / 64;
     if (kind == kLenMixed) return launch_angles_n<N, XMixed<N, P>>(which, ax, az, b, F, st);
+    if constexpr (N <= 2048)
+        if (kind == kLenMixedPrime) return launch_angles_n<N, XMixed<N, P, true>>(which, ax, az, b, F, st);
     return kind == kLenBluestein ? launch_angles_n<N, XBlue<N, P>>(which, ax, az, b, F, st)
                                  : launch_angles_n<N, XPow2<N, P>>(which, ax, az, b, F, st);
 }
@@ -1669,6 +1678,8 @@ int launch_ewem_len(int kind, const March2DArgs& ap, const March2DArgs& as, cons
 {
     constexpr int P = N >= 1024 ? 8 : N / 64;
     if (kind == kLenMixed) return launch_ewem_n<N, XMixed<N, P>>(ap, as, e, adj, st);
+    if constexpr (N <= 2048)
+        if (kind == kLenMixedPrime) return launch_ewem_n<N, XMixed<N, P, true>>(ap, as, e, adj, st);
     return kind == kLenBluestein ? launch_ewem_n<N, XBlue<N, P>>(ap, as, e, adj, st)
                                  : launch_ewem_n<N, XPow2<N, P>>(ap, as, e, adj, st);
 }

@@ -11,13 +11,13 @@ int launch_ewem3d_n(int which, const March3DArgs& ap, const March3DArgs& as, con
 template <int N, int BL>
 int launch3_n(int which, const March3DArgs& a, int F, int phase, hipStream_t st);
 
-// Array length of a 3-D line transform of n points: n for powers of two 128..1024, else the
-// Bluestein length (the power of two >= max(128, 2n - 1), up to 1024: n <= 512; n = 1 is the
+// Array length of a 3-D line transform of n points: n for powers of two 128..1024, the next power of two
+// for mixed-radix lengths (2, 3, 5 up to 1024; with factors 7, 11, 13 up to 512), else the Bluestein length (the power of two >= max(128, 2n - 1), up to 1024: n <= 512; n = 1 is the
 // nkx of a single inline, nmx = 1); 0 if neither.
 int march3d_kind(int n)
 {
     if (n >= 128 && !(n & (n - 1))) return kLenPow2;
-    return mixed_radix_plan(n, nullptr) ? kLenMixed : kLenBluestein;
+    return mixed_kind(n);
 }
 
 int march3d_len(int n)
@@ -26,7 +26,8 @@ int march3d_len(int n)
     const int kind = march3d_kind(n);
     if (kind == kLenPow2) return n <= 1024 ? n : 0;
     int m = 128;
-    if (kind == kLenMixed) {
+    if (is_mixed(kind)) {
+        if (kind == kLenMixedPrime && n > 512) return 0;
         while (m < n) m <<= 1;
         return m <= 1024 ? m : 0;
     }
@@ -50,7 +51,7 @@ int launch_ewem3d(int which, const March3DArgs& ap, const March3DArgs& as, const
         return set_error(SWEM_EINVAL, "3-D ewem: %d frequencies per workgroup (1..8)", F);
     const int kind = march3d_kind(n);
     if ((kind == kLenBluestein && (xpass ? !(ap.chx && ap.bchx) : !(ap.chy && ap.bchy))) ||
-        (kind == kLenMixed && (xpass ? ap.mrx.n : ap.mry.n) != n))
+        (is_mixed(kind) && (xpass ? ap.mrx.n : ap.mry.n) != n))
         return set_error(SWEM_EINVAL, "3-D ewem: transform tables missing (n=%d)", n);
     switch (kind * 16 + m / 128) {
 #define SWEM_E3(M, K) \
@@ -58,6 +59,7 @@ int launch_ewem3d(int which, const March3DArgs& ap, const March3DArgs& as, const
         SWEM_E3(128, 0) SWEM_E3(256, 0) SWEM_E3(512, 0) SWEM_E3(1024, 0)
         SWEM_E3(128, 1) SWEM_E3(256, 1) SWEM_E3(512, 1) SWEM_E3(1024, 1)
         SWEM_E3(128, 2) SWEM_E3(256, 2) SWEM_E3(512, 2) SWEM_E3(1024, 2)
+        SWEM_E3(128, 3) SWEM_E3(256, 3) SWEM_E3(512, 3)
 #undef SWEM_E3
     }
     return set_error(SWEM_EUNSUPPORTED, "3-D ewem: n=%d", n);
@@ -72,7 +74,7 @@ int launch_march3d(int which, const March3DArgs& a, int F, int phase, hipStream_
     const int kind = march3d_kind(n);
     if (kind == kLenBluestein && (xpass ? !(a.chx && a.bchx) : !(a.chy && a.bchy)))
         return set_error(SWEM_EINVAL, "3-D march: Bluestein tables missing (n=%d)", n);
-    if (kind == kLenMixed && (xpass ? a.mrx.n : a.mry.n) != n)
+    if (is_mixed(kind) && (xpass ? a.mrx.n : a.mry.n) != n)
         return set_error(SWEM_EINVAL, "3-D march: mixed-radix plan missing (n=%d)", n);
     // y-passes: up to 16 frequencies per workgroup (8 on a Bluestein y axis, whose kernels are
     // compiled for 512 threads to keep their longer transforms in registers; 8 for PSPI)
@@ -89,6 +91,7 @@ int launch_march3d(int which, const March3DArgs& a, int F, int phase, hipStream_
         SWEM_M3(128, 0) SWEM_M3(256, 0) SWEM_M3(512, 0) SWEM_M3(1024, 0)
         SWEM_M3(128, 1) SWEM_M3(256, 1) SWEM_M3(512, 1) SWEM_M3(1024, 1)
         SWEM_M3(128, 2) SWEM_M3(256, 2) SWEM_M3(512, 2) SWEM_M3(1024, 2)
+        SWEM_M3(128, 3) SWEM_M3(256, 3) SWEM_M3(512, 3)
 #undef SWEM_M3
     }
     return set_error(SWEM_EUNSUPPORTED, "3-D march: n=%d", n);

@@ -145,7 +145,7 @@ __device__ __forceinline__ bool yin(const March3DArgs& a, int i)
 }
 
 // Transform of one line of n points held by G lanes as N array points (lane t, slot q: point
-// t + G q).  KIND kLenPow2: n = N, the wave FFT.  kLenMixed: n = 2^a 3^b 5^c <= N, the
+// t + G q).  KIND kLenPow2: n = N, the wave FFT.  kLenMixed, kLenMixedPrime: the
 // mixed-radix transform in the wave's LDS buffer (tw: [n] of n).  kLenBluestein: Bluestein's
 // chirp-z identity on the power-of-two array length N >= 2n - 1, X_k = c_k IFFT_N(FFT_N(c x) B)_k
 // with the chirp c_j = exp(SIGN i pi j^2 / n) and B the spectrum of the wrapped conjugate chirp
@@ -158,9 +158,9 @@ __device__ __forceinline__ void line_fft(LinePoints<N, KIND>& v, float2* buf, co
     constexpr int G = Line<N, KIND>::G, P = Line<N, KIND>::P;
     if constexpr (KIND == kLenPow2) {
         wfft<N, SIGN, kSeedAhead, false, G>(v, buf, tw, t);
-    } else if constexpr (KIND == kLenMixed) {
+    } else if constexpr (is_mixed(KIND)) {
         int pp = 0;
-        mixed_fft<N, P, SIGN, false>(v, buf, buf, tw, mr, t, pp, []() { wave_sync_lds(); });
+        mixed_fft<N, P, SIGN, false, KIND == kLenMixedPrime>(v, buf, buf, tw, mr, t, pp, []() { wave_sync_lds(); });
     } else {
         auto chirp_mul = [&]() {
             float2 c[P];
