@@ -461,8 +461,8 @@ static void choose_chunks(swem_plan* p)
     const size_t per = table_bytes_per_freq(p);
     size_t cap = p->opt.table_bytes;
     if (!cap) {
-        size_t fr = 0, tot = 0;
-        cap = hipMemGetInfo(&fr, &tot) == hipSuccess ? std::min((size_t)32 << 30, fr / 4) : (size_t)8 << 30;
+        const size_t fr = device_free_bytes();
+        cap = fr ? std::min((size_t)32 << 30, fr / 4) : (size_t)8 << 30;
     }
     int nfc = (int)std::min<size_t>(p->nf, cap / per);
     if (nfc < p->nf) nfc = std::max(p->F, std::max(p->Ffwd, (nfc / (p->F * p->Ffwd)) * p->F * p->Ffwd));
@@ -481,9 +481,8 @@ static int alloc_tables(swem_plan* p)
 
 static size_t default_budget()
 {
-    size_t fr = 0, tot = 0;
-    if (hipMemGetInfo(&fr, &tot) != hipSuccess) return (size_t)8 << 30;
-    return std::min((size_t)96 << 30, fr / 2);
+    const size_t fr = device_free_bytes();
+    return fr ? std::min((size_t)96 << 30, fr / 2) : (size_t)8 << 30;
 }
 
 static int plan_events(swem_plan* p, int n)
@@ -516,7 +515,8 @@ static int set_igx(swem_plan* p, const float* sx, const float* sy, int nshot, hi
         p->igx_host[i] = ix * p->g.nmy + iy;
     }
     SWEM_TRY(p->igx.alloc(nshot));
-    if (p->served) return upload_bytes(p->igx.p, p->igx_host.data(), sizeof(int) * nshot);
+    // (a one-call plan would pin and unpin its own copy)
+    if (p->served || tl_dev_alloc) return upload_bytes(p->igx.p, p->igx_host.data(), sizeof(int) * nshot);
     if (p->igx_cap < nshot) {
         if (p->igx_pinned) (void)hipHostFree(p->igx_pinned);
         p->igx_pinned = nullptr;
@@ -1203,6 +1203,8 @@ int swem_plan_create(const swem_geometry* g, const float* vel, const float* wav,
 {
     if (!g || !vel || !wav || !out) return set_error(SWEM_EINVAL, "plan_create: null argument");
     *out = nullptr;
+    // a plan that outlives the call sizes itself by the free memory: nothing stays kept beside it
+    if (!tl_dev_alloc) trim_call_memory(opt ? opt->device : 0);
     swem_plan* p = new swem_plan();
     int rc = plan_setup(p, g, vel, opt);
     if (!rc) rc = plan_build(p, wav);
@@ -1548,36 +1550,31 @@ int swem_shots(const swem_geometry* g, const float* vel, const float* wav, const
                float* d, float* m, int adj, const swem_options* opt)
 {
     if (!g || !vel || !wav || !sx || !d || !m || nshot < 1) return set_error(SWEM_EINVAL, "shots: null argument");
+    CallMemory memory(opt ? opt->device : 0);
     swem_plan* p = nullptr;
     SWEM_TRY(swem_plan_create(g, vel, wav, opt, &p));
-    const size_t nm = (size_t)g->nmx * g->nmy, dbytes = (size_t)nshot * nm * g->nt * sizeof(float),
-                 mbytes = nm * g->nz * sizeof(float);
-    float *dd = nullptr, *dm = nullptr;
-    int rc = SWEM_OK;
-    hipError_t e = hipMalloc((void**)&dd, dbytes);
-    if (e == hipSuccess) e = hipMalloc((void**)&dm, mbytes);
-    if (e != hipSuccess) rc = hip_error(e, "hipMalloc", __FILE__, __LINE__);
-    if (!rc) {
+    const size_t nm = (size_t)g->nmx * g->nmy, nd = (size_t)nshot * nm * g->nt, nmz = nm * g->nz;
+    int rc;
+    {
+        DevBuf<float> dd, dm;
+        rc = dd.alloc(nd);
+        if (!rc) rc = dm.alloc(nmz);
+        auto down = [&](float* host, const float* dev, size_t n) {
+            const hipError_t e = hipMemcpy(host, dev, n * sizeof(float), hipMemcpyDeviceToHost);
+            return e == hipSuccess ? SWEM_OK : hip_error(e, "hipMemcpy", __FILE__, __LINE__);
+        };
         if (adj) {
-            e = hipMemcpy(dd, d, dbytes, hipMemcpyHostToDevice);
-            if (e != hipSuccess) rc = hip_error(e, "hipMemcpy", __FILE__, __LINE__);
-            if (!rc) rc = swem_plan_migrate(p, dd, sx, sy, nshot, dm, 0, nullptr);
-            if (!rc) {
-                e = hipMemcpy(m, dm, mbytes, hipMemcpyDeviceToHost);
-                if (e != hipSuccess) rc = hip_error(e, "hipMemcpy", __FILE__, __LINE__);
-            }
+            if (!rc) rc = upload_bytes(dd.p, d, nd * sizeof(float));
+            if (!rc) rc = swem_plan_migrate(p, dd.p, sx, sy, nshot, dm.p, 0, nullptr);
+            if (!rc) rc = down(m, dm.p, nmz);
         } else {
-            e = hipMemcpy(dm, m, mbytes, hipMemcpyHostToDevice);
-            if (e != hipSuccess) rc = hip_error(e, "hipMemcpy", __FILE__, __LINE__);
-            if (!rc) rc = swem_plan_model(p, dm, sx, sy, nshot, dd, nullptr);
-            if (!rc) {
-                e = hipMemcpy(d, dd, dbytes, hipMemcpyDeviceToHost);
-                if (e != hipSuccess) rc = hip_error(e, "hipMemcpy", __FILE__, __LINE__);
-            }
+            if (!rc) rc = upload_bytes(dm.p, m, nmz * sizeof(float));
+            if (!rc) rc = swem_plan_model(p, dm.p, sx, sy, nshot, dd.p, nullptr);
+            if (!rc) rc = down(d, dd.p, nd);
         }
+        dd.release();
+        dm.release();
     }
-    if (dd) (void)hipFree(dd);
-    if (dm) (void)hipFree(dm);
     swem_plan_destroy(p);
     return rc;
 }
@@ -1816,6 +1813,7 @@ int swem_compute_angles_ex(float* angx, float* angy, const float* wav, const swe
     swem_options o;
     if (opt) o = *opt;
     else swem_options_init(&o);
+    CallMemory memory(o.device);
     swem_plan* p = nullptr;
     SWEM_TRY(swem_plan_create(&ga, vel, wav, &o, &p));
     const int rc = angles_impl(p, sx, sy, angx, angy);
@@ -2213,6 +2211,7 @@ int swem_eshots(const swem_geometry* g, const float* vp, const float* vs, const 
     swem_options o;
     if (opt) o = *opt;
     else swem_options_init(&o);
+    CallMemory memory(o.device);
     swem_plan *pp = nullptr, *ps = nullptr;
     // both plans sample the band as ewem.c does (ewem.c:43-52)
     SWEM_TRY(plan_create_rule(&ge, vp, wav, &o, 1, &pp));
@@ -2246,7 +2245,14 @@ int swem_ewem(float* ux, float* uy, float* uz, float* mpp, float* mps1, float* m
 int swem_malloc(void** ptr, size_t bytes)
 {
     if (!ptr) return set_error(SWEM_EINVAL, "null pointer");
-    SWEM_HIP(hipMalloc(ptr, bytes));
+    hipError_t e = hipMalloc(ptr, bytes);
+    if (e == hipErrorOutOfMemory) {  // what the one-call entry points keep is given back first
+        (void)hipGetLastError();
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess) trim_call_memory(dev);
+        e = hipMalloc(ptr, bytes);
+    }
+    if (e != hipSuccess) return hip_error(e, "hipMalloc(ptr, bytes)", __FILE__, __LINE__);
     return SWEM_OK;
 }
 

@@ -10,10 +10,13 @@
 namespace swem {
 
 // Device memory source of DevBuf.  A thread that installs one (the serving loop's worker, for
-// the requests it admits) gets every plan allocation from it; otherwise hipMalloc / hipFree.
+// the requests it admits; CallMemory for the one-call entry points) gets every plan allocation from
+// it; otherwise hipMalloc / hipFree.
 struct DevAllocator {
     virtual void* alloc(size_t bytes) = 0;
     virtual void release(void* p, size_t bytes) = 0;
+    virtual size_t spare() const { return 0; }  // bytes it holds beyond what the device reports free
+    virtual const char* name() const { return "request memory block exhausted"; }
     virtual ~DevAllocator() = default;
 };
 // Host -> device copies of plan tables.  Installed by the serving loop: copies go through
@@ -22,6 +25,32 @@ struct HostStager {
     virtual int put(void* dev, const void* host, size_t bytes) = 0;
     virtual ~HostStager() = default;
 };
+// Memory of one call of a one-call entry point (swem_pool.cpp): while it lives, the thread's plan
+// allocations come from blocks kept between calls, and go back to them when it ends.
+struct CallMemory : DevAllocator {
+    explicit CallMemory(int device);
+    ~CallMemory() override;
+    void* alloc(size_t bytes) override;
+    void release(void* p, size_t bytes) override;
+    size_t spare() const override;
+    const char* name() const override { return "out of device memory"; }
+    CallMemory(const CallMemory&) = delete;
+    CallMemory& operator=(const CallMemory&) = delete;
+
+private:
+    struct Held {
+        void* p;
+        size_t n;
+        bool taken;
+    };
+    std::vector<Held> blocks;
+    int dev;
+    bool on = false;
+};
+// Frees the blocks kept for a device.
+void trim_call_memory(int dev);
+// Free device memory for a budget (0: unknown), kept blocks included inside a call that can take them.
+size_t device_free_bytes();
 extern thread_local DevAllocator* tl_dev_alloc;
 extern thread_local HostStager* tl_stager;
 
@@ -39,7 +68,7 @@ struct DevBuf {
         if (count == 0) return SWEM_OK;
         if (tl_dev_alloc) {
             p = static_cast<T*>(tl_dev_alloc->alloc(count * sizeof(T)));
-            if (!p) return set_error(SWEM_ENOMEM, "request memory block exhausted (%zu bytes more)", count * sizeof(T));
+            if (!p) return set_error(SWEM_ENOMEM, "%s (%zu bytes more)", tl_dev_alloc->name(), count * sizeof(T));
             from = tl_dev_alloc;
         } else {
             SWEM_HIP(hipMalloc((void**)&p, count * sizeof(T)));

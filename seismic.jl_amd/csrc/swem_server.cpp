@@ -614,6 +614,7 @@ int swem_server_create(const swem_server_config* cfg, swem_server** out)
     if (hipGetDeviceCount(&count) != hipSuccess || c.device < 0 || c.device >= count)
         return set_error(SWEM_EDEVICE, "server: device %d not available", c.device);
     SWEM_HIP(hipSetDevice(c.device));
+    trim_call_memory(c.device);
     if (!c.device_bytes) {
         size_t fr = 0, tot = 0;
         SWEM_HIP(hipMemGetInfo(&fr, &tot));
