@@ -1,4 +1,4 @@
-// swem_util.hip -- band-limited time<->frequency transforms (as a tiled SGEMM against an FP64-built
+// swem_util.hip -- band-limited time<->frequency transforms (as a matrix product with an FP64-built
 // Fourier basis), the compensated image reduction and a transpose.
 //
 // The reference transforms every trace with an r2c / c2r FFT of length (nw-1)*2 and keeps the
@@ -13,57 +13,144 @@
 
 namespace swem {
 
-// 64x64 output tile per 256-thread workgroup, 4x4 per thread, K tile 16.
-__global__ __launch_bounds__(256) void sgemm_nn(int M, int Nc, int K, const float* __restrict__ A, int lda,
-                                                const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc)
+// C = A B on the FP32 matrix cores (v_mfma_f32_32x32x2_f32), row-major, in two tilings with one
+// summation order, so that a row's result does not depend on how many rows share the launch (a shot's
+// spectra, hence its image, are the same in any batch): K is cut into segments of gemm_segment(K), a
+// segment is accumulated in k order by groups of eight (the four products of a group take its pairs
+// k + j and k + 4 + j), and the segment sums are added in order.
+//   gemm_tile   128 x 128 outputs per workgroup, four waves of 64 x 64, K tiles of 16 through LDS, the
+//               next tile's loads in flight during a tile.  For launches that fill the chip: 64 K rows,
+//               1130 columns, K 1500 ran 3.2 ms with 4 x 4 FP32 FMAs per thread.
+//   gemm_split  32 x 32 outputs per workgroup, one wave per segment straight from memory, the segment sums
+//               meeting in LDS.  For the others: one shot's 128 traces (30 tiles of 64 x 64) waited 200 us
+//               for a serial loop over K.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+constexpr int kGemmSegs = 16;
+
+static inline int gemm_segment(int K) { return std::max(128, ((K + kGemmSegs - 1) / kGemmSegs + 15) / 16 * 16); }
+
+// Row of a 32 x 32 accumulator's register r in lane half h; its column is lane mod 32.
+__device__ __forceinline__ int acc_row(int r, int h) { return (r >> 2) * 8 + h * 4 + (r & 3); }
+
+__global__ __launch_bounds__(256) void gemm_tile(int M, int Nc, int K, int seg, const float* __restrict__ A, int lda,
+                                                 const float* __restrict__ B, int ldb, float* __restrict__ C, int ldc)
 {
-    __shared__ float As[16][64 + 4];
-    __shared__ float Bs[16][64 + 4];
-    const int tid = threadIdx.x;
-    const int tx = tid & 15, ty = tid >> 4;
-    const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-    float acc[4][4];
+    constexpr int LD = 128 + 4;
+    __shared__ float As[16][LD];
+    __shared__ float Bs[16][LD];
+    const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l = lane & 31;
+    const int m0 = blockIdx.y * 128, n0 = blockIdx.x * 128;
+    const int wm = (tid >> 7) * 64, wn = ((tid >> 6) & 1) * 64;
+    // A: thread loads 8 consecutive k of row tid / 2; B: 8 consecutive columns of row tid / 16
+    const int am = tid >> 1, ak = (tid & 1) * 8, bk = tid >> 4, bn = (tid & 15) * 8;
+    const float* Ar = A + (size_t)(m0 + am) * lda;
+    float ra[8], rb[8];
+    auto fetch = [&](int k0) {
+        const bool arow = m0 + am < M, brow = k0 + bk < K;
+        const float* Br = B + (size_t)(k0 + bk) * ldb;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) ra[i] = arow && k0 + ak + i < K ? Ar[k0 + ak + i] : 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) rb[i] = brow && n0 + bn + i < Nc ? Br[n0 + bn + i] : 0.f;
+    };
+    f32x16 sum[2][2], acc[2][2];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+        for (int r = 0; r < 16; ++r) sum[i >> 1][i & 1][r] = acc[i >> 1][i & 1][r] = 0.f;
+    fetch(0);
     for (int k0 = 0; k0 < K; k0 += 16) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + i * 256;
-            const int mm = idx >> 4, kk = idx & 15;
-            As[kk][mm] = (m0 + mm < M && k0 + kk < K) ? A[(size_t)(m0 + mm) * lda + k0 + kk] : 0.f;
-        }
+        for (int i = 0; i < 8; ++i) As[ak + i][am] = ra[i];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + i * 256;
-            const int kk = idx >> 6, nn = idx & 63;
-            Bs[kk][nn] = (k0 + kk < K && n0 + nn < Nc) ? B[(size_t)(k0 + kk) * ldb + n0 + nn] : 0.f;
-        }
+        for (int i = 0; i < 8; ++i) Bs[bk][bn + i] = rb[i];
         __syncthreads();
+        if (k0 + 16 < K) fetch(k0 + 16);
 #pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            float av[4], bv[4];
+        for (int g = 0; g < 16; g += 8)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) av[i] = As[kk][ty + 16 * i];
+            for (int j = 0; j < 4; ++j) {
+                const int kk = g + j + 4 * h;
+                float av[2], bv[2];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) bv[j] = Bs[kk][tx + 16 * j];
+                for (int i = 0; i < 2; ++i) {
+                    av[i] = As[kk][wm + 32 * i + l];
+                    bv[i] = Bs[kk][wn + 32 * i + l];
+                }
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                for (int a = 0; a < 2; ++a)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(av[i], bv[j], acc[i][j]);
-        }
+                    for (int b = 0; b < 2; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+            }
         __syncthreads();
+        if ((k0 + 16) % seg == 0 || k0 + 16 >= K) {  // end of a segment
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        sum[a][b][r] += acc[a][b][r];
+                        acc[a][b][r] = 0.f;
+                    }
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int m = m0 + ty + 16 * i;
-        if (m >= M) continue;
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+            const int n = n0 + wn + 32 * b + l;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int m = m0 + wm + 32 * a + acc_row(r, h);
+                if (m < M && n < Nc) C[(size_t)m * ldc + n] = sum[a][b][r];
+            }
+        }
+}
+
+__global__ __launch_bounds__(64 * kGemmSegs) void gemm_split(int M, int Nc, int K, int seg, const float* __restrict__ A,
+                                                             int lda, const float* __restrict__ B, int ldb,
+                                                             float* __restrict__ C, int ldc)
+{
+    extern __shared__ float part[];  // [segments][32][32]
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, l = lane & 31;
+    const int m = blockIdx.y * 32 + l, n = blockIdx.x * 32 + l;
+    const int k1 = min(K, (w + 1) * seg);
+    const float* Ar = A + (size_t)min(m, M - 1) * lda;  // rows and columns beyond the matrix: read, not stored
+    const float* Bc = B + min(n, Nc - 1);
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+    int k = w * seg;
+#pragma unroll 4
+    for (; k + 8 <= k1; k += 8) {
+        float av[4], bv[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
-            const int n = n0 + tx + 16 * j;
-            if (n < Nc) C[(size_t)m * ldc + n] = acc[i][j];
+            av[j] = Ar[k + 4 * h + j];
+            bv[j] = Bc[(size_t)(k + 4 * h + j) * ldb];
         }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av[j], bv[j], acc, 0, 0, 0);
+    }
+    if (k < k1) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int kk = k + 4 * h + j;
+            const float av = kk < k1 ? Ar[kk] : 0.f, bv = kk < k1 ? Bc[(size_t)kk * ldb] : 0.f;
+            acc = __builtin_amdgcn_mfma_f32_32x32x2f32(av, bv, acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) part[w * 1024 + acc_row(r, h) * 32 + l] = acc[r];
+    __syncthreads();
+    const int nseg = blockDim.x >> 6;
+    for (int i = threadIdx.x; i < 1024; i += blockDim.x) {
+        float sum = 0.f;
+        for (int s = 0; s < nseg; ++s) sum += part[s * 1024 + i];
+        const int mm = blockIdx.y * 32 + (i >> 5), nn = blockIdx.x * 32 + (i & 31);
+        if (mm < M && nn < Nc) C[(size_t)mm * ldc + nn] = sum;
     }
 }
 
@@ -71,9 +158,18 @@ int launch_sgemm(int M, int Nc, int K, const float* A, int lda, const float* B, 
                  hipStream_t st)
 {
     if (M <= 0 || Nc <= 0 || K <= 0) return SWEM_OK;
-    if ((Nc + 63) / 64 > 65535 * 16 || (M + 63) / 64 > 65535) return set_error(SWEM_EINVAL, "sgemm: %d x %d too large", M, Nc);
-    dim3 grid((Nc + 63) / 64, (M + 63) / 64), block(256);
-    hipLaunchKernelGGL(sgemm_nn, grid, block, 0, st, M, Nc, K, A, lda, B, ldb, C, ldc);
+    const int seg = gemm_segment(K);
+    const long long tiles = ((Nc + 127) / 128) * (long long)((M + 127) / 128);
+    if ((Nc + 127) / 128 > 65535 * 16 || (M + 127) / 128 > 65535) return set_error(SWEM_EINVAL, "sgemm: %d x %d too large", M, Nc);
+    // one workgroup of gemm_tile per compute unit at least; below, the 32 x 32 tiles
+    if (tiles >= 256 || (M + 31) / 32 > 65535) {
+        hipLaunchKernelGGL(gemm_tile, dim3((Nc + 127) / 128, (M + 127) / 128), dim3(256), 0, st, M, Nc, K, seg, A, lda, B, ldb, C,
+                           ldc);
+    } else {
+        const int nseg = (K + seg - 1) / seg;
+        hipLaunchKernelGGL(gemm_split, dim3((Nc + 31) / 32, (M + 31) / 32), dim3(64 * nseg), nseg * 1024 * sizeof(float), st, M,
+                           Nc, K, seg, A, lda, B, ldb, C, ldc);
+    }
     SWEM_HIP(hipGetLastError());
     return SWEM_OK;
 }
