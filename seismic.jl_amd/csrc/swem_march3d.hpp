@@ -150,14 +150,15 @@ __device__ __forceinline__ bool yin(const March3DArgs& a, int i)
 // chirp-z identity on the power-of-two array length N >= 2n - 1, X_k = c_k IFFT_N(FFT_N(c x) B)_k
 // with the chirp c_j = exp(SIGN i pi j^2 / n) and B the spectrum of the wrapped conjugate chirp
 // over N, built in FP64 on the host (c = 0 for j >= n, so points beyond n enter and leave as zero).
-template <int N, int SIGN, int KIND>
+// HIN (power-of-two lengths): the upper half of the line is zero and is not read.
+template <int N, int SIGN, int KIND, bool HIN = false>
 __device__ __forceinline__ void line_fft(LinePoints<N, KIND>& v, float2* buf, const float2* __restrict__ tw,
                                          const float2* __restrict__ chirp, const float2* __restrict__ bch,
                                          const MixedRadix& mr, int n, int t)
 {
     constexpr int G = Line<N, KIND>::G, P = Line<N, KIND>::P;
     if constexpr (KIND == kLenPow2) {
-        wfft<N, SIGN, kSeedAhead, false, G>(v, buf, tw, t);
+        wfft<N, SIGN, kSeedAhead, HIN, G>(v, buf, tw, t);
     } else if constexpr (is_mixed(KIND)) {
         int pp = 0;
         mixed_fft<N, P, SIGN, false, KIND == kLenMixedPrime>(v, buf, buf, tw, mr, t, pp, []() { wave_sync_lds(); });
@@ -187,16 +188,16 @@ __device__ __forceinline__ void line_fft(LinePoints<N, KIND>& v, float2* buf, co
     }
 }
 
-template <int N, int SIGN, int BX>
+template <int N, int SIGN, int BX, bool HIN = false>
 __device__ __forceinline__ void xfft(LinePoints<N, BX>& v, float2* buf, const March3DArgs& a, int t)
 {
-    line_fft<N, SIGN, BX>(v, buf, a.twx, a.chx, a.bchx, a.mrx, a.nkx, t);
+    line_fft<N, SIGN, BX, HIN>(v, buf, a.twx, a.chx, a.bchx, a.mrx, a.nkx, t);
 }
 
-template <int N, int SIGN, int BY>
+template <int N, int SIGN, int BY, bool HIN = false>
 __device__ __forceinline__ void yfft(LinePoints<N, BY>& v, float2* buf, const March3DArgs& a, int t)
 {
-    line_fft<N, SIGN, BY>(v, buf, a.twy, a.chy, a.bchy, a.mry, a.nky, t);
+    line_fft<N, SIGN, BY, HIN>(v, buf, a.twy, a.chy, a.bchy, a.mry, a.nky, t);
 }
 
 }  // namespace
@@ -267,30 +268,31 @@ __device__ __forceinline__ void kz_phases64_col(const March3DArgs& a, double c0,
 // Staging of an x-pass workgroup's tile of C columns through LDS: thread (x0, c) = (threadIdx / C,
 // threadIdx mod C) moves the rows x0 + G j of column c, so global accesses are row segments of C
 // complex.  A line of fewer than 64 lanes stages its two wavefields in turn through one buffer per
-// column (ONE): with both in LDS at once it would hold half the waves per compute unit.
-template <int P, int G>
-__device__ __forceinline__ void tile_load(float2 (&st)[P], const float2* src, const March3DArgs& a, int x0, bool in)
+// column (ONE): with both in LDS at once it would hold half the waves per compute unit.  Q: the rows that
+// can hold x < nmx (P / 2 where 2 nmx <= N).
+template <int P, int G, int Q = P>
+__device__ __forceinline__ void tile_load(float2 (&st)[Q], const float2* src, const March3DArgs& a, int x0, bool in)
 {
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
+    for (int j = 0; j < Q; ++j) {
         const int x = x0 + G * j;
         st[j] = x < a.nmx && in ? src[(size_t)x * a.nky] : make_float2(0.f, 0.f);
     }
 }
-template <int P, int G>
-__device__ __forceinline__ void tile_put(const float2 (&st)[P], float2* dst, const March3DArgs& a, int x0)
+template <int P, int G, int Q = P>
+__device__ __forceinline__ void tile_put(const float2 (&st)[Q], float2* dst, const March3DArgs& a, int x0)
 {
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
+    for (int j = 0; j < Q; ++j) {
         const int x = x0 + G * j;
         if (x < a.nmx) dst[lds_pad(x)] = st[j];
     }
 }
-template <int P, int G>
+template <int P, int G, int Q = P>
 __device__ __forceinline__ void tile_store(float2* dst, const float2* src, const March3DArgs& a, int x0, bool in)
 {
 #pragma unroll
-    for (int j = 0; j < P; ++j) {
+    for (int j = 0; j < Q; ++j) {
         const int x = x0 + G * j;
         if (x < a.nmx && in) dst[(size_t)x * a.nky] = src[lds_pad(x)];
     }
@@ -302,10 +304,10 @@ __device__ __forceinline__ void tile_store(float2* dst, const float2* src, const
 // of C complex.  conj_src / conj_rec: use conj(L) (-dz).  Workgroups are renumbered so that each
 // XCD (consecutive workgroup ids go round robin over the 8 XCDs) takes a contiguous run of tiles:
 // neighbouring tiles share 128-byte lines, which then meet in one L2.
-template <int NX, int NWF, int C, int BX, int PREC>
+template <int NX, int NWF, int C, int BX, int PREC, bool HALF>
 __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 1024 ? 2 : (NWF == 2 && line_lanes(NX, BX) * 16 == NX ? 3 : 4)))) void march3d_cols(March3DArgs a)
 {
-    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;
+    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P, Q = HALF ? P / 2 : P;
     constexpr int L = LdsLen<NX>::value;
     extern __shared__ float2 smem[];
     const int tiles = (a.nky + C - 1) / C;  // the last tile is partial when C does not divide nky
@@ -328,21 +330,21 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
     auto column = [&](int k) {  // a column from its buffer into registers, forward x-FFT
         float2* buf = smem + (w * NB + (ONE ? 0 : k)) * L;
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int x = t + G * q;
             v[k][q] = x < a.nmx ? buf[lds_pad(x)] : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
-        xfft<NX, -1, BX>(v[k], buf, a, t);
+        xfft<NX, -1, BX, HALF>(v[k], buf, a, t);
     };
     {
-        float2 st[NWF][P];
+        float2 st[NWF][Q];
 #pragma unroll
-        for (int k = 0; k < NWF; ++k) tile_load<P, G>(st[k], state(a, item, wf_of(k)) + ky0 + c, a, x0, kin);
+        for (int k = 0; k < NWF; ++k) tile_load<P, G, Q>(st[k], state(a, item, wf_of(k)) + ky0 + c, a, x0, kin);
 #pragma unroll
         for (int k = 0; k < NWF; ++k) {
             if (ONE && k > 0) __syncthreads();  // the buffers are still in use by the first's transforms
-            tile_put<P, G>(st[k], smem + (c * NB + (ONE ? 0 : k)) * L, a, x0);
+            tile_put<P, G, Q>(st[k], smem + (c * NB + (ONE ? 0 : k)) * L, a, x0);
             if (ONE) {
                 __syncthreads();
                 column(k);
@@ -388,20 +390,20 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
         xfft<NX, +1, BX>(v[k], buf, a, t);
         wave_sync_lds();
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int x = t + G * q;
             if (x < a.nmx) buf[lds_pad(x)] = v[k][q];
         }
         if (ONE) {
             __syncthreads();
-            tile_store<P, G>(state(a, item, wf_of(k)) + ky0 + c1, smem + c1 * L, a, x1, kout);
+            tile_store<P, G, Q>(state(a, item, wf_of(k)) + ky0 + c1, smem + c1 * L, a, x1, kout);
         }
     }
     if constexpr (!ONE) {
         __syncthreads();
 #pragma unroll
         for (int k = 0; k < NWF; ++k)
-            tile_store<P, G>(state(a, item, wf_of(k)) + ky0 + c1, smem + (c1 * NB + k) * L, a, x1, kout);
+            tile_store<P, G, Q>(state(a, item, wf_of(k)) + ky0 + c1, smem + (c1 * NB + k) * L, a, x1, kout);
     }
 }
 
@@ -419,11 +421,11 @@ __device__ __forceinline__ float2* rslice(const March3DArgs& a, int item, int wf
 
 // x-pass: as march3d_cols up to the forward x-FFT, then per vref in use: kz phase of
 // vref[ir][iz] (conj for a -dz step), inverse x-FFT, slice tile written through LDS.
-template <int NX, int NWF, int C, int BX, int PREC>
+template <int NX, int NWF, int C, int BX, int PREC, bool HALF>
 __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 512 || line_lanes(NX, BX) * 16 == NX ? 2 : 4))) void march3d_cols_pspi(
     March3DArgs a)
 {
-    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;
+    constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P, Q = HALF ? P / 2 : P;
     constexpr int L = LdsLen<NX>::value;
     extern __shared__ float2 smem[];
     const int tiles = (a.nky + C - 1) / C;  // the last tile is partial when C does not divide nky
@@ -446,21 +448,21 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
     auto column = [&](int k) {  // a column from its buffer into registers, forward x-FFT
         float2* buf = smem + (w * NB + (ONE ? 0 : k)) * L;
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int x = t + G * q;
             v[k][q] = x < a.nmx ? buf[lds_pad(x)] : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
-        xfft<NX, -1, BX>(v[k], buf, a, t);
+        xfft<NX, -1, BX, HALF>(v[k], buf, a, t);
     };
     {
-        float2 st[NWF][P];
+        float2 st[NWF][Q];
 #pragma unroll
-        for (int k = 0; k < NWF; ++k) tile_load<P, G>(st[k], state(a, item, wf_of(k)) + ky0 + c, a, x0, kin);
+        for (int k = 0; k < NWF; ++k) tile_load<P, G, Q>(st[k], state(a, item, wf_of(k)) + ky0 + c, a, x0, kin);
 #pragma unroll
         for (int k = 0; k < NWF; ++k) {
             if (ONE && k > 0) __syncthreads();  // the buffers are still in use by the first's transforms
-            tile_put<P, G>(st[k], smem + (c * NB + (ONE ? 0 : k)) * L, a, x0);
+            tile_put<P, G, Q>(st[k], smem + (c * NB + (ONE ? 0 : k)) * L, a, x0);
             if (ONE) {
                 __syncthreads();
                 column(k);
@@ -510,13 +512,13 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
             xfft<NX, +1, BX>(bq, buf, a, t);
             wave_sync_lds();
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int x = t + G * q;
                 if (x < a.nmx) buf[lds_pad(x)] = bq[q];
             }
             if (ONE) {
                 __syncthreads();
-                tile_store<P, G>(rslice(a, item, wf_of(k), ir) + ky0 + c1, smem + c1 * L, a, x1, kout);
+                tile_store<P, G, Q>(rslice(a, item, wf_of(k), ir) + ky0 + c1, smem + c1 * L, a, x1, kout);
                 __syncthreads();  // the tile is rewritten by the next wavefield or vref
             }
         }
@@ -524,7 +526,7 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
             __syncthreads();
 #pragma unroll
             for (int k = 0; k < NWF; ++k)
-                tile_store<P, G>(rslice(a, item, wf_of(k), ir) + ky0 + c1, smem + (c1 * NB + k) * L, a, x1, kout);
+                tile_store<P, G, Q>(rslice(a, item, wf_of(k), ir) + ky0 + c1, smem + (c1 * NB + k) * L, a, x1, kout);
             __syncthreads();  // the tile is rewritten by the next vref
         }
     }
@@ -620,29 +622,29 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
 
 // u = the pspiop selection of row x of wavefield wf from the slices of depth iz_sel: inverse
 // y-FFT of each slice in use, per point the slice of its iref1, real part where cut.
-template <int NY, int BY>
+template <int NY, int BY, bool HALF>
 __device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, int wf, int x, LinePoints<NY, BY>& u,
                                                 float2* buf, int t)
 {
-    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P, Q = HALF ? P / 2 : P;
     const uint32_t used = a.used[a.iz_sel];
     const uint8_t* sr = a.sel + (size_t)a.iz_sel * a.nm + (size_t)x * a.nmy;
-    uint8_t s1[P];
+    uint8_t s1[Q];
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         const int y = t + G * q;
         s1[q] = y < a.nmy ? sr[y] : (uint8_t)0x7f;
         u[q] = make_float2(0.f, 0.f);
     }
     // linear mode: the weights of wem.c:476's interpolation, (1 - w2) for iref1 and w2 for iref2
     // at the cut points, 1 for iref1 elsewhere
-    uint8_t s2[P];
-    float wt2[P];
+    uint8_t s2[Q];
+    float wt2[Q];
     if (a.linear) {
         const uint8_t* sr2 = a.sel2 + (size_t)a.iz_sel * a.nm + (size_t)x * a.nmy;
         const float* wr = a.w2 + (size_t)a.iz_sel * a.nm + (size_t)x * a.nmy;
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int y = t + G * q;
             s2[q] = y < a.nmy ? sr2[y] : (uint8_t)0x7f;
             wt2[q] = y < a.nmy ? wr[y] : 0.f;
@@ -658,7 +660,7 @@ __device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, 
         wave_sync_lds();
         if (a.linear) {
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const bool cut = s1[q] >> 7;
                 float wt = (s1[q] & 0x7f) == ir ? (cut ? 1.f - wt2[q] : 1.f) : 0.f;
                 if (cut && s2[q] == ir) wt += wt2[q];
@@ -666,7 +668,7 @@ __device__ __forceinline__ void pspi_select_row(const March3DArgs& a, int item, 
             }
         } else {
 #pragma unroll
-            for (int q = 0; q < P; ++q)
+            for (int q = 0; q < Q; ++q)
                 if ((s1[q] & 0x7f) == ir) u[q] = (s1[q] >> 7) ? make_float2(bq[q].x, 0.f) : bq[q];
         }
     }
@@ -691,10 +693,10 @@ __device__ __forceinline__ float pspi3_weight(uint8_t s1, uint8_t s2, float w2, 
 //   phase 2 modelling receiver: select the previous step's result (zero at the first), inject
 //           m smig of this depth, forward y-FFT
 //   phase 3 modelling output: select the last step's result (zero when no step ran), spectra out
-template <int NY, int BY>
+template <int NY, int BY, bool HALF>
 __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, int phase)
 {
-    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P, Q = HALF ? P / 2 : P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const int ngroups = (a.nitem + F - 1) / F;
@@ -713,7 +715,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         float2 u[P];
         if (a.first) {
 #pragma unroll
-            for (int q = 0; q < P; ++q) u[q] = make_float2(0.f, 0.f);
+            for (int q = 0; q < Q; ++q) u[q] = make_float2(0.f, 0.f);
         } else {
             const float2* src = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
@@ -723,7 +725,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         }
         if (phase == 5) {
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int y = t + G * q;
                 if (y < a.nmy) a.dgw[((size_t)x * a.nmy + y) * a.nf + fl] = u[q];
             }
@@ -732,10 +734,10 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         const float2* sm = a.smig + ((size_t)item * a.nz + a.iz) * a.nm + (size_t)x * a.nmy;
         const float* mt = a.mT + (size_t)a.iz * a.nm + (size_t)x * a.nmy;
         const size_t o = (size_t)a.iz * a.nm + (size_t)x * a.nmy;
-        uint8_t s1[P], s2[P];
-        float wt2[P];
+        uint8_t s1[Q], s2[Q];
+        float wt2[Q];
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int y = t + G * q;
             if (y < a.nmy) {
                 u[q] = cadd(u[q], cscale(sm[y], mt[y]));
@@ -753,9 +755,9 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
             if (!((used >> ir) & 1u)) continue;
             float2 v[P];
 #pragma unroll
-            for (int q = 0; q < P; ++q) v[q] = cscale(u[q], pspi3_weight(s1[q], s2[q], wt2[q], ir));
+            for (int q = 0; q < Q; ++q) v[q] = cscale(u[q], pspi3_weight(s1[q], s2[q], wt2[q], ir));
             wave_sync_lds();
-            yfft<NY, -1, BY>(v, buf, a, t);
+            yfft<NY, -1, BY, HALF>(v, buf, a, t);
             float2* dst = rslice(a, item, 1, ir) + (size_t)x * a.nky;
 #pragma unroll
             for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = v[q];
@@ -767,10 +769,10 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         const int fl = a.f0 + item;
         float2 u[P];
         if (phase == 1) {
-            if (a.ds) pspi_select_row<NY, BY>(a, item, 0, x, u, buf, t);
+            if (a.ds) pspi_select_row<NY, BY, HALF>(a, item, 0, x, u, buf, t);
             float2* sm = a.smig + ((size_t)item * a.nz + a.iz) * a.nm + (size_t)x * a.nmy;
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int y = t + G * q;
                 if (y < a.nmy) sm[y] = a.ds ? u[q] : make_float2(0.f, 0.f);
             }
@@ -778,13 +780,13 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         } else {
             if (a.first) {
 #pragma unroll
-                for (int q = 0; q < P; ++q) u[q] = make_float2(0.f, 0.f);
+                for (int q = 0; q < Q; ++q) u[q] = make_float2(0.f, 0.f);
             } else {
-                pspi_select_row<NY, BY>(a, item, 1, x, u, buf, t);
+                pspi_select_row<NY, BY, HALF>(a, item, 1, x, u, buf, t);
             }
             if (phase == 3) {
 #pragma unroll
-                for (int q = 0; q < P; ++q) {
+                for (int q = 0; q < Q; ++q) {
                     const int y = t + G * q;
                     if (y < a.nmy) a.dgw[((size_t)x * a.nmy + y) * a.nf + fl] = u[q];
                 }
@@ -793,13 +795,13 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
             const float2* sm = a.smig + ((size_t)item * a.nz + a.iz) * a.nm + (size_t)x * a.nmy;
             const float* mt = a.mT + (size_t)a.iz * a.nm + (size_t)x * a.nmy;
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int y = t + G * q;
                 if (y < a.nmy) u[q] = cadd(u[q], cscale(sm[y], mt[y]));
             }
         }
         wave_sync_lds();
-        yfft<NY, -1, BY>(u, buf, a, t);
+        yfft<NY, -1, BY, HALF>(u, buf, a, t);
         float2* dst = state(a, item, phase == 1 ? 0 : 1) + (size_t)x * a.nky;
 #pragma unroll
         for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = u[q];
@@ -809,9 +811,9 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
     const int iw = a.ifmin + a.f0 + (active ? item : 0);
     float2 vs[P], vr[P];
 #pragma unroll
-    for (int q = 0; q < P; ++q) vs[q] = vr[q] = make_float2(0.f, 0.f);
+    for (int q = 0; q < Q; ++q) vs[q] = vr[q] = make_float2(0.f, 0.f);
     if (active && a.ds) {
-        pspi_select_row<NY, BY>(a, item, 0, x, vs, buf, t);
+        pspi_select_row<NY, BY, HALF>(a, item, 0, x, vs, buf, t);
     } else if (active && a.dr) {
         // an unstepped source: its state is FFT_y(u), so the inverse transform returns nky u
         const float2* src = state(a, item, 0) + (size_t)x * a.nky;
@@ -821,20 +823,20 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
         wave_sync_lds();
         const float rn = 1.f / (float)a.nky;  // exact when nky is a power of two
 #pragma unroll
-        for (int q = 0; q < P; ++q) vs[q] = cscale(vs[q], rn);
+        for (int q = 0; q < Q; ++q) vs[q] = cscale(vs[q], rn);
     }
-    if (active && a.dr) pspi_select_row<NY, BY>(a, item, 1, x, vr, buf, t);
-    float cc[P];
+    if (active && a.dr) pspi_select_row<NY, BY, HALF>(a, item, 1, x, vr, buf, t);
+    float cc[Q];
     const float factor = iw == 0 ? 1.f : 2.f;
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         if (t + G * q >= a.nmy) vs[q] = vr[q] = make_float2(0.f, 0.f);
         cc[q] = (active && a.dr) ? factor * (vr[q].x * vs[q].x + vr[q].y * vs[q].y) : 0.f;
     }
     wave_sync_lds();
     float* red = reinterpret_cast<float*>(buf);
 #pragma unroll
-    for (int q = 0; q < P; ++q) red[t + G * q] = cc[q];
+    for (int q = 0; q < Q; ++q) red[t + G * q] = cc[q];
     __syncthreads();
     float* part = a.partial + (size_t)g * a.nm + (size_t)x * a.nmy;
     for (int y = threadIdx.x; y < a.nmy; y += blockDim.x) {
@@ -844,14 +846,14 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
     }
     __syncthreads();
     if (active && a.ds && a.next_s) {
-        yfft<NY, -1, BY>(vs, buf, a, t);
+        yfft<NY, -1, BY, HALF>(vs, buf, a, t);
         float2* dst = state(a, item, 0) + (size_t)x * a.nky;
 #pragma unroll
         for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vs[q];
         wave_sync_lds();
     }
     if (active && a.dr && a.next_r) {
-        yfft<NY, -1, BY>(vr, buf, a, t);
+        yfft<NY, -1, BY, HALF>(vr, buf, a, t);
         float2* dst = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
         for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vr[q];
@@ -862,10 +864,10 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
 // of frequency item g F + f.  ds / dr: the source / receiver was stepped at this depth; next_s /
 // next_r: it is stepped at the next depth (its forward y-FFT is needed); the imaging runs when dr.
 // The split-step phase is computed once and applied conjugated to the source.
-template <int NY, int BY, int PREC>
+template <int NY, int BY, int PREC, bool HALF>
 __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs a, int F)
 {
-    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P, Q = HALF ? P / 2 : P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const int ngroups = (a.nitem + F - 1) / F;
@@ -901,11 +903,11 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
         }
     }
     if (need_r) yfft<NY, +1, BY>(vr, buf, a, t);
-    float cc[P];
+    float cc[Q];
     const float factor = iw == 0 ? 1.f : 2.f;
     const float tx = a.taper_x[x];
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         const int y = t + G * q;
         if (y < a.nmy) {
             if (a.ds || a.dr) {
@@ -923,7 +925,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
     wave_sync_lds();
     float* red = reinterpret_cast<float*>(buf);
 #pragma unroll
-    for (int q = 0; q < P; ++q) red[t + G * q] = cc[q];
+    for (int q = 0; q < Q; ++q) red[t + G * q] = cc[q];
     __syncthreads();
     float* part = a.partial + (size_t)g * a.nm + (size_t)x * a.nmy;
     for (int y = threadIdx.x; y < a.nmy; y += blockDim.x) {
@@ -934,14 +936,14 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
     __syncthreads();
     // forward y-FFTs that start the next step
     if (active && a.ds && a.next_s) {
-        yfft<NY, -1, BY>(vs, buf, a, t);
+        yfft<NY, -1, BY, HALF>(vs, buf, a, t);
         float2* dst = state(a, item, 0) + (size_t)x * a.nky;
 #pragma unroll
         for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vs[q];
         wave_sync_lds();
     }
     if (active && a.dr && a.next_r) {
-        yfft<NY, -1, BY>(vr, buf, a, t);
+        yfft<NY, -1, BY, HALF>(vr, buf, a, t);
         float2* dst = state(a, item, 1) + (size_t)x * a.nky;
 #pragma unroll
         for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) dst[t + G * q] = vr[q];
@@ -958,10 +960,10 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
 //           receiver's step; at the first call the state is the source trace, later IFFTy of
 //           the previous step's result is stored in smig at depth iz_sel; with ds the next step
 //           starts (taper, conj(SS), FFTy).
-template <int NY, int BY, int PREC>
+template <int NY, int BY, int PREC, bool HALF>
 __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs a, int F, int phase)
 {
-    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P;
+    constexpr int G = Line<NY, BY>::G, P = Line<NY, BY>::P, Q = HALF ? P / 2 : P;
     constexpr int L = LdsLen<NY>::value;
     extern __shared__ float2 smem[];
     const int ngroups = (a.nitem + F - 1) / F;
@@ -979,7 +981,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
         const float tx = a.taper_x[x];
         if (a.first) {
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int y = t + G * q;
                 v[q] = (y < a.nmy && x * a.nmy + y == a.igx) ? a.spec_s[fl] : make_float2(0.f, 0.f);
             }
@@ -989,20 +991,20 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
             yfft<NY, +1, BY>(v, buf, a, t);
             float2* sm = a.smig + ((size_t)item * a.nz + a.iz_sel) * a.nm + (size_t)x * a.nmy;
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int y = t + G * q;
                 if (y < a.nmy) sm[y] = v[q];
             }
         }
         if (!a.ds) return;
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int y = t + G * q;
             v[q] = y < a.nmy ? cmulc(cscale(v[q], tx * a.taper_y[y]), ss_phase<PREC>(a, wd, (size_t)x * a.nmy + y))
                              : make_float2(0.f, 0.f);
         }
         wave_sync_lds();
-        yfft<NY, -1, BY>(v, buf, a, t);
+        yfft<NY, -1, BY, HALF>(v, buf, a, t);
 #pragma unroll
         for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) row[t + G * q] = v[q];
         return;
@@ -1019,7 +1021,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
     float2* sm = a.smig + ((size_t)item * a.nz + a.iz) * a.nm + (size_t)x * a.nmy;
     const float* mt = a.mT + (size_t)a.iz * a.nm + (size_t)x * a.nmy;
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         const int y = t + G * q;
         if (y >= a.nmy) {
             v[q] = make_float2(0.f, 0.f);
@@ -1035,7 +1037,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
     }
     if (phase == 2) {
 #pragma unroll
-        for (int q = 0; q < P; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const int y = t + G * q;
             if (y < a.nmy) a.dgw[((size_t)x * a.nmy + y) * a.nf + fl] = v[q];
         }
@@ -1043,7 +1045,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_fwd(March3DArgs 
     }
     if (phase == 0 && !(a.ds && a.next_s)) return;  // state unchanged / no further step
     wave_sync_lds();
-    yfft<NY, -1, BY>(v, buf, a, t);
+    yfft<NY, -1, BY, HALF>(v, buf, a, t);
 #pragma unroll
     for (int q = 0; q < P; ++q) if (yin<BY>(a, t + G * q)) row[t + G * q] = v[q];
 }
@@ -1463,6 +1465,13 @@ static int launch3(K kernel, dim3 grid, dim3 block, size_t lds, hipStream_t st, 
 template <int N, int BL, int PREC>
 static int launch3_prec(int which, const March3DArgs& a, int F, int phase, hipStream_t st)
 {
+    // HALF kernels: a power-of-two axis with 2 n <= N live points (pad factor 2 and up).  The upper half of
+    // every line is zero going into the forward transform and dropped coming out of the inverse, so its
+    // first radix-2 stage, its staging and its registers go.  Per launch, general form -> HALF, at 256 x 256
+    // transforms: PSPI x-pass 240 -> 182 us and y-pass 176 -> 114 us (201 -> 139 VGPRs); split-step
+    // modelling march 37.3 -> 35.2 ms; 512 x 512 migration 418 -> 409 ms.  All lines live: the general form.
+    constexpr bool HALF = BL == kLenPow2;
+    auto half = [](int n, auto with, auto without) { return HALF && 2 * n <= N ? with : without; };
     constexpr int L = LdsLen<N>::value, G = Line<N, BL>::G;
     if (which == 0) {  // init
         const size_t rows = (size_t)a.nitem * 2 * a.nmx;
@@ -1476,8 +1485,9 @@ static int launch3_prec(int which, const March3DArgs& a, int F, int phase, hipSt
         const int C = nwf == 2 ? C2 : C1;
         const size_t lds = (size_t)C * tile_bufs(N, BL, nwf) * L * sizeof(float2);
         const dim3 grid(a.nitem * ((a.nky + C - 1) / C)), block(G * C);
-        return nwf == 2 ? launch3(march3d_cols<N, 2, C2, BL, PREC>, grid, block, lds, st, a)
-                        : launch3(march3d_cols<N, 1, C1, BL, PREC>, grid, block, lds, st, a);
+        const auto two = half(a.nmx, march3d_cols<N, 2, C2, BL, PREC, HALF>, march3d_cols<N, 2, C2, BL, PREC, false>);
+        const auto one = half(a.nmx, march3d_cols<N, 1, C1, BL, PREC, HALF>, march3d_cols<N, 1, C1, BL, PREC, false>);
+        return launch3(nwf == 2 ? two : one, grid, block, lds, st, a);
     }
     if (which == 4) {  // PSPI x-pass
         const int nwf = (a.wmask & 1) + ((a.wmask >> 1) & 1);
@@ -1485,8 +1495,9 @@ static int launch3_prec(int which, const March3DArgs& a, int F, int phase, hipSt
         const int C = nwf == 2 ? C2 : C1;
         const size_t lds = (size_t)C * tile_bufs(N, BL, nwf) * L * sizeof(float2);
         const dim3 grid(a.nitem * ((a.nky + C - 1) / C)), block(G * C);
-        return nwf == 2 ? launch3(march3d_cols_pspi<N, 2, C2, BL, PREC>, grid, block, lds, st, a)
-                        : launch3(march3d_cols_pspi<N, 1, C1, BL, PREC>, grid, block, lds, st, a);
+        const auto two = half(a.nmx, march3d_cols_pspi<N, 2, C2, BL, PREC, HALF>, march3d_cols_pspi<N, 2, C2, BL, PREC, false>);
+        const auto one = half(a.nmx, march3d_cols_pspi<N, 1, C1, BL, PREC, HALF>, march3d_cols_pspi<N, 1, C1, BL, PREC, false>);
+        return launch3(nwf == 2 ? two : one, grid, block, lds, st, a);
     }
     if (which == 6) {  // linear-mode modelling receiver x-pass (gather over vrefs)
         constexpr int CG = tile_cols(N, BL, 1);
@@ -1497,18 +1508,16 @@ static int launch3_prec(int which, const March3DArgs& a, int F, int phase, hipSt
     const int ngroups = (a.nitem + F - 1) / F;
     if (which == 5) {
         const size_t lds = (size_t)F * L * sizeof(float2);
-        return launch3(march3d_rows_pspi<N, BL>, dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F, phase);
+        return launch3(half(a.nmy, march3d_rows_pspi<N, BL, HALF>, march3d_rows_pspi<N, BL, false>), dim3(ngroups * a.nmx), dim3(G * F),
+                       lds, st, a, F, phase);
     }
     if (which == 2) {
         const size_t lds = (size_t)F * L * sizeof(float2);
-        return launch3(march3d_rows_adj<N, BL, PREC>, dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F);
+        return launch3(half(a.nmy, march3d_rows_adj<N, BL, PREC, HALF>, march3d_rows_adj<N, BL, PREC, false>), dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F);
     }
     const size_t lds = (size_t)F * L * sizeof(float2);
-    SWEM_HIP(hipFuncSetAttribute((const void*)march3d_rows_fwd<N, BL, PREC>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                 (int)lds));
-    hipLaunchKernelGGL((march3d_rows_fwd<N, BL, PREC>), dim3(ngroups * a.nmx), dim3(G * F), lds, st, a, F, phase);
-    SWEM_HIP(hipGetLastError());
-    return SWEM_OK;
+    return launch3(half(a.nmy, march3d_rows_fwd<N, BL, PREC, HALF>, march3d_rows_fwd<N, BL, PREC, false>), dim3(ngroups * a.nmx),
+                   dim3(G * F), lds, st, a, F, phase);
 }
 
 // The naive-FP32 phases (library sine and cosine per point) are kernels of their own: beside the KZ64
