@@ -725,6 +725,7 @@ __device__ __forceinline__ void adj_body_pair(const March2DArgs& a)
         const float2* held = xf.held.ptr();
         float2 *bu = smem, *bv = smem + LdsLen<N>::value;
         float2 L[P], sp[Q];
+        sync();  // the single steps above leave their last exchange unread by slower waves
         if (iz < a.nz) {
             c.iz = iz;
             xf.kload_row(L, krow(a, c, 0), a, t);
@@ -737,6 +738,7 @@ __device__ __forceinline__ void adj_body_pair(const March2DArgs& a)
                 if (z >= a.sz) adj_step<N, P, MODE, WAVE, HALF, X>(us, smem, pp, a, xf, c, true, true);
                 if (z >= a.gz) adj_step<N, P, MODE, WAVE, HALF, X>(ur, smem, pp, a, xf, c, true, false);
                 image(iz, z >= a.gz);
+                sync();
                 c.iz = min(iz + 1, a.nz - 1);
                 xf.kload_row(L, krow(a, c, 0), a, t);
                 ss_load<T, Q>(sp, a, c);

@@ -46,3 +46,18 @@ def test_half_lines_2d(gpu, pspi, mode, nx, padx):
     e1, e2 = both(g, vel, wav, g.dmx * (nx // 3), 0.0, d, m, mode)
     print(f"nkx={nx * padx} padx={padx} pspi={pspi} mode={mode}: migrate {e1:.3e} model {e2:.3e}", flush=True)
     assert e1 <= TOL and e2 <= TOL
+
+
+@pytest.mark.parametrize("variant", [seiswem.VARIANT_AUTO, seiswem.VARIANT_PAIR, seiswem.VARIANT_PAIR8])
+@pytest.mark.parametrize("nx", [256, 512, 1024])
+def test_single_steps_before_the_lockstep_ones(gpu, nx, variant):
+    """A source below the receivers: the first depths step the receiver alone, the rest both in lockstep
+    through the same LDS buffers."""
+    g, vel, wav, rng = case(False, nx, 2, 16, 64, seed=nx + 1)
+    g.sz = g.oz + 4.5 * g.dz
+    d = rng.standard_normal((g.nm, g.nt)).astype(np.float32)
+    sx = g.dmx * (nx // 3)
+    m = seiswem.ShotProfileWEM(d[None], True, vel=vel, wav=wav, geom=g, sx=[sx], variant=variant)
+    err = rel_l2(m, O.wem(oparams(g), vel, wav, sx, d=d, adj=True))
+    print(f"nkx={2 * nx} variant={variant}: migrate {err:.3e}", flush=True)
+    assert err <= TOL
