@@ -1511,21 +1511,79 @@ int launch_angles_len(int which, int kind, const March2DArgs& ax, const March2DA
 // recombined; the P and S images correlate the potentials with the source.  The separation
 // matrix of wavenumber kx (kx = dkx ikx for ikx < nkx/2, else -(dkx nkx - dkx ikx)) uses the
 // depth's layer velocities vp0 = 1/po_p, vs0 = 1/po_s and is computed in place.
+// Two wavefields through the transform: in lockstep on a power-of-two length (fft2), else in turn.
+// A depth takes seven dependent pairs of transforms at two waves per SIMD (200 VGPRs), so barriers and
+// exchanges, not the vector ALUs, bound the march; the potentials and the components always go in pairs.
+// 4 shots of 512 traces x 300 depths x 576 frequencies, adjoint: 22.0 ms in turn over whole lines, 20.8
+// with the zero half dropped, 17.5 in lockstep as well.  Three waves per SIMD spill (216 bytes): no faster.
+template <int N, int P, int SIGN, bool HIN, class X>
+__device__ __forceinline__ void ewem_fft(float2 (&u)[P], float2 (&v)[P], float2* lds, int& pp, const March2DArgs& a,
+                                         const X& xf, int t)
+{
+    if constexpr (std::is_same<X, XPow2<N, P, false, kSeedHeld>>::value) {
+        fft2<N, P, SIGN, HIN>(u, v, lds, lds + LdsLen<N>::value, xf.held.ptr(), t, [] { subgroup_sync<N / P>(); });
+    } else {
+        xf.template fft<SIGN, false, HIN>(u, lds, a, t, pp);
+        xf.template fft<SIGN, false, HIN>(v, lds, a, t, pp);
+    }
+}
+
+// The split-step steps of the two potentials, each with its own phase tables: BACK the forward
+// operator (split step first, then the phases of -dz), else the adjoint one.
+template <int N, int P, bool HALF, bool BACK, class X>
+__device__ __forceinline__ void ewem_step(float2 (&u)[P], float2 (&v)[P], float2* lds, int& pp, const March2DArgs& ap,
+                                          const March2DArgs& as, const X& xf, const StepCtx& c)
+{
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
+    float2 L[P], sp[Q], ss[Q];
+    if constexpr (BACK) {
+        ss_load<T, Q>(sp, ap, c);
+        ss_load<T, Q>(ss, as, c);
+#pragma unroll
+        for (int q = 0; q < Q; ++q) {
+            u[q] = cmulc(u[q], sp[q]);
+            v[q] = cmulc(v[q], ss[q]);
+        }
+    }
+    xf.kload_row(L, krow(ap, c, 0), ap, c.t);
+    ewem_fft<N, P, -1, HALF>(u, v, lds, pp, ap, xf, c.t);
+#pragma unroll
+    for (int q = 0; q < P; ++q) u[q] = cmul_c(u[q], L[q], BACK);
+    xf.kload_row(L, krow(as, c, 0), as, c.t);
+#pragma unroll
+    for (int q = 0; q < P; ++q) v[q] = cmul_c(v[q], L[q], BACK);
+    if constexpr (!BACK) {
+        ss_load<T, Q>(sp, ap, c);
+        ss_load<T, Q>(ss, as, c);
+    }
+    ewem_fft<N, P, +1, false>(u, v, lds, pp, ap, xf, c.t);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        if constexpr (BACK) {
+            if (c.t + q * T >= ap.nmx) u[q] = v[q] = make_float2(0.f, 0.f);
+        } else {
+            u[q] = cmul(u[q], sp[q]);
+            v[q] = cmul(v[q], ss[q]);
+        }
+    }
+    zero_tail<P, Q>(u);
+    zero_tail<P, Q>(v);
+}
+
 // (i1, i2) -> (o1, o2) through the wavenumber domain; o1, o2 are zero at x >= nmx.
-template <int N, int P, class X>
+template <int N, int P, bool HALF, class X>
 __device__ __forceinline__ void esep(const float2 (&i1)[P], const float2 (&i2)[P], float2 (&o1)[P], float2 (&o2)[P],
                                      float2* lds, int& pp, const March2DArgs& a, const X& xf, const EwemArgs& e, int t, float w,
                                      float vp, float vs, bool sep, bool adj)
 {
-    constexpr int T = N / P;
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
     const int n = a.nkx;
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         o1[q] = i1[q];
         o2[q] = i2[q];
     }
-    xf.template fft<-1, false>(o1, lds, a, t, pp);
-    xf.template fft<-1, false>(o2, lds, a, t, pp);
+    ewem_fft<N, P, -1, HALF>(o1, o2, lds, pp, a, xf, t);
 #pragma unroll
     for (int q = 0; q < P; ++q) {
         const int k = t + q * T;
@@ -1536,18 +1594,19 @@ __device__ __forceinline__ void esep(const float2 (&i1)[P], const float2 (&i2)[P
         o1[q] = k < n ? cscale(r1, a.inv_nk) : make_float2(0.f, 0.f);
         o2[q] = k < n ? cscale(r2, a.inv_nk) : make_float2(0.f, 0.f);
     }
-    xf.template fft<+1, false>(o1, lds, a, t, pp);
-    xf.template fft<+1, false>(o2, lds, a, t, pp);
+    ewem_fft<N, P, +1, false>(o1, o2, lds, pp, a, xf, t);
 #pragma unroll
-    for (int q = 0; q < P; ++q)
+    for (int q = 0; q < Q; ++q)
         if (t + q * T >= a.nmx) o1[q] = o2[q] = make_float2(0.f, 0.f);
+    zero_tail<P, Q>(o1);
+    zero_tail<P, Q>(o2);
 }
 
-template <int N, int P, class X, bool ADJ>
+template <int N, int P, bool HALF, class X, bool ADJ>
 __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void ewem_march(March2DArgs ap,
                                                                                              March2DArgs as, EwemArgs e)
 {
-    constexpr int T = N / P;
+    constexpr int T = N / P, Q = HALF ? P / 2 : P;
     extern __shared__ float2 smem[];
     int g, shot;
     decode_block(ap.ngroups, ap.nshot, g, shot);
@@ -1568,12 +1627,15 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
     const size_t sp = (size_t)shot * ap.nmx * e.nf;  // this shot's spectra
     float2 us[P], rx[P], rz[P];
 #pragma unroll
-    for (int q = 0; q < P; ++q) {
+    for (int q = 0; q < Q; ++q) {
         const int x = t + q * T;
         us[q] = (active && x == igx) ? ap.spec_s[fl] : make_float2(0.f, 0.f);
         rx[q] = (ADJ && active && x < ap.nmx) ? e.spx[sp + (size_t)x * e.nf + fl] : make_float2(0.f, 0.f);
         rz[q] = (ADJ && active && x < ap.nmx) ? e.spz[sp + (size_t)x * e.nf + fl] : make_float2(0.f, 0.f);
     }
+    zero_tail<P, Q>(us);
+    zero_tail<P, Q>(rx);
+    zero_tail<P, Q>(rz);
     // partial images / stored source of (shot, frequency)
     const size_t vol = ((size_t)shot * ap.ngroups + (active ? fc : 0)) * ap.nz * ap.nmx;
     if constexpr (ADJ) {
@@ -1581,20 +1643,20 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
             c.iz = iz;
             const float z = ap.oz + ap.dz * (float)iz;
             const bool ds = z >= ap.sz, dr = z >= ap.gz;
-            if (ds) ssf_adj_step<N, P, false, true, false, X>(us, smem, pp, ap, xf, c, true);
+            if (ds) ssf_adj_step<N, P, false, true, HALF, X>(us, smem, pp, ap, xf, c, true);
+            subgroup_sync<T>();  // the lockstep transforms write both buffers, the single one's last exchange with them
             float2 up[P], u2[P];
             if (dr) {
                 const float vp = e.vp0[iz], vs = e.vs0[iz];
-                esep<N, P, X>(rx, rz, up, u2, smem, pp, ap, xf, e, t, w, vp, vs, true, true);
-                ssf_adj_step<N, P, false, true, false, X>(up, smem, pp, ap, xf, c, false);
-                ssf_adj_step<N, P, false, true, false, X>(u2, smem, pp, as, xf, c, false);
-                esep<N, P, X>(up, u2, rx, rz, smem, pp, ap, xf, e, t, w, vp, vs, false, true);
+                esep<N, P, HALF, X>(rx, rz, up, u2, smem, pp, ap, xf, e, t, w, vp, vs, true, true);
+                ewem_step<N, P, HALF, false, X>(up, u2, smem, pp, ap, as, xf, c);
+                esep<N, P, HALF, X>(up, u2, rx, rz, smem, pp, ap, xf, e, t, w, vp, vs, false, true);
             }
             if (active) {
                 const auto rp = buf_rsrc(e.ppart + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 4u);
                 const auto rs = buf_rsrc(e.spart + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 4u);
 #pragma unroll
-                for (int q = 0; q < P; ++q) {
+                for (int q = 0; q < Q; ++q) {
                     const float2 sm = ds ? cscale(us[q], e.inv_maxs) : make_float2(0.f, 0.f);
                     const uint32_t off = (uint32_t)(t + q * T) * 4u;
                     buf_store1(rp, off, dr ? factor * (sm.x * up[q].x + sm.y * up[q].y) : 0.f);
@@ -1607,29 +1669,30 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
             c.iz = iz;
             const float z = ap.oz + ap.dz * (float)iz;
             const bool ds = z >= ap.sz;
-            if (ds) ssf_adj_step<N, P, false, true, false, X>(us, smem, pp, ap, xf, c, true);
+            if (ds) ssf_adj_step<N, P, false, true, HALF, X>(us, smem, pp, ap, xf, c, true);
             if (active) {
                 const auto sr = buf_rsrc(e.smig + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 8u);
 #pragma unroll
-                for (int q = 0; q < P; ++q)
+                for (int q = 0; q < Q; ++q)
                     buf_store2(sr, (uint32_t)(t + q * T) * 8u, ds ? cscale(us[q], e.inv_maxs) : make_float2(0.f, 0.f));
             }
         }
+        subgroup_sync<T>();  // as in the migration
         for (int iz = ap.nz - 1; iz >= 0; --iz) {  // receiver upward (ewem.c:328-346)
             c.iz = iz;
             const float z = ap.oz + ap.dz * (float)iz;
             if (!(z >= ap.gz)) continue;
             const float vp = e.vp0[iz], vs = e.vs0[iz];
             float2 up[P], u2[P];
-            esep<N, P, X>(rx, rz, up, u2, smem, pp, ap, xf, e, t, w, vp, vs, true, false);
+            esep<N, P, HALF, X>(rx, rz, up, u2, smem, pp, ap, xf, e, t, w, vp, vs, true, false);
             if (active) {
                 const auto sr = buf_rsrc(e.smig + vol + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 8u);
                 const auto mp = buf_rsrc(e.mppT + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 4u);
                 const auto ms = buf_rsrc(e.mpsT + (size_t)iz * ap.nmx, (uint32_t)ap.nmx * 4u);
-                float2 sv[P];
-                float mpv[P], msv[P];
+                float2 sv[Q];
+                float mpv[Q], msv[Q];
 #pragma unroll
-                for (int q = 0; q < P; ++q) {
+                for (int q = 0; q < Q; ++q) {
                     const uint32_t x = (uint32_t)(t + q * T);
                     sv[q] = buf_load2(sr, x * 8u);
                     mpv[q] = buf_load1(mp, x * 4u);
@@ -1637,21 +1700,17 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
                 }
                 __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                for (int q = 0; q < P; ++q) {
+                for (int q = 0; q < Q; ++q) {
                     up[q] = cadd(up[q], cscale(sv[q], mpv[q]));
                     u2[q] = cadd(u2[q], cscale(sv[q], msv[q]));
                 }
             }
-            float2 sp[P];
-            ss_load<T, P>(sp, ap, c);
-            ssf_fwd_step<N, P, false, false, X>(up, smem, pp, ap, xf, c, sp);
-            ss_load<T, P>(sp, as, c);
-            ssf_fwd_step<N, P, false, false, X>(u2, smem, pp, as, xf, c, sp);
-            esep<N, P, X>(up, u2, rx, rz, smem, pp, ap, xf, e, t, w, vp, vs, false, false);
+            ewem_step<N, P, HALF, true, X>(up, u2, smem, pp, ap, as, xf, c);
+            esep<N, P, HALF, X>(up, u2, rx, rz, smem, pp, ap, xf, e, t, w, vp, vs, false, false);
         }
         if (active) {
 #pragma unroll
-            for (int q = 0; q < P; ++q) {
+            for (int q = 0; q < Q; ++q) {
                 const int x = t + q * T;
                 if (x < ap.nmx) {
                     e.dgx[sp + (size_t)x * e.nf + fl] = rx[q];
@@ -1662,12 +1721,12 @@ __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void
     }
 }
 
-template <int N, class X>
+template <int N, class X, bool HALF = false>
 static int launch_ewem_n(const March2DArgs& ap, const March2DArgs& as, const EwemArgs& e, int adj, hipStream_t st)
 {
     constexpr int P = N >= 1024 ? 8 : N / 64, T = N / P;
     const size_t lds = (size_t)LdsLen<N>::value * 2 * sizeof(float2);
-    auto k = adj ? ewem_march<N, P, X, true> : ewem_march<N, P, X, false>;
+    auto k = adj ? ewem_march<N, P, HALF, X, true> : ewem_march<N, P, HALF, X, false>;
     SWEM_HIP(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, dim3(march2d_grid_blocks(ap.ngroups, ap.nshot)), dim3(T), lds, st, ap, as, e);
     SWEM_HIP(hipGetLastError());
@@ -1683,7 +1742,8 @@ int launch_ewem_len(int kind, const March2DArgs& ap, const March2DArgs& as, cons
     if constexpr (N <= 2048)
         if (kind == kLenMixedPrime) return launch_ewem_n<N, XMixed<N, P, true>>(ap, as, e, adj, st);
     return kind == kLenBluestein ? launch_ewem_n<N, XBlue<N, P>>(ap, as, e, adj, st)
-                                 : launch_ewem_n<N, XPow2<N, P>>(ap, as, e, adj, st);
+           : 2 * ap.nmx <= N         ? launch_ewem_n<N, XPow2<N, P, false, kSeedHeld>, true>(ap, as, e, adj, st)
+                                     : launch_ewem_n<N, XPow2<N, P, false, kSeedHeld>>(ap, as, e, adj, st);
 }
 
 }  // namespace swem
