@@ -1140,11 +1140,24 @@ __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void
 
 #define SWEM_SUBGROUP_BOUNDS(P) __launch_bounds__((P) == 16 ? 512 : kMaxBlock)
 
+// Where the marches of one wavefield per thread keep their twiddle seeds.  Held in registers they drop the
+// table loads and address arithmetic of every transform; the half-line kernels have the registers for it,
+// the general form at 16 points per thread spills (288 to 388 bytes) and so does the 128-register budget
+// of the large workgroups with 8.  Read ahead -> held, 8 shots x 100 depths, 1024 / 512 traces, and 16
+// shots of 256: split-step modelling 4.9 -> 3.8, 2.3 -> 1.8, 2.5 -> 1.6 ms; PSPI modelling 10.9 -> 9.2,
+// 5.1 -> 4.2, 5.4 -> 4.0; linear modelling 11.5 -> 10.1, 5.3 -> 4.6, 5.5 -> 4.3; linear migration 11.3 ->
+// 9.9, 5.3 -> 4.7, 5.9 -> 4.7.  Two vrefs of a PSPI step in lockstep on top spill (188 bytes): 76 -> 81 ms
+// where held alone gives 63.
+constexpr int held_if(bool fits) { return fits ? kSeedHeld : kSeedAhead; }
+
 template <int N, int MODE, int P>
 __global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_adj(March2DArgs a) { adj_body<N, P, MODE, false>(a); }
 
 template <int N, int MODE, int P, bool HALF>
-__global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_fwd(March2DArgs a) { fwd_body<N, P, MODE, false, HALF>(a); }
+__global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_fwd(March2DArgs a)
+{
+    fwd_body<N, P, MODE, false, HALF, XPow2<N, P, false, held_if(HALF && P == 16)>>(a);
+}
 
 template <int N, int MODE>
 __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_w(March2DArgs a)
@@ -1155,7 +1168,7 @@ __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2)))
 template <int N, int MODE, bool HALF>
 __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_w(March2DArgs a)
 {
-    fwd_body<N, N / 64, MODE, true, HALF>(a);
+    fwd_body<N, N / 64, MODE, true, HALF, XPow2<N, N / 64, true, held_if(HALF && N <= 1024)>>(a);
 }
 
 // PAIR: 16 points per thread from nkx = 1024 (nkx/16 threads, radix-16 passes), one wave with
@@ -1163,13 +1176,13 @@ __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2)))
 template <int N, int MODE, int P, bool HALF>
 __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_pair(March2DArgs a)
 {
-    adj_body_pair<N, P, MODE, false, HALF, XPow2<N, P, false, MODE == kModeSSF ? kSeedHeld : kSeedAhead>>(a);
+    adj_body_pair<N, P, MODE, false, HALF, XPow2<N, P, false, held_if(HALF || MODE == kModeSSF)>>(a);
 }
 
 template <int N, int MODE, bool HALF>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_pair_w(March2DArgs a)
 {
-    adj_body_pair<N, N / 64, MODE, true, HALF, XPow2<N, N / 64, true, MODE == kModeSSF ? kSeedHeld : kSeedAhead>>(a);
+    adj_body_pair<N, N / 64, MODE, true, HALF, XPow2<N, N / 64, true, held_if(HALF || MODE == kModeSSF)>>(a);
 }
 
 // Transform lengths that are not powers of two: Bluestein through the array length M (one
