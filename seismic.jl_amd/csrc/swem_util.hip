@@ -24,7 +24,7 @@ namespace swem {
 //               69 of the 146 TFLOP/s that a large FP32 product reaches.
 //   gemm_split  32 x 32 outputs per workgroup, one wave per segment straight from memory, the segment sums
 //               meeting in LDS.  For the others: one shot's 128 traces (30 tiles of 64 x 64) waited 200 us
-//               for a serial loop over K; that launch takes about 30 us now.
+//               for a serial loop over K; that launch takes under 30 us now.
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 constexpr int kGemmSegs = 16;
 
