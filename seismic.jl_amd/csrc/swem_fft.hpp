@@ -73,17 +73,65 @@ __device__ __forceinline__ void bfly1(float2& a, float2& b)
 
 constexpr int bitrev(int i, int n) { return n <= 1 ? 0 : (i & 1) * (n / 2) + bitrev(i >> 1, n / 2); }
 
-// Twiddles of a radix-R butterfly, R = 2, 4, 8 or 16, whose input r is multiplied by w^r: it runs
-// as log2 R radix-2 stages on inputs in bit-reversed order, and the stage of block size S takes
+// Twiddles of a radix-R butterfly, R = 2, 4, 8 or 16, whose input r is multiplied by w^r, in two forms.
+// Staged: log2 R radix-2 stages on inputs in bit-reversed order; the stage of block size S takes
 // w^(R/S) W_S^m, m < S / 4 (m < 1 for S = 2); the upper quarter is SIGN i times these, a swap.
 // So R / 2 seeds in all: [S = 2: w^(R/2)] [S = 4: w^(R/4)] [S = 8: w^(R/8), w^(R/8) W_8]
-// [S = 16: w, w W_16, w W_8, w W_16^3], each one entry of the twiddle table.
-template <int R>
+// [S = 16: w, w W_16, w W_8, w W_16^3], each one entry of the twiddle table.  An input passes up to
+// log2 R of them, whose roundings add up.
+// Direct: an input passes one table entry per radix-4 level (radix 4: w, w^2, w^3; radix 16 as 4 x 4:
+// w^4, w^8, w^12, then w^c W_16^(c m), c = 1, 3 with m < 4 and c = 2 with m < 2, the rest by a swap; radix 8:
+// w .. w^7 before a plain butterfly), in as many operations at radix 4 and 16 but with up to half as many
+// seeds again.  The entries' rounding is the same at every depth of a march and adds up: error against 64 bits
+// of 200 steps FFT, phase, IFFT in float arithmetic, powers by one product of two entries | staged | direct:
+//   256 points  9.3e-6 (four radix-4 passes, no products) | 12.6e-6 | 9.3e-6, in radix-4 or in radix-16 passes
+//   128 points  12.0e-6 (seven radix-2 passes) | 11.9e-6 as 16 x 8
+//   512, 1024, 2048 points  14.6e-6, 16.2e-6, 18.3e-6 | 12.7e-6, 13.2e-6, 13.5e-6
+// So lines of 256 points take the direct form (128 x 128 3-D modelling 35.4 -> 37.3 ms, PSPI migration 49.4 ->
+// 50.5 ms, one 2-D shot of 128 traces 0.381 -> 0.374 ms); the longer lines' kernels hold their seeds in registers
+// and have none left for more.
+constexpr bool direct_twiddles(int N) { return N == 256; }
+template <int R, bool DIRECT>
 constexpr int seed_count()
 {
-    return R / 2;
+    return !DIRECT ? R / 2 : R == 16 ? 13 : R - 1;
 }
 constexpr int seed_off(int S) { return S <= 2 ? 0 : S / 4; }
+
+// Radix-4 butterfly in place, natural order: inputs 1, 2, 3 times w1, w2, w3 (ONE2: w2 = 1).
+template <int SIGN, bool ONE2 = false>
+__device__ __forceinline__ void radix4(float2& x0, float2& x1, float2& x2, float2& x3, float2 w1, float2 w2, float2 w3)
+{
+    if constexpr (ONE2) bfly1(x0, x2);
+    else bfly(x0, x2, w2);
+    float2 t = make_float2(fmaf(w1.x, x1.x, -(w1.y * x1.y)), fmaf(w1.x, x1.y, w1.y * x1.x));
+    bfly(t, x3, w3);
+    const float2 d = mul_si<SIGN>(x3), a = x0, b = x2;
+    x0 = cadd(a, t);
+    x2 = csub(a, t);
+    x1 = cadd(b, d);
+    x3 = csub(b, d);
+}
+// The same with unit twiddles; HIN: x2 = x3 = 0, not read.
+template <int SIGN, bool HIN = false>
+__device__ __forceinline__ void radix4_plain(float2& x0, float2& x1, float2& x2, float2& x3)
+{
+    if constexpr (HIN) {
+        const float2 a = x0, t = x1, d = mul_si<SIGN>(x1);
+        x0 = cadd(a, t);
+        x2 = csub(a, t);
+        x1 = cadd(a, d);
+        x3 = csub(a, d);
+    } else {
+        bfly1(x0, x2);
+        bfly1(x1, x3);
+        const float2 t = x1, d = mul_si<SIGN>(x3), a = x0, b = x2;
+        x0 = cadd(a, t);
+        x2 = csub(a, t);
+        x1 = cadd(b, d);
+        x3 = csub(b, d);
+    }
+}
 
 // The radix-R butterfly in place on x[0..R), natural order in and out.  TW: with the seeds s
 // (those of exp(-...), conjugated here for SIGN > 0); otherwise w = 1 and the constants are
@@ -124,6 +172,67 @@ __device__ __forceinline__ void dft_pow2(float2 (&x)[R], const float2* s)
     }
 #pragma unroll
     for (int i = 0; i < R; ++i) x[i] = y[i];
+}
+
+// The direct form.  Seeds s (of exp(-...), conjugated here for SIGN > 0) in the order named above.
+template <int R, int SIGN, bool TW, bool HIN = false>
+__device__ __forceinline__ void dft_direct(float2 (&x)[R], const float2* s)
+{
+    auto seed = [&](int i) { return SIGN > 0 ? cconj(s[i]) : s[i]; };
+    if constexpr (R <= 2 || (R == 4 && !TW)) {
+        dft_pow2<R, SIGN, TW, HIN>(x, s);
+    } else if constexpr (R == 4) {
+        radix4<SIGN>(x[0], x[1], x[2], x[3], seed(0), seed(1), seed(2));
+    } else if constexpr (R == 8) {
+        if constexpr (TW) {
+#pragma unroll
+            for (int r = 1; r < 8; ++r) {
+                const float2 w = seed(r - 1), v = x[r];
+                x[r] = make_float2(fmaf(w.x, v.x, -(w.y * v.y)), fmaf(w.x, v.y, w.y * v.x));
+            }
+        }
+        dft_pow2<8, SIGN, false, HIN>(x, nullptr);
+    } else {
+        // x[4 a + c]: over a, then over c with the twiddles w^c W_16^(c m)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if constexpr (TW) radix4<SIGN>(x[c], x[4 + c], x[8 + c], x[12 + c], seed(0), seed(1), seed(2));
+            else radix4_plain<SIGN, HIN>(x[c], x[4 + c], x[8 + c], x[12 + c]);
+        }
+        // slot 4 m + c now holds the m-th output of column c
+        float2 y[16];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            float2 c0 = x[4 * m], c1 = x[4 * m + 1], c2 = m < 2 ? x[4 * m + 2] : mul_si<SIGN>(x[4 * m + 2]), c3 = x[4 * m + 3];
+            if constexpr (TW) {
+                radix4<SIGN>(c0, c1, c2, c3, seed(3 + m), seed(7 + (m & 1)), seed(9 + m));
+            } else if (m == 0) {
+                radix4_plain<SIGN>(c0, c1, c2, c3);
+            } else {
+                // W_16^m, W_16^(2 m) (m odd: W_8, for m = 3 after the swap), W_16^(3 m)
+                const float2 w1 = make_float2(kCos8[m], SIGN * kSin8[m]);
+                const float2 w3 = m == 1 ? make_float2(kCos8[3], SIGN * kSin8[3])
+                                : m == 2 ? make_float2(-kCos8[2], SIGN * kSin8[2])
+                                         : make_float2(-kCos8[1], -SIGN * kSin8[1]);
+                if (m == 2) radix4<SIGN, true>(c0, c1, c2, c3, w1, w1, w3);
+                else radix4<SIGN>(c0, c1, c2, c3, w1, make_float2(kCos8[2], SIGN * kSin8[2]), w3);
+            }
+            y[m] = c0;
+            y[m + 4] = c1;
+            y[m + 8] = c2;
+            y[m + 12] = c3;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = y[i];
+    }
+}
+
+// A pass's butterfly of a line of N points.
+template <int N, int R, int SIGN, bool TW, bool HIN = false>
+__device__ __forceinline__ void dft_pass(float2 (&x)[R], const float2* s)
+{
+    if constexpr (direct_twiddles(N)) dft_direct<R, SIGN, TW, HIN>(x, s);
+    else dft_pow2<R, SIGN, TW, HIN>(x, s);
 }
 
 template <int R, int SIGN>
@@ -269,8 +378,9 @@ constexpr int fft_passes()
 }
 
 // One pass of fft<N,P>.  Twiddle seeds of a pass after the first (NS > 1, radix R): for each
-// butterfly b of a thread the R / 2 stage twiddles of dft_pow2 with w = exp(-2 pi i k / (NS R)),
-// k = (t + b T) mod NS: w^(R/S) W_S^m is the table entry N / (S NS) (k + m NS), below N / 2.
+// butterfly b of a thread the seeds of dft_pass with w = exp(-2 pi i k / (NS R)),
+// k = (t + b T) mod NS: w^(R/S) W_S^m is the table entry N / (S NS) (k + m NS), below N / 2;
+// w^e W_R^(e m) the entry e N / (R NS) (k + m NS), below N.
 template <int N, int P, int NS>
 struct FPass {
     static constexpr int T = N / P;
@@ -278,7 +388,7 @@ struct FPass {
     static constexpr int R = REM >= P ? P : REM;
     static constexpr int B = P / R;
     static constexpr bool LAST = (NS * R == N);
-    static constexpr int S = seed_count<R>();
+    static constexpr int S = seed_count<R, direct_twiddles(N)>();
     static constexpr int NTW = NS > 1 ? B * S : 1;  // twiddle seeds per thread (1: unused slot)
 };
 
@@ -286,12 +396,32 @@ struct FPass {
 template <int N, int NS, int R>
 __device__ __forceinline__ void pass_seeds(const float2* __restrict__ tw, uint32_t k, float2* s)
 {
+    const char* table = reinterpret_cast<const char*>(tw);
+    if constexpr (direct_twiddles(N)) {
+        auto entry = [&](int e, int m) {  // w^e W_R^(e m)
+            return *reinterpret_cast<const float2*>(table + k * (uint32_t)(8 * e * (N / (R * NS))) + 8 * e * m * (N / R));
+        };
+        if constexpr (R == 16) {
+#pragma unroll
+            for (int a = 1; a < 4; ++a) s[a - 1] = entry(4 * a, 0);
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                s[3 + m] = entry(1, m);
+                if (m < 2) s[7 + m] = entry(2, m);
+                s[9 + m] = entry(3, m);
+            }
+        } else {
+#pragma unroll
+            for (int r = 1; r < R; ++r) s[r - 1] = entry(r, 0);
+        }
+        return;
+    }
 #pragma unroll
     for (int S = 2; S <= R; S *= 2)
 #pragma unroll
         for (int m = 0; m < (S >= 4 ? S / 4 : 1); ++m)
-            s[seed_off(S) + m] = *reinterpret_cast<const float2*>(reinterpret_cast<const char*>(tw) +
-                                                                  k * (uint32_t)(8 * (N / (S * NS))) + 8 * m * (N / S));
+            s[seed_off(S) + m] =
+                *reinterpret_cast<const float2*>(table + k * (uint32_t)(8 * (N / (S * NS))) + 8 * m * (N / S));
 }
 
 // The seeds of pass NS.  Byte offsets from the wave-uniform table: one 32-bit offset register and an
@@ -376,8 +506,8 @@ __device__ __forceinline__ void fft_pass(float2 (&v)[P], float2* lds, const floa
         float2 x[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) x[r] = v[b + r * B];
-        if constexpr (NS > 1) dft_pow2<R, SIGN, true>(x, &w[b * S::S]);
-        else dft_pow2<R, SIGN, false, HIN>(x, nullptr);
+        if constexpr (NS > 1) dft_pass<N, R, SIGN, true>(x, &w[b * S::S]);
+        else dft_pass<N, R, SIGN, false, HIN>(x, nullptr);
         if constexpr (S::LAST) {
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + r * B] = x[r];
@@ -423,7 +553,7 @@ struct WPass {
     static constexpr int R = REM >= RMAX ? RMAX : REM;
     static constexpr int B = P / R;
     static constexpr bool LAST = (NS * R == N);
-    static constexpr int S = seed_count<R>();
+    static constexpr int S = seed_count<R, direct_twiddles(N)>();
     static constexpr int NTW = NS > 1 ? B * S : 1;  // twiddle seeds per lane (1: unused slot)
 };
 
@@ -492,8 +622,8 @@ __device__ __forceinline__ void wfft_pass(float2 (&v)[N / G], float2* buf, const
         float2 x[R];
 #pragma unroll
         for (int r = 0; r < R; ++r) x[r] = v[b + r * B];
-        if constexpr (NS > 1) dft_pow2<R, SIGN, true>(x, &w[b * S::S]);
-        else dft_pow2<R, SIGN, false, HIN>(x, nullptr);
+        if constexpr (NS > 1) dft_pass<N, R, SIGN, true>(x, &w[b * S::S]);
+        else dft_pass<N, R, SIGN, false, HIN>(x, nullptr);
         if constexpr (S::LAST) {
 #pragma unroll
             for (int r = 0; r < R; ++r) v[b + r * B] = x[r];
@@ -545,8 +675,8 @@ __device__ __forceinline__ void fft2_pass(float2 (&u)[P], float2 (&v)[P], float2
             float2 x[R];
 #pragma unroll
             for (int r = 0; r < R; ++r) x[r] = f[b + r * B];
-            if constexpr (NS > 1) dft_pow2<R, SIGN, true>(x, &w[b * S::S]);
-            else dft_pow2<R, SIGN, false, HIN>(x, nullptr);
+            if constexpr (NS > 1) dft_pass<N, R, SIGN, true>(x, &w[b * S::S]);
+            else dft_pass<N, R, SIGN, false, HIN>(x, nullptr);
             if constexpr (S::LAST) {
 #pragma unroll
                 for (int r = 0; r < R; ++r) f[b + r * B] = x[r];
