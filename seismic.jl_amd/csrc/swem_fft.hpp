@@ -716,10 +716,15 @@ __device__ __forceinline__ void fft2(float2 (&u)[P], float2 (&v)[P], float2* bu,
 // the pass; the points are then loaded back.  Each thread holds at most IT = ceil(P / R)
 // butterflies of a pass.  PP: two buffers alternated per pass (one barrier per pass), parity `pp`
 // carried as in fft; otherwise one buffer with a barrier between a pass's loads and its stores.
-// Twiddles: w = tw[k n / (NS R)] from the table tw[j] = exp(-2 pi i j / n), its powers by
+// Twiddles from the table tw[j] = exp(-2 pi i j / n).  Lengths of 2, 3 and 5: w = tw[k n / (NS R)], its powers by
 // products, w^r = w^h w^(r-h) with h the largest power of two below r (one load per butterfly:
 // seeds as in fft, four loads per radix-8 butterfly, measured slower here, 818 -> 943 ms for a
-// 250 x 250 3-D shot).  LDS indices are unpadded: the loads and the later passes' stores run at unit lane
+// 250 x 250 3-D shot).  With a radix 7, 11 or 13 (TABLE): every power is its own entry.  The products' rounding is
+// the same at every depth and adds up; those lengths ran Bluestein's identity before, which has no products of
+// entries, and the packed PSPI march at 700 points came out at 2.1e-5 of its image by products, 1.7e-6 by
+// entries and 1.4e-6 by Bluestein (split step: 1.07e-6, 8.1e-7, 2.7e-6).  It costs 3 to 40 % of the march (one
+// shot of 350 traces 377 -> 398 us, eight linear ones of 550 traces 2.85 -> 4.05 ms); Bluestein took 522 us and 12.1 ms.
+// LDS indices are unpadded: the loads and the later passes' stores run at unit lane
 // stride, the first pass's stores at stride R.
 
 // The seeds of dft_pow2 from w alone: w^(R/2) .. w by squares, the W_8 multiple by sums.
@@ -741,7 +746,7 @@ __device__ __forceinline__ void radix_seeds(float2 w, float2 (&s)[R / 2])
     }
 }
 
-template <int R, int SIGN, int IT, bool PP, class Sync>
+template <int R, int SIGN, int IT, bool PP, bool TABLE, class Sync>
 __device__ __forceinline__ void mixed_pass(const float2* src, float2* dst, const float2* __restrict__ tw, int n,
                                            int ns, int tws, uint32_t magic, int t, int T, Sync sync)
 {
@@ -754,18 +759,27 @@ __device__ __forceinline__ void mixed_pass(const float2* src, float2* dst, const
         if (i == 0 || b < nb) {
             const int k = ns > 1 ? b - (int)__umulhi((uint32_t)b, magic) * ns : 0;
             base[i] = (b - k) * R + k;
+            float2 pw[R];
+            if (TABLE && ns > 1) {
+#pragma unroll
+                for (int r = 1; r < R; ++r) {
+                    const float2 w = b < nb ? tw[r * k * tws] : make_float2(1.f, 0.f);
+                    pw[r] = SIGN > 0 ? cconj(w) : w;
+                }
+            }
             float2 w1 = make_float2(1.f, 0.f);
-            if (ns > 1 && b < nb) w1 = tw[k * tws];
+            if (!TABLE && ns > 1 && b < nb) w1 = tw[k * tws];
 #pragma unroll
             for (int r = 0; r < R; ++r) x[i][r] = b < nb ? src[b + r * nb] : make_float2(0.f, 0.f);
             if (ns > 1) {
-                float2 pw[R];
-                pw[1] = SIGN > 0 ? cconj(w1) : w1;
+                if constexpr (!TABLE) {
+                    pw[1] = SIGN > 0 ? cconj(w1) : w1;
 #pragma unroll
-                for (int r = 2; r < R; ++r) {
-                    int h = 1;
-                    while (2 * h < r) h *= 2;
-                    pw[r] = cmul(pw[h], pw[r - h]);
+                    for (int r = 2; r < R; ++r) {
+                        int h = 1;
+                        while (2 * h < r) h *= 2;
+                        pw[r] = cmul(pw[h], pw[r - h]);
+                    }
                 }
 #pragma unroll
                 for (int r = 1; r < R; ++r) x[i][r] = cmul(x[i][r], pw[r]);
@@ -806,19 +820,19 @@ __device__ __forceinline__ void mixed_fft(float2 (&v)[P], float2* buf0, float2* 
         const int r = mr.r[p];
         if constexpr (PRIME) {
             if (r == 7 || r > 8) {
-                if (r == 7) mixed_pass<7, SIGN, (P + 6) / 7, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
-                else if (r == 11) mixed_pass<11, SIGN, (P + 10) / 11, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
-                else mixed_pass<13, SIGN, (P + 12) / 13, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
+                if (r == 7) mixed_pass<7, SIGN, (P + 6) / 7, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
+                else if (r == 11) mixed_pass<11, SIGN, (P + 10) / 11, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
+                else mixed_pass<13, SIGN, (P + 12) / 13, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync);
                 cur = nxt;
                 continue;
             }
         }
         switch (r) {
-        case 8: mixed_pass<8, SIGN, (P + 7) / 8, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
-        case 4: mixed_pass<4, SIGN, (P + 3) / 4, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
-        case 2: mixed_pass<2, SIGN, (P + 1) / 2, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
-        case 3: mixed_pass<3, SIGN, (P + 2) / 3, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
-        default: mixed_pass<5, SIGN, (P + 4) / 5, PP>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
+        case 8: mixed_pass<8, SIGN, (P + 7) / 8, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
+        case 4: mixed_pass<4, SIGN, (P + 3) / 4, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
+        case 2: mixed_pass<2, SIGN, (P + 1) / 2, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
+        case 3: mixed_pass<3, SIGN, (P + 2) / 3, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
+        default: mixed_pass<5, SIGN, (P + 4) / 5, PP, PRIME>(cur, nxt, tw, n, ns, tws, mg, t, T, sync); break;
         }
         cur = nxt;
     }

@@ -6,6 +6,8 @@ A march repeats one transform with the same table entries at every depth, so the
 not.  A line of 256 points takes four radix-4 levels, hence at most one entry per level and input; its march
 may be no further from 64 bits than one of plain products and sums with those same entries.  What differs
 between the two is the rounding of the sums, which is a few per cent of the error of 200 depths: bound 1.05.
+The same holds for lengths with factors 7, 11 and 13, whose passes take one table entry per input, against
+the same butterflies with those entries.
 """
 import ctypes
 import os
@@ -56,24 +58,58 @@ def test_line(lib, n, p, sign, half):
     assert err <= np.sqrt(3 * np.log2(n)) * 2.0 ** -24
 
 
-@pytest.mark.parametrize("p", [4, 8, 16])
-def test_march_error_of_256_points(lib, p):
-    n, steps = 256, 200
-    mine, plain = 0.0, 0.0
-    for s in range(12):
-        k = np.minimum(np.arange(n), n - np.arange(n))
-        a = 1.0 - (k / ((0.2 + 0.02 * s) * n)) ** 2
-        phase = np.where(a > 0, np.exp(1j * (3 + 0.5 * s) * np.sqrt(np.abs(a))), np.exp(-1.2 * np.sqrt(np.abs(a)))) / n
-        z = np.zeros(n, complex)
-        z[n // 8 + s * n // 40] = 1 + 0.3j
+def _case(n, s):
+    """(phase of a step, start) of the s-th medium"""
+    k = np.minimum(np.arange(n), n - np.arange(n))
+    a = 1.0 - (k / ((0.2 + 0.02 * s) * n)) ** 2
+    phase = np.where(a > 0, np.exp(1j * (3 + 0.5 * s) * np.sqrt(np.abs(a))), np.exp(-1.2 * np.sqrt(np.abs(a)))) / n
+    z = np.zeros(n, complex)
+    z[n // 8 + s * n // 40] = 1 + 0.3j
+    return phase, z
+
+
+def _errors(n, steps, media, run):
+    """mean errors of run(0, ...) and run(1, ...) over some media"""
+    e = np.zeros(2)
+    for s in range(media):
+        phase, z = _case(n, s)
         ph, x = _floats(phase), [_floats(z), _floats(z)]
         z = x[0].astype(np.float64) @ [1, 1j]
         for _ in range(steps):
             z = np.fft.ifft(np.fft.fft(z) * phase) * n
             z[n // 2:] = 0
-        assert lib.fft_march_256(p, _ptr(x[0]), _ptr(ph), steps) == 0
-        assert lib.fft_march_256(0, _ptr(x[1]), _ptr(ph), steps) == 0
-        e = [np.linalg.norm(v.astype(np.float64) @ [1, 1j] - z) / np.linalg.norm(z) for v in x]
-        mine, plain = mine + e[0] / 12, plain + e[1] / 12
+        for i in (0, 1):
+            assert run(i, _ptr(x[i]), _ptr(ph), steps) == 0
+            e[i] += np.linalg.norm(x[i].astype(np.float64) @ [1, 1j] - z) / np.linalg.norm(z) / media
+    return e
+
+
+@pytest.mark.parametrize("p", [4, 8, 16])
+def test_march_error_of_256_points(lib, p):
+    mine, plain = _errors(256, 200, 12, lambda i, x, ph, n: lib.fft_march_256(0 if i else p, x, ph, n))
     print(f"{p} points per thread: {mine:.2e}, plain {plain:.2e}")
     assert mine <= 1.05 * plain
+
+
+@pytest.mark.parametrize("n", [91, 140, 700, 1014, 2002])
+def test_march_error_with_prime_factors(lib, n):
+    mine, plain = _errors(n, 60, 4, lambda i, x, ph, k: lib.mixed_march(n, i, x, ph, k, 0))
+    print(f"{n} points: {mine:.2e}, plain {plain:.2e}")
+    assert mine <= 1.05 * plain
+
+
+@pytest.mark.parametrize("sign", [-1, 1])
+@pytest.mark.parametrize("n", [7, 91, 100, 121, 160, 700, 1014, 2000, 2002])
+def test_mixed_line(lib, n, sign):
+    rng = np.random.default_rng(n)
+    x = _floats(rng.standard_normal(n) + 1j * rng.standard_normal(n))
+    ref = x.astype(np.float64) @ [1, 1j]
+    ref = np.fft.fft(ref) if sign < 0 else np.fft.ifft(ref) * n
+    assert lib.mixed_march(n, 0, _ptr(x), None, 0, sign) == 0
+    err = np.linalg.norm(x.astype(np.float64) @ [1, 1j] - ref) / np.linalg.norm(ref)
+    # as above, a butterfly of radix r counted as the r sums of its definition
+    r, k = 0, n
+    for q in (13, 11, 7, 5, 3, 2):
+        while k % q == 0:
+            r, k = r + q, k // q
+    assert err <= np.sqrt(3 * r) * 2.0 ** -24
