@@ -139,8 +139,9 @@ struct HeldSeeds<N, P, true, kSeedHeld> {
     __device__ __forceinline__ const float2* ptr() const { return s.w; }
 };
 
-template <int N, int P, bool WAVE_ = false, int SEED = kSeedAhead>
+template <int N, int P, bool WAVE_ = false, int SEED = kSeedAhead, bool AHEAD = true>
 struct XPow2 {
+    static constexpr bool kAhead = AHEAD, kPow2 = true;
     HeldSeeds<N, P, WAVE_, SEED> held;
     __device__ __forceinline__ XPow2(const March2DArgs& a, int t) : held(a.tw, t) {}
     // HIN: slots q >= P/2 are zero on input (see fft)
@@ -162,6 +163,7 @@ struct XPow2 {
 
 template <int M, int P>
 struct XBlue {
+    static constexpr bool kAhead = true, kPow2 = false;
     static constexpr int T = M / P;
     uint32_t koff[P];  // byte offsets of the thread's points in a kz row (0 beyond n)
     __device__ __forceinline__ XBlue(const March2DArgs& a, int t)
@@ -217,8 +219,9 @@ struct XBlue {
 
 // XMixed: a mixed-radix length n = nkx (PRIME: with factors 7, 11, 13) in the power-of-two array of M >= n points,
 // transformed in the subgroup's two LDS buffers (mixed_fft); entries j >= n stay zero.
-template <int M, int P, bool PRIME = false>
+template <int M, int P, bool PRIME = false, bool AHEAD = true>
 struct XMixed {
+    static constexpr bool kAhead = AHEAD, kPow2 = false;
     XBlue<M, P> b;  // the kz row offsets
     __device__ __forceinline__ XMixed(const March2DArgs& a, int t) : b(a, t) {}
     template <int SIGN, bool WAVE, bool HIN = false>
@@ -295,18 +298,20 @@ __device__ __forceinline__ void ssf_adj_step(float2 (&u)[P], float2* lds, int& p
 {
     constexpr int T = N / P, Q = HALF ? P / 2 : P;
     float2 L[P], sp[Q];
-    if constexpr (ACT) xf.kload_row(L, krow(a, c, 0), a, c.t);
+    if constexpr (ACT && X::kAhead) xf.kload_row(L, krow(a, c, 0), a, c.t);
     xf.template fft<-1, WAVE, HALF>(u, lds, a, c.t, pp);
     if constexpr (ACT) {
+        if constexpr (!X::kAhead) xf.kload_row(L, krow(a, c, 0), a, c.t);
 #pragma unroll
         for (int q = 0; q < P; ++q) u[q] = cmul_c(u[q], L[q], conj);
-        ss_load<T, Q>(sp, a, c);
+        if constexpr (X::kAhead) ss_load<T, Q>(sp, a, c);
     } else {
 #pragma unroll
         for (int q = 0; q < P; ++q) u[q] = cscale(u[q], a.inv_nk);
     }
     xf.template fft<+1, WAVE>(u, lds, a, c.t, pp);
     if constexpr (ACT) {
+        if constexpr (!X::kAhead) ss_load<T, Q>(sp, a, c);
 #pragma unroll
         for (int q = 0; q < Q; ++q) u[q] = cmul_c(u[q], sp[q], conj);
     } else {
@@ -360,34 +365,39 @@ __device__ __forceinline__ void pspi_select_step(float2 (&u)[P], float2* lds, in
     constexpr int T = N / P, Q = HALF ? P / 2 : P;
     uint32_t todo = a.used[c.iz] & ((1u << a.nref) - 1u);
     const int first = __builtin_ctz(todo | 0x80000000u);
-    // each vref's row is read while the transform before its use runs
+    // each vref's row is read while the transform before its use runs (kAhead)
     float2 L[P];
     auto next_row = [&]() {
         if (ACT && todo) xf.kload_row(L, krow(a, c, __builtin_ctz(todo)), a, c.t);
     };
-    next_row();
+    if constexpr (X::kAhead) next_row();
     float2 U[Q];
     uint8_t s1[Q], s2[Q];
     float w2[Q];
-    const size_t rowx = (size_t)c.iz * N;
+    auto selection = [&]() {
+        const size_t rowx = (size_t)c.iz * N;
 #pragma unroll
-    for (int q = 0; q < Q; ++q) {
-        const int x = c.t + q * T;
-        s1[q] = a.sel[rowx + x];
-        if constexpr (MODE == kModePspiLinear) {
-            s2[q] = a.sel2[rowx + x];
-            w2[q] = a.w2[rowx + x];
+        for (int q = 0; q < Q; ++q) {
+            const int x = c.t + q * T;
+            s1[q] = a.sel[rowx + x];
+            if constexpr (MODE == kModePspiLinear) {
+                s2[q] = a.sel2[rowx + x];
+                w2[q] = a.w2[rowx + x];
+            }
+            U[q] = make_float2(0.f, 0.f);
         }
-        U[q] = make_float2(0.f, 0.f);
-    }
+    };
+    if constexpr (X::kAhead) selection();
     xf.template fft<-1, WAVE, HALF>(u, lds, a, c.t, pp);
+    if constexpr (!X::kAhead) selection();
     while (todo) {
         const int ir = __builtin_ctz(todo);
+        if constexpr (!X::kAhead) next_row();
         todo &= todo - 1u;
         float2 B[P];
 #pragma unroll
         for (int q = 0; q < P; ++q) B[q] = ACT ? cmul_c(u[q], L[q], conj) : cscale(u[q], a.inv_nk);
-        next_row();
+        if constexpr (X::kAhead) next_row();
         xf.template fft<+1, WAVE>(B, lds, a, c.t, pp);
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
@@ -429,11 +439,12 @@ __device__ __forceinline__ void pspi_weight_step(float2 (&u)[P], float2* lds, in
     for (uint32_t todo = a.used[c.iz] & ((1u << a.nref) - 1u); todo; todo &= todo - 1u) {
         const int ir = __builtin_ctz(todo);
         float2 L[P], B[P];
-        xf.kload_row(L, krow(a, c, ir), a, c.t);
+        if constexpr (X::kAhead) xf.kload_row(L, krow(a, c, ir), a, c.t);
 #pragma unroll
         for (int q = 0; q < Q; ++q) B[q] = cscale(u[q], pspi_linear_weight(ir, s1[q], s2[q], w2[q]));
         zero_tail<P, Q>(B);
         xf.template fft<-1, WAVE, HALF>(B, lds, a, c.t, pp);
+        if constexpr (!X::kAhead) xf.kload_row(L, krow(a, c, ir), a, c.t);
 #pragma unroll
         for (int q = 0; q < P; ++q) {
             acc[q].x = fmaf(B[q].x, L[q].x, fmaf(B[q].y, L[q].y, acc[q].x));
@@ -557,7 +568,7 @@ __device__ __forceinline__ void adj_body(const March2DArgs& a)
 
 // Modelling march: NSUB subgroups, one frequency each, no interaction between subgroups.
 //
-// The receiver's depth reads (stored source, image, split-step phases) are issued one depth ahead:
+// The receiver's depth reads (stored source, image, split-step phases) are issued one depth ahead (kAhead):
 // they come from HBM and would otherwise be waited for at the start of every step.
 template <int N, int P, int MODE, bool WAVE, bool HALF, class X = XPow2<N, P, WAVE>>
 __device__ __forceinline__ void fwd_body(const March2DArgs& a)
@@ -633,26 +644,28 @@ __device__ __forceinline__ void fwd_body(const March2DArgs& a)
     auto stepped = [&](int iz) { return a.oz + a.dz * (float)iz >= a.gz; };
     int iz = a.nz - 1;
     while (iz >= 0 && !stepped(iz)) --iz;
-    if (iz >= 0) fetch(iz);
+    if (X::kAhead && iz >= 0) fetch(iz);
     while (iz >= 0) {
         int next = iz - 1;
         while (next >= 0 && !stepped(next)) --next;
+        if constexpr (!X::kAhead) fetch(iz);
 #pragma unroll
         for (int q = 0; q < Q; ++q) u[q] = make_float2(fmaf(sv[q].x, mv[q], u[q].x), fmaf(sv[q].y, mv[q], u[q].y));
         if constexpr (MODE == kModeSSF) {
             float2 L1[P];
             c.iz = iz;
-            xf.kload_row(L1, krow(a, c, 0), a, t);
+            if constexpr (X::kAhead) xf.kload_row(L1, krow(a, c, 0), a, t);
 #pragma unroll
             for (int q = 0; q < Q; ++q) u[q] = cmulc(u[q], sp[q]);
-            if (next >= 0) fetch(next);
+            if (X::kAhead && next >= 0) fetch(next);
             xf.template fft<-1, WAVE, HALF>(u, lds, a, t, pp);
+            if constexpr (!X::kAhead) xf.kload_row(L1, krow(a, c, 0), a, t);
 #pragma unroll
             for (int q = 0; q < P; ++q) u[q] = cmulc(u[q], L1[q]);
             xf.template fft<+1, WAVE>(u, lds, a, t, pp);
             zero_tail<P, Q>(u);  // within the live slots the next split-step row cuts at nmx
         } else {
-            if (next >= 0) fetch(next);
+            if (X::kAhead && next >= 0) fetch(next);
             c.iz = iz;
             if constexpr (MODE == kModePspiCompat)
                 pspi_select_step<N, P, MODE, WAVE, true, HALF, X>(u, lds, pp, a, xf, c, true);
@@ -840,7 +853,7 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
     constexpr int Q = HALF ? P / 2 : P;  // live slots
     constexpr int K = kUncutSparse;
     constexpr int NW = T / 64;  // waves of the subgroup
-    constexpr bool POW2 = std::is_same<X, XPow2<N, P, WAVE, kSeedHeld>>::value;
+    constexpr bool POW2 = X::kPow2;
     // Bluestein lengths: the table tw is of the array length, not of nkx, so no direct sums (the
     // uncut points' e and output always come from transforms)
     constexpr bool BLUE = std::is_same<X, XBlue<N, P>>::value;
@@ -921,15 +934,18 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
         uint32_t todo = a.used[iz] & ((1u << a.nref) - 1u);
         if (direct_cr) todo &= ~(1u << cr);
         // the rows of the depth in turn: those of todo, then cr's for the uncut points; each is
-        // read while the transform before its use runs
+        // read while the transform before its use runs (kAhead)
         float2 Lr[P];
         auto next_row = [&](uint32_t left) {
             if (left || cnt > 0) xf.kload_row(Lr, krow(a, c, left ? __builtin_ctz(left) : cr), a, t);
         };
-        next_row(todo);
+        if constexpr (X::kAhead) next_row(todo);
         uint32_t s1[Q];
+        auto selection = [&]() {
 #pragma unroll
-        for (int q = 0; q < Q; ++q) s1[q] = a.sel[(size_t)iz * N + t + q * T];
+            for (int q = 0; q < Q; ++q) s1[q] = a.sel[(size_t)iz * N + t + q * T];
+        };
+        if constexpr (X::kAhead) selection();
         // HALF: slots q >= P/2 of z and e are zero (x >= N/2 >= nmx is never selected)
         xf.template fft<-1, WAVE, HALF>(z, smem, a, t, pp);
         if (prev_cnt < 0 || prev_cnt > (BLUE ? 0 : K)) {
@@ -966,11 +982,13 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
             w0 = twid(t * crow[3]);
             st = twid(T * crow[3]);
         }
+        if constexpr (!X::kAhead) selection();
         float2 out[Q];
 #pragma unroll
         for (int q = 0; q < Q; ++q) out[q] = make_float2(0.f, 0.f);
         while (todo) {
             const uint32_t ir = (uint32_t)__builtin_ctz(todo);
+            if constexpr (!X::kAhead) next_row(todo);
             todo &= todo - 1u;
             float2 w[P];
 #pragma unroll
@@ -978,12 +996,13 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
                 const float2 L = Lr[q];
                 w[q] = make_float2(z[q].x * L.x + e[q].x * L.y, z[q].y * L.x + e[q].y * L.y);
             }
-            next_row(todo);
+            if constexpr (X::kAhead) next_row(todo);
             xf.template fft<+1, WAVE>(w, smem, a, t, pp);
 #pragma unroll
             for (int q = 0; q < Q; ++q)
                 if ((s1[q] & 0x7fu) == ir) out[q] = w[q];
         }
+        if constexpr (!X::kAhead) next_row(0);
         float2 en[Q];  // the new e
 #pragma unroll
         for (int q = 0; q < Q; ++q) en[q] = make_float2(0.f, 0.f);
@@ -1116,10 +1135,27 @@ __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
     }
 }
 
+#define SWEM_SUBGROUP_BOUNDS(P) __launch_bounds__((P) == 16 ? 512 : kMaxBlock)
+
+// Where the marches keep their twiddle seeds, and whether they read rows, selections and the stored source
+// ahead of their use.  Seeds held in registers drop the table loads and address arithmetic of every transform;
+// the half-line kernels have the registers for it, the general form at 16 points per thread spills
+// and so does the 128-register budget of the large workgroups with 8.  Read ahead -> held, 8 shots x 100 depths,
+// 1024 / 512 traces, and 16 shots of 256: split-step modelling 4.9 -> 3.8, 2.3 -> 1.8, 2.5 -> 1.6 ms; PSPI modelling
+// 10.9 -> 9.2, 5.1 -> 4.2, 5.4 -> 4.0; linear modelling 11.5 -> 10.1, 5.3 -> 4.6, 5.5 -> 4.3; linear migration 11.3 ->
+// 9.9, 5.3 -> 4.7, 5.9 -> 4.7.  Two vrefs of a PSPI step in lockstep on top spill (188 bytes): 76 -> 81 ms
+// where held alone gives 63.
+// The read-ahead needs 16 to 80 registers more.  The general lines at 16 points per thread (and 8 in the large
+// workgroups) read at the use and step the two wavefields in turn: 16 shots x 20 depths of 4096 points (pad
+// factor 1), ahead -> at the use: split-step migration 4.1 -> 3.0 ms, modelling 5.0 -> 3.2, linear migration 12.3 -> 7.6,
+// linear modelling 11.1 -> 6.8.  So do the mixed-radix marches but the half-line migration and split-step
+// modelling, whose workgroups would lose a wave per SIMD: 8 shots x 20 depths, nkx 3000, PSPI modelling 8.4 -> 5.1 ms.
+constexpr int held_if(bool fits) { return fits ? kSeedHeld : kSeedAhead; }
+
 template <int N, int P, bool HALF>
 __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_packed(March2DArgs a)
 {
-    adj_body_packed<N, P, false, HALF>(a);
+    adj_body_packed<N, P, false, HALF, XPow2<N, P, false, held_if(HALF), HALF>>(a);
 }
 
 template <int N, bool HALF>
@@ -1141,37 +1177,28 @@ __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void
     adj_body_packed<M, P, false, HALF, XBlue<M, P>>(a);
 }
 
-#define SWEM_SUBGROUP_BOUNDS(P) __launch_bounds__((P) == 16 ? 512 : kMaxBlock)
-
-// Where the marches of one wavefield per thread keep their twiddle seeds.  Held in registers they drop the
-// table loads and address arithmetic of every transform; the half-line kernels have the registers for it,
-// the general form at 16 points per thread spills (288 to 388 bytes) and so does the 128-register budget
-// of the large workgroups with 8.  Read ahead -> held, 8 shots x 100 depths, 1024 / 512 traces, and 16
-// shots of 256: split-step modelling 4.9 -> 3.8, 2.3 -> 1.8, 2.5 -> 1.6 ms; PSPI modelling 10.9 -> 9.2,
-// 5.1 -> 4.2, 5.4 -> 4.0; linear modelling 11.5 -> 10.1, 5.3 -> 4.6, 5.5 -> 4.3; linear migration 11.3 ->
-// 9.9, 5.3 -> 4.7, 5.9 -> 4.7.  Two vrefs of a PSPI step in lockstep on top spill (188 bytes): 76 -> 81 ms
-// where held alone gives 63.
-constexpr int held_if(bool fits) { return fits ? kSeedHeld : kSeedAhead; }
-
 template <int N, int MODE, int P>
-__global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_adj(March2DArgs a) { adj_body<N, P, MODE, false>(a); }
+__global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_adj(March2DArgs a)
+{
+    adj_body<N, P, MODE, false, XPow2<N, P, false, P < 16 ? kSeedAhead : kSeedPass, P < 8>>(a);
+}
 
 template <int N, int MODE, int P, bool HALF>
 __global__ SWEM_SUBGROUP_BOUNDS(P) void march2d_fwd(March2DArgs a)
 {
-    fwd_body<N, P, MODE, false, HALF, XPow2<N, P, false, held_if(HALF && P == 16)>>(a);
+    fwd_body<N, P, MODE, false, HALF, XPow2<N, P, false, held_if(HALF && P == 16), HALF || P < 8>>(a);
 }
 
 template <int N, int MODE>
 __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_w(March2DArgs a)
 {
-    adj_body<N, N / 64, MODE, true>(a);
+    adj_body<N, N / 64, MODE, true, XPow2<N, N / 64, true, kSeedAhead, N < 1024>>(a);
 }
 
 template <int N, int MODE, bool HALF>
 __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_w(March2DArgs a)
 {
-    fwd_body<N, N / 64, MODE, true, HALF, XPow2<N, N / 64, true, held_if(HALF && N <= 1024)>>(a);
+    fwd_body<N, N / 64, MODE, true, HALF, XPow2<N, N / 64, true, held_if(HALF && N <= 1024), HALF || N < 1024>>(a);
 }
 
 // PAIR: 16 points per thread from nkx = 1024 (nkx/16 threads, radix-16 passes), one wave with
@@ -1179,7 +1206,8 @@ __global__ __launch_bounds__(kWaveBlock) __attribute__((amdgpu_waves_per_eu(2)))
 template <int N, int MODE, int P, bool HALF>
 __global__ __launch_bounds__(N / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_pair(March2DArgs a)
 {
-    adj_body_pair<N, P, MODE, false, HALF, XPow2<N, P, false, held_if(HALF || MODE == kModeSSF)>>(a);
+    adj_body_pair<N, P, MODE, false, HALF,
+                  XPow2<N, P, false, held_if(HALF || (MODE == kModeSSF && P < 16)), HALF || P < 16>>(a);
 }
 
 template <int N, int MODE, bool HALF>
@@ -1207,13 +1235,13 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void m
 template <int M, int MODE, int P, bool HALF, bool PRIME>
 __global__ __launch_bounds__(M / P) __attribute__((amdgpu_waves_per_eu(2))) void march2d_adj_mixed(March2DArgs a)
 {
-    adj_body_pair<M, P, MODE, false, HALF, XMixed<M, P, PRIME>>(a);
+    adj_body_pair<M, P, MODE, false, HALF, XMixed<M, P, PRIME, HALF>>(a);
 }
 
 template <int M, int MODE, int P, bool HALF, bool PRIME>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void march2d_fwd_mixed(March2DArgs a)
 {
-    fwd_body<M, P, MODE, false, HALF, XMixed<M, P, PRIME>>(a);
+    fwd_body<M, P, MODE, false, HALF, XMixed<M, P, PRIME, HALF && MODE == kModeSSF>>(a);
 }
 
 // ------------------------------------------------------------------ launches of one array length
