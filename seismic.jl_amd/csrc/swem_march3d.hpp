@@ -535,9 +535,11 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
 // x-pass of the linear-mode modelling receiver (the transpose of march3d_cols_pspi): for every
 // vref in use at the depth, the slice R[ir] (the weighted wavefield, y transformed) is x
 // transformed and multiplied by its kz phase (conj for the -dz step), the products are summed,
-// and one inverse x-FFT gives the stepped receiver (y transformed) in the state.
+// and one inverse x-FFT gives the stepped receiver (y transformed) in the state.  16 points per lane, their sums
+// and seeds take 207 to 256 registers: two waves per SIMD (at four, 126 spilled registers; 128 x 128 x 10
+// linear modelling, pad factor 2, 3.4 -> 2.3 ms).
 template <int NX, int C, int BX, int PREC>
-__global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 512 ? 2 : 4))) void march3d_cols_gather(
+__global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_waves_per_eu(NX >= 512 || line_lanes(NX, BX) * 16 == NX ? 2 : 4))) void march3d_cols_gather(
     March3DArgs a)
 {
     constexpr int G = Line<NX, BX>::G, P = Line<NX, BX>::P;

@@ -52,3 +52,11 @@ def test_mixed_radix_waves(n, tmp_path):
         assert k[name][0] <= 128 and k[name][1] == 0, (name, k[name])
     for name in (f"march2d_adj_mixed<{n}, 2, 8, false, false>", f"march2d_fwd_mixed<{n}, 2, 8, false, false>"):
         assert k[name][0] <= 168 and k[name][1] == 0, (name, k[name])
+
+
+@pytest.mark.parametrize("n,c", [(128, 32), (256, 16)])
+def test_linear_x_pass_does_not_spill(n, c, tmp_path):
+    k = kernels(f"swem_march3d_{n}.o", str(tmp_path))
+    for prec in (0, 1):
+        name = f"march3d_cols_gather<{n}, {c}, 0, {prec}>"
+        assert k[name][1] == 0, (name, k[name])
