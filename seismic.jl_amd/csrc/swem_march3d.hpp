@@ -491,18 +491,23 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
         const double p2 = a.p2[(size_t)a.iz * a.nref + ir];
         const float p2f = a.p2f[(size_t)a.iz * a.nref + ir];
         const double c0 = wd * wd * p2 - ky * ky;
-        // the two wavefields of a migration share each phase (the one-wavefield shapes keep
-        // computing it per point: the mirrored set would spill there)
+        // the two wavefields of a migration share each phase, in FP32 too (its square root, sine and cosine are
+        // half of the pass: 128 x 128 x 10 shot 3.9 -> 2.6 ms); the one-wavefield shapes keep computing it per
+        // point: the set would spill there
         float2 phm[P];
-        const bool mirror = NWF == 2 && BX == kLenPow2 && PREC == SWEM_PREC_KZ64;
-        if constexpr (NWF == 2 && BX == kLenPow2)
-            if (mirror) kz_phases64_col<NX>(a, c0, t, phm);
+        constexpr bool shared = NWF == 2 && BX == kLenPow2;
+        if constexpr (shared && PREC == SWEM_PREC_KZ64) {
+            kz_phases64_col<NX>(a, c0, t, phm);
+        } else if constexpr (shared) {
+#pragma unroll
+            for (int q = 0; q < P; ++q) phm[q] = kz_phase(a, wd, p2, p2f, t + G * q, iky);
+        }
 #pragma unroll
         for (int k = 0; k < NWF; ++k) {
             float2 bq[P];
 #pragma unroll
             for (int q = 0; q < P; ++q) {
-                const float2 ph = mirror ? phm[q]
+                const float2 ph = shared ? phm[q]
                                   : PREC == SWEM_PREC_KZ64 ? kz_phase64(a, c0, t + G * q)
                                                              : kz_phase(a, wd, p2, p2f, t + G * q, iky);
                 bq[q] = cmul(v[k][q], make_float2(ph.x, cj[k] ? -ph.y : ph.y));
