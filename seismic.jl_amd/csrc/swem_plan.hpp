@@ -3,6 +3,7 @@
 #pragma once
 #include <cstddef>
 #include <cstdint>
+#include <utility>
 #include <vector>
 
 #include "swem_internal.hpp"
@@ -56,11 +57,24 @@ extern thread_local HostStager* tl_stager;
 
 int upload_bytes(void* dev, const void* host, size_t bytes);
 
+// Device memory of one owner: freed with it (by hipFree, which waits for the device, or back to the
+// allocator it came from, which must outlive it).
 template <typename T>
 struct DevBuf {
     T* p = nullptr;
     size_t n = 0;
     DevAllocator* from = nullptr;
+    DevBuf() = default;
+    ~DevBuf() { release(); }
+    DevBuf(DevBuf&& o) noexcept { *this = std::move(o); }
+    DevBuf& operator=(DevBuf&& o) noexcept
+    {
+        std::swap(p, o.p);
+        std::swap(n, o.n);
+        std::swap(from, o.from);
+        o.release();
+        return *this;
+    }
     int alloc(size_t count)
     {
         if (count <= n && p) return SWEM_OK;

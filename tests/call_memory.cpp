@@ -1,0 +1,121 @@
+// Device memory of plans and one-call entry points (swem_plan.hpp, swem_pool.cpp) over a device made of
+// counters: hipMalloc hands out host addresses against a set capacity.  One scenario per run
+// (test_call_memory.py); exit status 0 where it holds.
+#include <cstdarg>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <string>
+
+#include "swem_plan.hpp"
+
+// ------------------------------------------------------------------ the device
+static size_t g_capacity = size_t(100) << 30, g_used = 0, g_mallocs = 0, g_syncs = 0;
+static int g_device = 0;
+static std::map<void*, std::pair<size_t, int>> g_live;  // bytes and device
+
+extern "C" {
+hipError_t hipMalloc(void** p, size_t n)
+{
+    g_mallocs++;
+    if (g_used + n > g_capacity) return hipErrorOutOfMemory;
+    *p = std::malloc(1);
+    g_live[*p] = {n, g_device};
+    g_used += n;
+    return hipSuccess;
+}
+hipError_t hipFree(void* p)
+{
+    auto it = g_live.find(p);
+    if (it == g_live.end()) std::abort();
+    g_used -= it->second.first;
+    g_live.erase(it);
+    std::free(p);
+    return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) { return *d = g_device, hipSuccess; }
+hipError_t hipSetDevice(int d) { return g_device = d, hipSuccess; }
+hipError_t hipDeviceSynchronize(void) { return g_syncs++, hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+hipError_t hipMemGetInfo(size_t* fr, size_t* tot) { return *fr = g_capacity - g_used, *tot = g_capacity, hipSuccess; }
+const char* hipGetErrorString(hipError_t) { return "device error"; }
+}
+
+namespace swem {
+thread_local DevAllocator* tl_dev_alloc = nullptr;
+thread_local HostStager* tl_stager = nullptr;
+int set_error(int code, const char*, ...) { return code; }
+int hip_error(hipError_t e, const char*, const char*, int) { return e == hipErrorOutOfMemory ? SWEM_ENOMEM : SWEM_EDEVICE; }
+int upload_bytes(void*, const void*, size_t) { return SWEM_OK; }
+}  // namespace swem
+
+using namespace swem;
+constexpr size_t GiB = size_t(1) << 30, MiB = size_t(1) << 20;
+
+#define EXPECT(x)                                                             \
+    do {                                                                      \
+        if (!(x)) return std::printf("line %d: %s\n", __LINE__, #x), 1;       \
+    } while (0)
+
+// a call that takes the given sizes at once
+template <class... S>
+static int call(int device, S... bytes)
+{
+    CallMemory memory(device);
+    DevBuf<char> b[sizeof...(bytes)];
+    const size_t n[] = {(size_t)bytes...};
+    for (size_t i = 0; i < sizeof...(bytes); i++) SWEM_TRY(b[i].alloc(n[i]));
+    return SWEM_OK;
+}
+
+static int reuse()
+{
+    EXPECT(call(0, 3 * GiB, 70 * MiB) == SWEM_OK);
+    const size_t first = g_mallocs;
+    EXPECT(call(0, 3 * GiB - 5, 70 * MiB) == SWEM_OK && g_mallocs == first);  // the same blocks
+    EXPECT(call(0, GiB) == SWEM_OK && g_mallocs == first + 1);                // not a block three times as large
+    EXPECT(g_used == 4 * GiB + 70 * MiB && g_syncs == 3);
+    return 0;
+}
+
+static int bounds()
+{
+    EXPECT(call(0, 9 * GiB, 9 * GiB) == SWEM_OK && g_used == 9 * GiB);  // at most 16 GiB stay
+    for (int i = 0; i < 4; i++) EXPECT(call(0, 2 * GiB) == SWEM_OK && g_used == 11 * GiB);
+    EXPECT(call(0, 2 * GiB) == SWEM_OK && g_used == 2 * GiB);  // unused by the last four calls
+    return 0;
+}
+
+static int given_back()
+{
+    EXPECT(call(0, 5 * GiB) == SWEM_OK && g_used == 5 * GiB);
+    EXPECT(call(1, 3 * GiB) == SWEM_OK && g_used == 8 * GiB);
+    trim_call_memory(0);
+    EXPECT(g_used == 3 * GiB);
+    trim_call_memory(1);
+    EXPECT(g_used == 0 && g_live.empty());
+    return 0;
+}
+
+static int buffers_free_themselves()
+{
+    {
+        DevBuf<char> a, b;
+        EXPECT(a.alloc(MiB) == SWEM_OK && b.alloc(2 * MiB) == SWEM_OK && g_used == 3 * MiB);
+        DevBuf<char> c(std::move(a));
+        EXPECT(!a.p && c.p && c.n == MiB);
+        b = std::move(c);
+        EXPECT(g_used == MiB && b.n == MiB && !c.p);
+    }
+    EXPECT(g_used == 0 && g_live.empty());
+    return 0;
+}
+
+int main(int, char** argv)
+{
+    const std::map<std::string, int (*)()> all = {
+        {"reuse", reuse}, {"bounds", bounds}, {"given_back", given_back},
+        {"buffers_free_themselves", buffers_free_themselves}};
+    return all.at(argv[1])();
+}
