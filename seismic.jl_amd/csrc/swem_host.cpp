@@ -1365,8 +1365,8 @@ struct TuneBuffers {
     int init(const swem_plan* p, int nshot)
     {
         const size_t nm = p->nm, nt = p->g.nt, nz = p->g.nz;
-        SWEM_HIP(hipMalloc((void**)&d, (size_t)nshot * nm * nt * sizeof(float)));
-        SWEM_HIP(hipMalloc((void**)&m, nm * nz * sizeof(float)));
+        SWEM_HIP(device_malloc((void**)&d, (size_t)nshot * nm * nt * sizeof(float)));
+        SWEM_HIP(device_malloc((void**)&m, nm * nz * sizeof(float)));
         if (p->three_d) {
             SWEM_HIP(hipMemset(d, 0, (size_t)nshot * nm * nt * sizeof(float)));
         } else {
@@ -2245,14 +2245,7 @@ int swem_ewem(float* ux, float* uy, float* uz, float* mpp, float* mps1, float* m
 int swem_malloc(void** ptr, size_t bytes)
 {
     if (!ptr) return set_error(SWEM_EINVAL, "null pointer");
-    hipError_t e = hipMalloc(ptr, bytes);
-    if (e == hipErrorOutOfMemory) {  // what the one-call entry points keep is given back first
-        (void)hipGetLastError();
-        int dev = 0;
-        if (hipGetDevice(&dev) == hipSuccess) trim_call_memory(dev);
-        e = hipMalloc(ptr, bytes);
-    }
-    if (e != hipSuccess) return hip_error(e, "hipMalloc(ptr, bytes)", __FILE__, __LINE__);
+    SWEM_HIP(device_malloc(ptr, bytes));
     return SWEM_OK;
 }
 
@@ -2304,7 +2297,7 @@ int swem_vec_dot(const float* x, const float* y, size_t n, double* out, void* st
     SWEM_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) return set_error(SWEM_EDEVICE, "vec_dot: device %d", dev);
     if (!scratch[dev]) {
-        SWEM_HIP(hipMalloc((void**)&scratch[dev], sizeof(double) * vec_dot_scratch_doubles()));
+        SWEM_HIP(device_malloc((void**)&scratch[dev], sizeof(double) * vec_dot_scratch_doubles()));
         SWEM_HIP(hipHostMalloc((void**)&host[dev], sizeof(double), hipHostMallocDefault));
     }
     hipStream_t st = (hipStream_t)stream;

@@ -50,6 +50,8 @@ private:
 };
 // Frees the blocks kept for a device.
 void trim_call_memory(int dev);
+// hipMalloc on the current device; when it is out of memory, once more after the blocks kept there are freed.
+hipError_t device_malloc(void** p, size_t bytes);
 // Free device memory for a budget (0: unknown), kept blocks included inside a call that can take them.
 size_t device_free_bytes();
 extern thread_local DevAllocator* tl_dev_alloc;
@@ -85,7 +87,7 @@ struct DevBuf {
             if (!p) return set_error(SWEM_ENOMEM, "%s (%zu bytes more)", tl_dev_alloc->name(), count * sizeof(T));
             from = tl_dev_alloc;
         } else {
-            SWEM_HIP(hipMalloc((void**)&p, count * sizeof(T)));
+            SWEM_HIP(device_malloc((void**)&p, count * sizeof(T)));
         }
         n = count;
         return SWEM_OK;

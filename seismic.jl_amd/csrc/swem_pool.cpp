@@ -60,6 +60,22 @@ void trim(Pool& q)
 
 void trim_call_memory(int dev) { trim(pool_of(dev)); }
 
+hipError_t device_malloc(void** p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        int dev = 0;
+        if (hipGetDevice(&dev) == hipSuccess) trim_call_memory(dev);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = nullptr;
+    }
+    return e;
+}
+
 CallMemory::CallMemory(int device) : dev(device)
 {
     if (tl_dev_alloc) return;  // inside a served request or another call
@@ -121,14 +137,7 @@ void* CallMemory::alloc(size_t bytes)
     }
     if (!p) {
         n = (bytes + 255) & ~size_t(255);
-        if (hipMalloc(&p, n) != hipSuccess) {
-            (void)hipGetLastError();
-            trim(q);
-            if (hipMalloc(&p, n) != hipSuccess) {
-                (void)hipGetLastError();
-                return nullptr;
-            }
-        }
+        if (device_malloc(&p, n) != hipSuccess) return nullptr;
     }
     blocks.push_back({p, n, true});
     return p;

@@ -623,7 +623,7 @@ int swem_server_create(const swem_server_config* cfg, swem_server** out)
     if (!c.pinned_bytes) c.pinned_bytes = (size_t)4 << 30;
     auto s = std::make_unique<swem_server>();
     s->cfg = c;
-    SWEM_HIP(hipMalloc((void**)&s->dev_base, c.device_bytes));
+    SWEM_HIP(device_malloc((void**)&s->dev_base, c.device_bytes));
     if (hipHostMalloc((void**)&s->pin_base, c.pinned_bytes, hipHostMallocDefault) != hipSuccess) {
         (void)hipFree(s->dev_base);
         return set_error(SWEM_ENOMEM, "server: %zu bytes of pinned host memory", c.pinned_bytes);

@@ -98,6 +98,19 @@ static int given_back()
     return 0;
 }
 
+// a resident plan's buffers grow after a call has filled the list
+static int growth_after_call()
+{
+    g_capacity = 20 * GiB;
+    DevBuf<char> table, work;
+    EXPECT(table.alloc(4 * GiB) == SWEM_OK);
+    EXPECT(call(0, 8 * GiB, 6 * GiB) == SWEM_OK && g_used == 18 * GiB);
+    EXPECT(work.alloc(12 * GiB) == SWEM_OK && g_used == 16 * GiB);
+    void* p = nullptr;
+    EXPECT(device_malloc(&p, 5 * GiB) == hipErrorOutOfMemory && !p);  // not there at all
+    return 0;
+}
+
 static int buffers_free_themselves()
 {
     {
@@ -116,6 +129,6 @@ int main(int, char** argv)
 {
     const std::map<std::string, int (*)()> all = {
         {"reuse", reuse}, {"bounds", bounds}, {"given_back", given_back},
-        {"buffers_free_themselves", buffers_free_themselves}};
+        {"growth_after_call", growth_after_call}, {"buffers_free_themselves", buffers_free_themselves}};
     return all.at(argv[1])();
 }
