@@ -1550,33 +1550,34 @@ int swem_shots(const swem_geometry* g, const float* vel, const float* wav, const
                float* d, float* m, int adj, const swem_options* opt)
 {
     if (!g || !vel || !wav || !sx || !d || !m || nshot < 1) return set_error(SWEM_EINVAL, "shots: null argument");
-    CallMemory memory(opt ? opt->device : 0);
-    swem_plan* p = nullptr;
-    SWEM_TRY(swem_plan_create(g, vel, wav, opt, &p));
-    const size_t nm = (size_t)g->nmx * g->nmy, nd = (size_t)nshot * nm * g->nt, nmz = nm * g->nz;
-    int rc;
-    {
-        DevBuf<float> dd, dm;
-        rc = dd.alloc(nd);
-        if (!rc) rc = dm.alloc(nmz);
-        auto down = [&](float* host, const float* dev, size_t n) {
-            const hipError_t e = hipMemcpy(host, dev, n * sizeof(float), hipMemcpyDeviceToHost);
-            return e == hipSuccess ? SWEM_OK : hip_error(e, "hipMemcpy", __FILE__, __LINE__);
-        };
-        if (adj) {
-            if (!rc) rc = upload_bytes(dd.p, d, nd * sizeof(float));
-            if (!rc) rc = swem_plan_migrate(p, dd.p, sx, sy, nshot, dm.p, 0, nullptr);
-            if (!rc) rc = down(m, dm.p, nmz);
-        } else {
-            if (!rc) rc = upload_bytes(dm.p, m, nmz * sizeof(float));
-            if (!rc) rc = swem_plan_model(p, dm.p, sx, sy, nshot, dd.p, nullptr);
-            if (!rc) rc = down(d, dd.p, nd);
+    return one_call(opt ? opt->device : 0, [&]() -> int {
+        swem_plan* p = nullptr;
+        SWEM_TRY(swem_plan_create(g, vel, wav, opt, &p));
+        const size_t nm = (size_t)g->nmx * g->nmy, nd = (size_t)nshot * nm * g->nt, nmz = nm * g->nz;
+        int rc;
+        {
+            DevBuf<float> dd, dm;
+            rc = dd.alloc(nd);
+            if (!rc) rc = dm.alloc(nmz);
+            auto down = [&](float* host, const float* dev, size_t n) {
+                const hipError_t e = hipMemcpy(host, dev, n * sizeof(float), hipMemcpyDeviceToHost);
+                return e == hipSuccess ? SWEM_OK : hip_error(e, "hipMemcpy", __FILE__, __LINE__);
+            };
+            if (adj) {
+                if (!rc) rc = upload_bytes(dd.p, d, nd * sizeof(float));
+                if (!rc) rc = swem_plan_migrate(p, dd.p, sx, sy, nshot, dm.p, 0, nullptr);
+                if (!rc) rc = down(m, dm.p, nmz);
+            } else {
+                if (!rc) rc = upload_bytes(dm.p, m, nmz * sizeof(float));
+                if (!rc) rc = swem_plan_model(p, dm.p, sx, sy, nshot, dd.p, nullptr);
+                if (!rc) rc = down(d, dd.p, nd);
+            }
+            dd.release();
+            dm.release();
         }
-        dd.release();
-        dm.release();
-    }
-    swem_plan_destroy(p);
-    return rc;
+        swem_plan_destroy(p);
+        return rc;
+    });
 }
 
 int swem_wem_ex(float* d, float* m, const float* wav, const swem_geometry* g, float sx, float sy, const float* vel,
@@ -1813,12 +1814,13 @@ int swem_compute_angles_ex(float* angx, float* angy, const float* wav, const swe
     swem_options o;
     if (opt) o = *opt;
     else swem_options_init(&o);
-    CallMemory memory(o.device);
-    swem_plan* p = nullptr;
-    SWEM_TRY(swem_plan_create(&ga, vel, wav, &o, &p));
-    const int rc = angles_impl(p, sx, sy, angx, angy);
-    swem_plan_destroy(p);
-    return rc;
+    return one_call(o.device, [&]() -> int {
+        swem_plan* p = nullptr;
+        SWEM_TRY(swem_plan_create(&ga, vel, wav, &o, &p));
+        const int rc = angles_impl(p, sx, sy, angx, angy);
+        swem_plan_destroy(p);
+        return rc;
+    });
 }
 
 int swem_compute_angles(float* angx, float* angy, const float* wav, int nt, float ot, float dt, int nmx, float omx,
@@ -2211,20 +2213,21 @@ int swem_eshots(const swem_geometry* g, const float* vp, const float* vs, const 
     swem_options o;
     if (opt) o = *opt;
     else swem_options_init(&o);
-    CallMemory memory(o.device);
-    swem_plan *pp = nullptr, *ps = nullptr;
-    // both plans sample the band as ewem.c does (ewem.c:43-52)
-    SWEM_TRY(plan_create_rule(&ge, vp, wav, &o, 1, &pp));
-    int rc = plan_create_rule(&ge, vs, wav, &o, 1, &ps);
-    if (!rc && (pp->s.ntfft != ntfft || pp->s.ifmin != ifmin || pp->s.ifmax != ifmax))
-        rc = set_error(SWEM_EDEVICE, "ewem: internal band mismatch (ntfft %d, [%d, %d)) against (%d, [%d, %d))", ntfft,
-                       ifmin, ifmax, pp->s.ntfft, pp->s.ifmin, pp->s.ifmax);
-    if (!rc)
-        rc = three_d ? eshots3d_impl(pp, ps, nshot, sx, sy, ux, uy, uz, mpp, mps1, mps2, wav, adj)
-                     : eshots_impl(pp, ps, nshot, igx.data(), ux, uy, uz, mpp, mps1, mps2, wav, adj);
-    if (ps) swem_plan_destroy(ps);
-    swem_plan_destroy(pp);
-    return rc;
+    return one_call(o.device, [&]() -> int {
+        swem_plan *pp = nullptr, *ps = nullptr;
+        // both plans sample the band as ewem.c does (ewem.c:43-52)
+        SWEM_TRY(plan_create_rule(&ge, vp, wav, &o, 1, &pp));
+        int rc = plan_create_rule(&ge, vs, wav, &o, 1, &ps);
+        if (!rc && (pp->s.ntfft != ntfft || pp->s.ifmin != ifmin || pp->s.ifmax != ifmax))
+            rc = set_error(SWEM_EDEVICE, "ewem: internal band mismatch (ntfft %d, [%d, %d)) against (%d, [%d, %d))", ntfft,
+                           ifmin, ifmax, pp->s.ntfft, pp->s.ifmin, pp->s.ifmax);
+        if (!rc)
+            rc = three_d ? eshots3d_impl(pp, ps, nshot, sx, sy, ux, uy, uz, mpp, mps1, mps2, wav, adj)
+                         : eshots_impl(pp, ps, nshot, igx.data(), ux, uy, uz, mpp, mps1, mps2, wav, adj);
+        if (ps) swem_plan_destroy(ps);
+        swem_plan_destroy(pp);
+        return rc;
+    });
 }
 
 int swem_ewem(float* ux, float* uy, float* uz, float* mpp, float* mps1, float* mps2, const float* wav, int nt,

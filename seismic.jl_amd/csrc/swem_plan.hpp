@@ -35,6 +35,7 @@ struct CallMemory : DevAllocator {
     void release(void* p, size_t bytes) override;
     size_t spare() const override;
     const char* name() const override { return "out of device memory"; }
+    bool installed() const { return on; }
     CallMemory(const CallMemory&) = delete;
     CallMemory& operator=(const CallMemory&) = delete;
 
@@ -56,6 +57,21 @@ hipError_t device_malloc(void** p, size_t bytes);
 size_t device_free_bytes();
 extern thread_local DevAllocator* tl_dev_alloc;
 extern thread_local HostStager* tl_stager;
+
+// Runs a one-call entry point (a status; its inputs unchanged, its outputs written whole) on kept blocks.
+// Where that runs out of memory -- a kept block may be a third larger than what was asked for, and a block
+// that the call has released stays with it -- everything goes back and it runs once more on plain allocations.
+template <class Body>
+int one_call(int device, Body&& body)
+{
+    {
+        CallMemory memory(device);
+        const int rc = body();
+        if (rc != SWEM_ENOMEM || !memory.installed()) return rc;
+    }
+    trim_call_memory(device);
+    return body();
+}
 
 int upload_bytes(void* dev, const void* host, size_t bytes);
 

@@ -62,11 +62,12 @@ constexpr size_t GiB = size_t(1) << 30, MiB = size_t(1) << 20;
 template <class... S>
 static int call(int device, S... bytes)
 {
-    CallMemory memory(device);
-    DevBuf<char> b[sizeof...(bytes)];
-    const size_t n[] = {(size_t)bytes...};
-    for (size_t i = 0; i < sizeof...(bytes); i++) SWEM_TRY(b[i].alloc(n[i]));
-    return SWEM_OK;
+    return one_call(device, [&] {
+        DevBuf<char> b[sizeof...(bytes)];
+        const size_t n[] = {(size_t)bytes...};
+        for (size_t i = 0; i < sizeof...(bytes); i++) SWEM_TRY(b[i].alloc(n[i]));
+        return SWEM_OK;
+    });
 }
 
 static int reuse()
@@ -111,6 +112,25 @@ static int growth_after_call()
     return 0;
 }
 
+// a call near the limit gets what plain allocations would give it: blocks that it released itself, and
+// what kept blocks are larger than it asked for
+static int call_at_the_limit()
+{
+    g_capacity = 20 * GiB;
+    const int rc = one_call(0, [&] {
+        DevBuf<char> a, b;
+        SWEM_TRY(a.alloc(12 * GiB));
+        a.release();
+        return b.alloc(15 * GiB);
+    });
+    EXPECT(rc == SWEM_OK);
+    trim_call_memory(0);
+    EXPECT(call(0, 8 * GiB, 8 * GiB) == SWEM_OK);
+    EXPECT(call(0, 6 * GiB + 1, 6 * GiB + 1, 7 * GiB) == SWEM_OK);
+    EXPECT(call(0, 21 * GiB) == SWEM_ENOMEM);
+    return 0;
+}
+
 static int buffers_free_themselves()
 {
     {
@@ -129,6 +149,7 @@ int main(int, char** argv)
 {
     const std::map<std::string, int (*)()> all = {
         {"reuse", reuse}, {"bounds", bounds}, {"given_back", given_back},
-        {"growth_after_call", growth_after_call}, {"buffers_free_themselves", buffers_free_themselves}};
+        {"growth_after_call", growth_after_call}, {"call_at_the_limit", call_at_the_limit},
+        {"buffers_free_themselves", buffers_free_themselves}};
     return all.at(argv[1])();
 }

@@ -6,7 +6,7 @@ import pytest
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "seismic.jl_amd", "csrc")
-SCENARIOS = ["reuse", "bounds", "given_back", "buffers_free_themselves", "growth_after_call"]
+SCENARIOS = ["reuse", "bounds", "given_back", "buffers_free_themselves", "growth_after_call", "call_at_the_limit"]
 
 
 @pytest.fixture(scope="module")
