@@ -12,6 +12,7 @@
 // belongs to one call at a time; it returns to the list after the device has finished the call.
 #include <algorithm>
 #include <mutex>
+#include <new>
 
 #include "swem_plan.hpp"
 
@@ -93,6 +94,12 @@ CallMemory::~CallMemory()
     Pool& q = pool_of(dev);
     std::lock_guard<std::mutex> lock(q.mu);
     const unsigned long long now = ++q.calls;
+    try {
+        q.free.reserve(q.free.size() + blocks.size());
+    } catch (const std::bad_alloc&) {  // no room to note them: they go
+        for (const Held& b : blocks) (void)hipFree(b.p);
+        return;
+    }
     for (const Held& b : blocks) {
         q.free.push_back({b.p, b.n, now});
         q.kept += b.n;
@@ -118,6 +125,11 @@ void* CallMemory::alloc(size_t bytes)
     if (own) {
         own->taken = true;
         return own->p;
+    }
+    try {
+        blocks.reserve(blocks.size() + 1);
+    } catch (const std::bad_alloc&) {
+        return nullptr;
     }
     Pool& q = pool_of(dev);
     void* p = nullptr;

@@ -6,9 +6,12 @@
 #include <cstdlib>
 #include <cstring>
 #include <map>
+#include <new>
 #include <string>
 
 #include "swem_plan.hpp"
+
+static long g_new_left = -1;  // host allocations until one fails (-1: none does)
 
 // ------------------------------------------------------------------ the device
 static size_t g_capacity = size_t(100) << 30, g_used = 0, g_mallocs = 0, g_syncs = 0;
@@ -21,7 +24,10 @@ hipError_t hipMalloc(void** p, size_t n)
     g_mallocs++;
     if (g_used + n > g_capacity) return hipErrorOutOfMemory;
     *p = std::malloc(1);
+    const long left = g_new_left;  // (not of the library)
+    g_new_left = -1;
     g_live[*p] = {n, g_device};
+    g_new_left = left;
     g_used += n;
     return hipSuccess;
 }
@@ -41,6 +47,17 @@ hipError_t hipGetLastError(void) { return hipSuccess; }
 hipError_t hipMemGetInfo(size_t* fr, size_t* tot) { return *fr = g_capacity - g_used, *tot = g_capacity, hipSuccess; }
 const char* hipGetErrorString(hipError_t) { return "device error"; }
 }
+
+// ------------------------------------------------------------------ the host: allocations that fail on demand
+void* operator new(size_t n)
+{
+    if (g_new_left == 0) throw std::bad_alloc();
+    if (g_new_left > 0) g_new_left--;
+    if (void* p = std::malloc(n ? n : 1)) return p;
+    throw std::bad_alloc();
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace swem {
 thread_local DevAllocator* tl_dev_alloc = nullptr;
@@ -145,11 +162,27 @@ static int buffers_free_themselves()
     return 0;
 }
 
+// no exception leaves the entry points, wherever the host runs out of memory
+static int host_memory()
+{
+    EXPECT(call(0, MiB, 2 * MiB) == SWEM_OK);
+    for (long left = 0; left < 12; left++) {
+        g_new_left = left;
+        const int rc = call(0, MiB, 2 * MiB, (3 + left) * MiB);
+        g_new_left = -1;
+        EXPECT(rc == SWEM_OK || rc == SWEM_ENOMEM);
+        EXPECT(!tl_dev_alloc);
+    }
+    trim_call_memory(0);
+    EXPECT(g_used == 0 && g_live.empty());
+    return 0;
+}
+
 int main(int, char** argv)
 {
     const std::map<std::string, int (*)()> all = {
         {"reuse", reuse}, {"bounds", bounds}, {"given_back", given_back},
         {"growth_after_call", growth_after_call}, {"call_at_the_limit", call_at_the_limit},
-        {"buffers_free_themselves", buffers_free_themselves}};
+        {"buffers_free_themselves", buffers_free_themselves}, {"host_memory", host_memory}};
     return all.at(argv[1])();
 }
