@@ -45,10 +45,12 @@ struct Pool {
     }
 };
 
-Pool& pool_of(int dev)
+bool has_pool(int dev) { return dev >= 0 && dev < kDevices; }
+
+Pool& pool_of(int dev)  // of a device that has one
 {
     static Pool* pools = new Pool[kDevices];  // never destroyed: the runtime may be gone at exit
-    return pools[dev >= 0 && dev < kDevices ? dev : 0];
+    return pools[dev];
 }
 
 void trim(Pool& q)
@@ -59,7 +61,10 @@ void trim(Pool& q)
 
 }  // namespace
 
-void trim_call_memory(int dev) { trim(pool_of(dev)); }
+void trim_call_memory(int dev)
+{
+    if (has_pool(dev)) trim(pool_of(dev));
+}
 
 hipError_t device_malloc(void** p, size_t bytes)
 {
@@ -79,7 +84,8 @@ hipError_t device_malloc(void** p, size_t bytes)
 
 CallMemory::CallMemory(int device) : dev(device)
 {
-    if (tl_dev_alloc) return;  // inside a served request or another call
+    // inside a served request or another call, or no list for the device: plain allocations
+    if (tl_dev_alloc || !has_pool(device)) return;
     tl_dev_alloc = this;
     on = true;
 }

@@ -178,11 +178,31 @@ static int host_memory()
     return 0;
 }
 
+// a block belongs to the device it was taken on
+static int many_devices()
+{
+    for (int d : {0, 63, 64, 200}) {
+        g_device = d;
+        EXPECT(call(d, MiB) == SWEM_OK);
+    }
+    for (int d : {0, 63, 64, 200}) {
+        g_device = d;
+        const int rc = one_call(d, [&] {
+            DevBuf<char> b;
+            SWEM_TRY(b.alloc(MiB));
+            return g_live[b.p].second == d ? SWEM_OK : SWEM_EDEVICE;
+        });
+        EXPECT(rc == SWEM_OK);
+    }
+    return 0;
+}
+
 int main(int, char** argv)
 {
     const std::map<std::string, int (*)()> all = {
         {"reuse", reuse}, {"bounds", bounds}, {"given_back", given_back},
         {"growth_after_call", growth_after_call}, {"call_at_the_limit", call_at_the_limit},
-        {"buffers_free_themselves", buffers_free_themselves}, {"host_memory", host_memory}};
+        {"buffers_free_themselves", buffers_free_themselves}, {"host_memory", host_memory},
+        {"many_devices", many_devices}};
     return all.at(argv[1])();
 }

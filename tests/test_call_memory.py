@@ -7,7 +7,7 @@ import pytest
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(os.path.dirname(HERE), "seismic.jl_amd", "csrc")
 SCENARIOS = ["reuse", "bounds", "given_back", "buffers_free_themselves", "growth_after_call", "call_at_the_limit",
-             "host_memory"]
+             "host_memory", "many_devices"]
 
 
 @pytest.fixture(scope="module")
