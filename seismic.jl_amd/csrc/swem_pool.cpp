@@ -6,8 +6,9 @@
 // its 10.5 GB of phase tables (the 1024 x 500 PSPI grid) anew waited up to 300 ms for a 12 ms march
 // (339 -> 23 ms per call in a loop of calls).
 //
-// The list is bounded (kKeep per device, least recently used blocks go first), drops blocks that the
-// last few calls did not take, and is given back whole before a plan or a server is created and when
+// The list is bounded (kKeep per device and a share of the device's free memory, so that several processes
+// on one device, each with its list, leave it room; least recently used blocks go first), drops blocks that
+// the last few calls did not take, and is given back whole before a plan or a server is created and when
 // an allocation of the library fails, so those see the memory a process without it would.  A block
 // belongs to one call at a time; it returns to the list after the device has finished the call.
 #include <algorithm>
@@ -20,7 +21,8 @@ namespace swem {
 
 namespace {
 
-constexpr size_t kKeep = size_t(16) << 30;  // bytes kept per device between calls
+constexpr size_t kKeep = size_t(16) << 30;  // bytes kept per device between calls, at most,
+constexpr size_t kShare = 8;                // and of the free memory at the end of a call one part in this many
 constexpr int kIdleCalls = 4;               // calls a block may stay unused
 constexpr int kDevices = 64;
 
@@ -112,7 +114,9 @@ CallMemory::~CallMemory()
     }
     for (size_t i = q.free.size(); i-- > 0;)
         if (q.free[i].used + kIdleCalls < now) q.drop(i);
-    while (q.kept > kKeep) {
+    size_t fr = 0, tot = 0, most = kKeep;
+    if (hipMemGetInfo(&fr, &tot) == hipSuccess) most = std::min(kKeep, (fr + q.kept) / kShare);
+    while (q.kept > most) {
         size_t old = 0;  // the least recently used, the largest of them
         for (size_t i = 1; i < q.free.size(); i++)
             if (q.free[i].used < q.free[old].used || (q.free[i].used == q.free[old].used && q.free[i].n > q.free[old].n)) old = i;

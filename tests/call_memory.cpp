@@ -14,7 +14,7 @@
 static long g_new_left = -1;  // host allocations until one fails (-1: none does)
 
 // ------------------------------------------------------------------ the device
-static size_t g_capacity = size_t(100) << 30, g_used = 0, g_mallocs = 0, g_syncs = 0;
+static size_t g_capacity = size_t(288) << 30, g_used = 0, g_mallocs = 0, g_syncs = 0;
 static int g_device = 0;
 static std::map<void*, std::pair<size_t, int>> g_live;  // bytes and device
 
@@ -102,6 +102,12 @@ static int bounds()
     EXPECT(call(0, 9 * GiB, 9 * GiB) == SWEM_OK && g_used == 9 * GiB);  // at most 16 GiB stay
     for (int i = 0; i < 4; i++) EXPECT(call(0, 2 * GiB) == SWEM_OK && g_used == 11 * GiB);
     EXPECT(call(0, 2 * GiB) == SWEM_OK && g_used == 2 * GiB);  // unused by the last four calls
+    // other processes have taken the rest: an eighth of what is left
+    g_capacity = 40 * GiB;
+    EXPECT(call(0, 4 * GiB, 2 * GiB) == SWEM_OK && g_used == 2 * GiB);
+    EXPECT(call(0, 4 * GiB) == SWEM_OK && g_used == 4 * GiB);
+    g_capacity = 10 * GiB;
+    EXPECT(call(0, 2 * GiB) == SWEM_OK && g_used == 0);
     return 0;
 }
 
@@ -119,10 +125,10 @@ static int given_back()
 // a resident plan's buffers grow after a call has filled the list
 static int growth_after_call()
 {
-    g_capacity = 20 * GiB;
     DevBuf<char> table, work;
     EXPECT(table.alloc(4 * GiB) == SWEM_OK);
     EXPECT(call(0, 8 * GiB, 6 * GiB) == SWEM_OK && g_used == 18 * GiB);
+    g_capacity = 20 * GiB;  // others took the rest
     EXPECT(work.alloc(12 * GiB) == SWEM_OK && g_used == 16 * GiB);
     void* p = nullptr;
     EXPECT(device_malloc(&p, 5 * GiB) == hipErrorOutOfMemory && !p);  // not there at all
@@ -142,7 +148,9 @@ static int call_at_the_limit()
     });
     EXPECT(rc == SWEM_OK);
     trim_call_memory(0);
+    g_capacity = 288 * GiB;
     EXPECT(call(0, 8 * GiB, 8 * GiB) == SWEM_OK);
+    g_capacity = 20 * GiB;
     EXPECT(call(0, 6 * GiB + 1, 6 * GiB + 1, 7 * GiB) == SWEM_OK);
     EXPECT(call(0, 21 * GiB) == SWEM_ENOMEM);
     return 0;
