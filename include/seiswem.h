@@ -335,6 +335,14 @@ int swem_memcpy_dtoh(void* dst, const void* src, size_t bytes);
 int swem_memcpy_dtod(void* dst, const void* src, size_t bytes);
 int swem_memset(void* ptr, int value, size_t bytes);
 int swem_synchronize(void);
+/* Frees the device memory that the one-call entry points (swem_shots, swem_wem, swem_ewem,
+ * swem_eshots, swem_compute_angles and their _ex forms, and the file drivers) keep between
+ * calls: up to 16 GiB per process and device and at most an eighth of the device's free memory,
+ * so that a loop of calls does not allocate and clear its tables anew each time.  Creating a
+ * plan or a server and an allocation of the library that would fail free it too; other users of
+ * the device see it as taken until then.  Calls that are running keep theirs.  SWEM_EINVAL for a
+ * negative device. */
+int swem_release_memory(int device);
 
 /* Device vector operations of the least-squares solver, for vectors resident in device memory
  * (models [nm][nz], records [nshot][nm][nt]):

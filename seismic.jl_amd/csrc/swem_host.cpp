@@ -2324,6 +2324,13 @@ int swem_synchronize(void)
     return SWEM_OK;
 }
 
+int swem_release_memory(int device)
+{
+    if (device < 0) return set_error(SWEM_EINVAL, "release_memory: device %d", device);
+    trim_call_memory(device);
+    return SWEM_OK;
+}
+
 int swem_sampling(const swem_geometry* g, int* out)
 {
     if (!g || !out) return set_error(SWEM_EINVAL, "sampling: null argument");

@@ -8,8 +8,9 @@
 //
 // The list is bounded (kKeep per device and a share of the device's free memory, so that several processes
 // on one device, each with its list, leave it room; least recently used blocks go first), drops blocks that
-// the last few calls did not take, and is given back whole before a plan or a server is created and when
-// an allocation of the library fails, so those see the memory a process without it would.  A block
+// the last few calls did not take, and is given back whole before a plan or a server is created, when
+// an allocation of the library fails, so those see the memory a process without it would, and by
+// swem_release_memory.  A block
 // belongs to one call at a time; it returns to the list after the device has finished the call.
 #include <algorithm>
 #include <mutex>

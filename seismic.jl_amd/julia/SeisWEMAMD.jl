@@ -51,6 +51,13 @@ function check(rc::Cint)
 end
 
 """
+    release_memory(device=0)
+
+Frees the device memory that the one-call functions keep between calls.
+"""
+release_memory(device::Integer=0) = check(ccall((:swem_release_memory, libseiswem), Cint, (Cint,), device))
+
+"""
     wem!(d, m, wav, vel; nt, ot, dt, nmx, omx, dmx, nmy, omy, dmy, sx, sy, nz, oz, dz, gz, sz,
          nref, fmin, fmax, padt, padx, adj, pspi, verbose=false)
 

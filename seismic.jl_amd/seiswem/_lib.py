@@ -27,6 +27,7 @@ EXPORTS = (
     "swem_plan_create", "swem_plan_destroy", "swem_plan_migrate", "swem_plan_migrate_each", "swem_plan_migrate_noalloc",
     "swem_plan_model", "swem_plan_timing", "swem_plan_autotune", "swem_plan_autotune_ex", "swem_plan_set_graphs", "swem_plan_bytes",
     "swem_malloc", "swem_free", "swem_memcpy_htod", "swem_memcpy_dtoh", "swem_memcpy_dtod", "swem_memset", "swem_synchronize",
+    "swem_release_memory",
     "swem_sampling", "swem_source_index", "swem_pspi_tables", "swem_taper",
     "swem_seis_extent_init", "swem_seis_read_header", "swem_seis_read", "swem_seis_write",
     "swem_server_config_init", "swem_server_create", "swem_server_destroy", "swem_batch_submit",
@@ -193,6 +194,7 @@ def load():
         "swem_memcpy_dtod": ([vp, vp, ctypes.c_size_t], ctypes.c_int),
         "swem_memset": ([vp, ctypes.c_int, ctypes.c_size_t], ctypes.c_int),
         "swem_synchronize": ([], ctypes.c_int),
+        "swem_release_memory": ([ctypes.c_int], ctypes.c_int),
         "swem_sampling": ([gp, i32p], ctypes.c_int),
         "swem_source_index": ([gp, ctypes.c_float, ctypes.c_float, i32p, i32p], ctypes.c_int),
         "swem_pspi_tables": ([gp, f32p, f32p, i32p, i32p, P(ctypes.c_ubyte)], ctypes.c_int),

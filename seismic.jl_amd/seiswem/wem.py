@@ -198,6 +198,12 @@ def synchronize():
     check(load().swem_synchronize())
 
 
+def release_memory(device: int = 0):
+    """Frees the device memory that the one-call functions (ShotProfileWEM, wem, ShotProfileEWEM, ewem,
+    compute_angles) keep between calls (swem_release_memory)."""
+    check(load().swem_release_memory(int(device)))
+
+
 def copy_device(dst: DeviceArray, src: DeviceArray):
     """Device-to-device copy of a whole buffer."""
     if dst.nbytes != src.nbytes:

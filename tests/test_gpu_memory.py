@@ -30,3 +30,41 @@ def test_plans_leave_nothing(gpu):
     for _ in range(160):
         seiswem.Plan(g, vel, wav).close()
     assert _used() - before <= 4 * MIB  # 20 MiB of tables, were they left
+
+
+def _migrate(nx, nz):
+    g, vel, wav = _case(nx=nx, nz=nz)
+    rng = np.random.default_rng(nx + nz)
+    d = rng.standard_normal((1, g.nm, g.nt)).astype(np.float32)
+    m = seiswem.ShotProfileWEM(d, True, vel=vel, wav=wav, geom=g, sx=[100.0])
+    return g, vel, wav, d, m
+
+
+def test_host_calls_keep_and_give_back(gpu):
+    """Host calls of alternating sizes, each on blocks that others have written: the image of a resident plan,
+    bit for bit.  What they keep goes by release_memory and before a plan is created."""
+    sizes = [(256, 400), (64, 20), (256, 390), (250, 400), (128, 100), (256, 400)]
+    images = [_migrate(nx, nz) for nx, nz in sizes]
+    # the phase tables of the last call: 400 depths x 153 frequencies x (257 wavenumbers + 256 traces) x 8 bytes
+    tables = 400 * 153 * (257 + 256) * 8
+    kept = _used()
+    seiswem.release_memory()
+    assert kept - _used() >= tables
+    for g, vel, wav, d, m in images:
+        plan = seiswem.Plan(g, vel, wav)
+        ref = plan.migrate(seiswem.DeviceArray(d.shape, d), [100.0]).download()
+        plan.close()
+        assert np.array_equal(m, ref) and np.any(m)
+    _migrate(256, 400)
+    g, vel, wav = _case()
+    kept = _used()
+    plan = seiswem.Plan(g, vel, wav)
+    assert kept - _used() >= tables - 32 * MIB  # the new plan's own buffers are smaller than that
+    plan.close()
+
+
+def test_release_memory_refuses_a_negative_device(gpu):
+    with pytest.raises(seiswem.SwemError) as e:
+        seiswem.release_memory(-1)
+    assert e.value.code == seiswem.SWEM_EINVAL
+    seiswem.release_memory(63)  # nothing kept there
