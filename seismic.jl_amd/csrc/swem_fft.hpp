@@ -726,26 +726,6 @@ __device__ __forceinline__ void fft2(float2 (&u)[P], float2 (&v)[P], float2* bu,
 // shot of 350 traces 377 -> 398 us, eight linear ones of 550 traces 2.85 -> 4.05 ms); Bluestein took 522 us and 12.1 ms.
 // LDS indices are unpadded: the loads and the later passes' stores run at unit lane
 // stride, the first pass's stores at stride R.
-
-// The seeds of dft_pow2 from w alone: w^(R/2) .. w by squares, the W_8 multiple by sums.
-template <int R>
-__device__ __forceinline__ void radix_seeds(float2 w, float2 (&s)[R / 2])
-{
-    static_assert(R == 2 || R == 4 || R == 8, "radices of mixed_fft");
-    auto square = [](float2 a) { return make_float2(fmaf(a.x, a.x, -(a.y * a.y)), (a.x + a.x) * a.y); };
-    if constexpr (R == 2) {
-        s[0] = w;
-    } else if constexpr (R == 4) {
-        s[0] = square(w);
-        s[1] = w;
-    } else {
-        s[1] = square(w);
-        s[0] = square(s[1]);
-        s[2] = w;
-        s[3] = make_float2(kCos8[2] * (w.x + w.y), kCos8[2] * (w.y - w.x));
-    }
-}
-
 template <int R, int SIGN, int IT, bool PP, bool TABLE, class Sync>
 __device__ __forceinline__ void mixed_pass(const float2* src, float2* dst, const float2* __restrict__ tw, int n,
                                            int ns, int tws, uint32_t magic, int t, int T, Sync sync)
