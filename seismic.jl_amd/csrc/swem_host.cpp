@@ -1078,7 +1078,7 @@ int plan_setup(swem_plan* p, const swem_geometry* g, const float* vel, const swe
     if (!(g->dz != 0.f)) return set_error(SWEM_EINVAL, "dz must be non-zero");
     SWEM_TRY(check_device(o.device));
     if (p->three_d) {
-        // y-pass workgroups: one wave per frequency (both wavefields in migration)
+        // y-pass workgroups: one line of lanes per frequency (both wavefields in migration)
         if (o.freqs_per_block > 0) p->F3 = p->F3f = o.freqs_per_block;
         const int fmax = (g->pspi || p->narr_y != p->s.nky) ? 8 : 16;  // Bluestein y-passes: 512 threads
         if (p->F3 < 1 || p->F3 > fmax || p->F3f > fmax)

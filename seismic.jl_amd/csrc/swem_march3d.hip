@@ -47,7 +47,7 @@ int launch_ewem3d(int which, const March3DArgs& ap, const March3DArgs& as, const
     const int n = xpass ? ap.nkx : ap.nky, m = march3d_len(n);
     if (!march3d_supported(ap.nkx, ap.nky) || ap.nmx > ap.nkx || ap.nmy > ap.nky || ap.nitem < 1 || !e.W)
         return set_error(SWEM_EINVAL, "3-D ewem: inconsistent launch (nkx=%d nky=%d)", ap.nkx, ap.nky);
-    if (which == 2 && (F < 1 || F > 8))  // the y-pass holds three rows per wave: 512 threads
+    if (which == 2 && (F < 1 || F > 8))  // the y-pass holds three rows per line of lanes: 512 threads
         return set_error(SWEM_EINVAL, "3-D ewem: %d frequencies per workgroup (1..8)", F);
     const int kind = march3d_kind(n);
     if ((kind == kLenBluestein && (xpass ? !(ap.chx && ap.bchx) : !(ap.chy && ap.bchy))) ||

@@ -18,8 +18,8 @@
 // out as  [FFTy] FFTx L IFFTx | IFFTy SS taper image FFTy ...  and the forward step (wem.c:321-
 // 332, 362-369) taper -> SS -> FFT2 -> L -> IFFT2 as  IFFTy inject taper SS FFTy | FFTx L IFFTx.
 // An item is one frequency of one shot; a launch covers every item of the frequency chunk.
-// Transforms are wave-level (one 64-lane wave per row / column, N/64 points per lane, no
-// workgroup barrier inside a transform).  An axis whose length n is not a power of two 128..1024
+// Transforms stay inside a wave: a row / column takes one 64-lane wave, or a share of one (8 to 32
+// lanes) below 512 points (line_lanes), with no workgroup barrier inside a transform.  An axis whose length n is not a power of two 128..1024
 // is transformed through Bluestein's identity on an array of N >= 2n - 1 points (line_fft).
 #pragma once
 #include "swem_esep.hpp"
@@ -146,7 +146,7 @@ __device__ __forceinline__ bool yin(const March3DArgs& a, int i)
 
 // Transform of one line of n points held by G lanes as N array points (lane t, slot q: point
 // t + G q).  KIND kLenPow2: n = N, the wave FFT.  kLenMixed, kLenMixedPrime: the
-// mixed-radix transform in the wave's LDS buffer (tw: [n] of n).  kLenBluestein: Bluestein's
+// mixed-radix transform in the line's LDS buffer (tw: [n] of n).  kLenBluestein: Bluestein's
 // chirp-z identity on the power-of-two array length N >= 2n - 1, X_k = c_k IFFT_N(FFT_N(c x) B)_k
 // with the chirp c_j = exp(SIGN i pi j^2 / n) and B the spectrum of the wrapped conjugate chirp
 // over N, built in FP64 on the host (c = 0 for j >= n, so points beyond n enter and leave as zero).
@@ -204,7 +204,7 @@ __device__ __forceinline__ void yfft(LinePoints<N, BY>& v, float2* buf, const Ma
 
 // Initial wavefields of the chunk (adjoint: source delta at the shot position and receiver
 // spectra; forward: source delta, receiver zero), forward y-FFT, stored as the step state.
-// Workgroup: WAVES rows (one wave each); grid: nitem * 2 * nmx rows.
+// Workgroup: 256 lanes, 256 / G rows; grid: nitem * 2 * nmx rows.
 template <int NY, int BY>
 __global__ __launch_bounds__(256) void march3d_init(March3DArgs a)
 {
@@ -214,7 +214,9 @@ __global__ __launch_bounds__(256) void march3d_init(March3DArgs a)
     const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const size_t row = (size_t)blockIdx.x * (256 / G) + w;
     const size_t nrow = (size_t)a.nitem * 2 * a.nmx;
-    if (row >= nrow) return;  // whole waves only: the transform below has no workgroup barrier
+    // whole lines leave, which below 512 points may be part of a wave: the transform below has no
+    // workgroup barrier and each line owns its buffer
+    if (row >= nrow) return;
     const int x = (int)(row % a.nmx);
     const int wf = (int)((row / a.nmx) & 1);
     const int item = (int)(row / ((size_t)2 * a.nmx));
@@ -298,7 +300,7 @@ __device__ __forceinline__ void tile_store(float2* dst, const float2* src, const
     }
 }
 
-// x-pass.  Workgroup: C waves, wave w owns column ky0 + w of every stepped wavefield (NWF = 2:
+// x-pass.  Workgroup: C lines, line w owns column ky0 + w of every stepped wavefield (NWF = 2:
 // source and receiver, which share the kz phase; NWF = 1: the one wmask names).  The tile of C
 // consecutive ky columns is staged through LDS so the global reads and writes are row segments
 // of C complex.  conj_src / conj_rec: use conj(L) (-dz).  Workgroups are renumbered so that each
@@ -691,7 +693,7 @@ __device__ __forceinline__ float pspi3_weight(uint8_t s1, uint8_t s2, float w2, 
     return wt;
 }
 
-// y-pass of PSPI, F waves (frequencies g F + f) of one row x.
+// y-pass of PSPI, F lines (frequencies g F + f) of one row x.
 //   phase 0 migration: select the stepped wavefields (the source is re-read from its state when
 //           only the receiver steps), image (summed over the F frequencies in a fixed order),
 //           forward y-FFT of what steps next
@@ -867,7 +869,7 @@ __global__ __launch_bounds__(512) void march3d_rows_pspi(March3DArgs a, int F, i
     }
 }
 
-// y-pass of the migration (adjoint): F waves, wave f owns row x of the source and the receiver
+// y-pass of the migration (adjoint): F lines, line f owns row x of the source and the receiver
 // of frequency item g F + f.  ds / dr: the source / receiver was stepped at this depth; next_s /
 // next_r: it is stepped at the next depth (its forward y-FFT is needed); the imaging runs when dr.
 // The split-step phase is computed once and applied conjugated to the source.
@@ -957,7 +959,7 @@ __global__ __launch_bounds__(BY ? 512 : 1024) void march3d_rows_adj(March3DArgs 
     }
 }
 
-// y-pass of modelling (forward), one wavefield per wave, F frequencies of one row x.
+// y-pass of modelling (forward), one wavefield per line, F frequencies of one row x.
 //   phase 0 (source march): IFFTy, SS (conj) and taper as the adjoint source, store the
 //           spatial source of this depth in smig (zero where z < sz), FFTy for the next step.
 //   phase 1 (receiver march, upward): IFFTy of the previous step's result (skipped at the first
@@ -1071,7 +1073,7 @@ __device__ __forceinline__ float2* eslot(const March3DArgs& a, const Ewem3DArgs&
 }
 
 // Initial state: the source delta at igx (slot 0) and the receiver spectra (slots 1 and 2, zero
-// when modelling), forward y-FFT.  One wave per row; grid: nitem * 3 * nmx rows.
+// when modelling), forward y-FFT.  256 / G rows per workgroup; grid: nitem * 3 * nmx rows.
 template <int NY, int BY>
 __global__ __launch_bounds__(256) void ewem3d_init(March3DArgs a, Ewem3DArgs e)
 {
@@ -1080,7 +1082,7 @@ __global__ __launch_bounds__(256) void ewem3d_init(March3DArgs a, Ewem3DArgs e)
     __shared__ float2 lds[256 / G * L];
     const int w = threadIdx.x / G, t = threadIdx.x & (G - 1);
     const size_t row = (size_t)blockIdx.x * (256 / G) + w;
-    if (row >= (size_t)a.nitem * 3 * a.nmx) return;  // whole waves only
+    if (row >= (size_t)a.nitem * 3 * a.nmx) return;  // whole lines, as in march3d_init
     const int x = (int)(row % a.nmx);
     const int s = (int)((row / a.nmx) % 3);
     const int item = (int)(row / ((size_t)3 * a.nmx));
@@ -1251,7 +1253,7 @@ __global__ __launch_bounds__((line_lanes(NX, BX) * C)) __attribute__((amdgpu_wav
     }
 }
 
-// y-pass, F waves (frequencies g F + f) of one row x.
+// y-pass, F lines (frequencies g F + f) of one row x.
 //   phase 0 migration: the stepped source (inverse y-FFT, conj split-step phase of vp, taper) and
 //           potentials (split-step phases of vp and vs, taper); images factor Re(conj(s / maxs) up)
 //           and factor Re(conj(s / maxs) us2) summed over the F frequencies (zero where the source is
