@@ -845,7 +845,7 @@ __device__ __forceinline__ float subgroup_sum(float v, float* red)
 // of the transforms stay in registers for the whole march, a kz row is read while the transform
 // before it runs, the selection bytes and the direct sums' twiddles at the start of the depth, and
 // the wave sums take no LDS.  64 shots of 1024 traces x 500 depths x 641 frequencies: 282 -> 217 ms, VALUs
-// 89 % busy at 2843 instructions per wave and depth.
+// 90 % busy at 2906 instructions per wave and depth.
 template <int N, int P, bool WAVE, bool HALF, class X = XPow2<N, P, WAVE, kSeedHeld>>
 __device__ __forceinline__ void adj_body_packed(const March2DArgs& a)
 {

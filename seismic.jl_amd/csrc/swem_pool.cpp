@@ -4,14 +4,14 @@
 // A call's blocks go back to a per-device list instead of hipFree, and the next call takes blocks that
 // fit from it: the driver clears freed memory before it hands it out again, so a call that allocates
 // its 10.5 GB of phase tables (the 1024 x 500 PSPI grid) anew waited up to 300 ms for a 12 ms march
-// (339 -> 23 ms per call in a loop of calls).
+// (339 -> 20 ms per call in a loop of calls).
 //
 // The list is bounded (kKeep per device and a share of the device's free memory, so that several processes
 // on one device, each with its list, leave it room; least recently used blocks go first), drops blocks that
 // the last few calls did not take, and is given back whole before a plan or a server is created, when
 // an allocation of the library fails, so those see the memory a process without it would, and by
-// swem_release_memory.  A block
-// belongs to one call at a time; it returns to the list after the device has finished the call.
+// swem_release_memory.  A block belongs to one call at a time; it returns to the list after the
+// device has finished the call.
 #include <algorithm>
 #include <mutex>
 #include <new>
